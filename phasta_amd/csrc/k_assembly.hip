@@ -2434,13 +2434,16 @@ __global__ void k_mfg_point(const double* __restrict__ ypre, const double* __res
                             double s, const double* __restrict__ D,  // nullptr: no U^-1
                             const uint8_t* __restrict__ bcm, const double* __restrict__ BC,
                             const int* __restrict__ iper, double* __restrict__ ypack,
-                            long long n, int bc) {
+                            long long n, int bc, const double* dn, long long* t0) {
   const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (t0 && k == 0) *t0 = wall_clock64();
   if (k >= n) return;
   const long long m = bc ? (long long)iper[k] : k;
+  const double nd = dn ? *dn : 1.0;
   double v[5];
 #pragma unroll
-  for (int f = 0; f < 5; ++f) v[f] = d ? ypre[f * n + m] + s * d[f * n + m] : ypre[f * n + m];
+  for (int f = 0; f < 5; ++f)
+    v[f] = d ? ypre[f * n + m] + s * (d[f * n + m] / nd) : ypre[f * n + m];
   // i3LU 'backward' (i3lu.f:119-139) with the node's factors
   if (D) {
 #pragma unroll
@@ -2835,10 +2838,11 @@ int launch_mres(phg_ctx* c, const double* yp, double* out, bool accumulate, bool
 }
 
 int launch_mfg_point(phg_ctx* c, const double* ypre, const double* d, double s, double* ypack,
-                     bool bc, bool lu) {
+                     bool bc, bool lu, const double* dn, long long* t0) {
   const long long n = c->nshg;
   k_mfg_point<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(
-      ypre, d, s, lu ? c->bdiag : nullptr, c->bcm, c->BCv, c->iper, ypack, n, bc ? 1 : 0);
+      ypre, d, s, lu ? c->bdiag : nullptr, c->bcm, c->BCv, c->iper, ypack, n, bc ? 1 : 0, dn,
+      t0);
   PHG_HIP(hipGetLastError());
   return 0;
 }

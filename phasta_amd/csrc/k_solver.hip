@@ -146,11 +146,11 @@ template <typename TI, typename TO>
 __global__ void __launch_bounds__(kPreWaves * kGroup) k_spsi3pre(
     const TI* __restrict__ aos, TO* __restrict__ vals, const int* __restrict__ s2c,
     const int* __restrict__ scol, const long long* __restrict__ grp_slot,
-    const double* __restrict__ D, long long n) {
+    const int* __restrict__ rowmap, const double* __restrict__ D, long long n) {
   const long long g = blockIdx.x;
   const int w = threadIdx.x / kGroup, r = threadIdx.x % kGroup;
-  const long long row = g * kGroup + r;
-  if (row >= n) return;
+  const long long row = rowmap[g * kGroup + r];
+  if (row < 0) return;
   double lo[5][5];
 #pragma unroll
   for (int i = 1; i < 5; ++i)
@@ -235,23 +235,32 @@ __global__ void __launch_bounds__(kPreWaves * kGroup) k_spsi3pre(
 // (rows +-1, +-(N+1), +-(N+1)^2 on the box) then stay in that XCD's L2.
 constexpr int kSpmvWaves = 4;
 
+// rowmap: row of each (group, lane), -1 padding.  fam: per (group, lane) the
+// number of periodic slaves whose rows follow the lane's (a master), kFamSlave
+// for a slave's row, 0 otherwise.  With fold set the epilogue applies bc3per:
+// a master's sum takes its slaves' sums in ascending order from LDS and the
+// slaves get zero, as k_fold_vec does in a launch of its own (5 to 14 us per
+// product, as long as the whole product up to 16^3).
+// gate (nullable): the product is skipped when *gate is set (a Krylov
+// iteration enqueued before the host knew that the last one had converged).
 template <typename T, typename Acc>
 __global__ void __launch_bounds__(kSpmvWaves * kGroup) k_spmv(
     const T* __restrict__ vals, const int* __restrict__ scolp,
-    const long long* __restrict__ grp_slot, const double* __restrict__ p, double* __restrict__ q,
-    long long n, long long ngroups) {
+    const long long* __restrict__ grp_slot, const int* __restrict__ rowmap,
+    const uint8_t* __restrict__ fam, const double* __restrict__ p, double* __restrict__ q,
+    long long n, long long ngroups, int fold, const int* gate, long long* t0) {
+  if (gate && *gate) return;
+  if (t0 && blockIdx.x == 0 && threadIdx.x == 0) *t0 = wall_clock64();
   __shared__ Acc part[kSpmvWaves][5][kGroup];
   const long long per = (gridDim.x + 7) / 8;
   const long long g = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (g >= ngroups) return;  // whole workgroup
   const int w = threadIdx.x / kGroup, r = threadIdx.x % kGroup;
-  const long long row = g * kGroup + r;
   const long long s0 = grp_slot[g] + w, s1 = grp_slot[g + 1];
-  Acc t0 = 0, t1 = 0, t2 = 0, t3 = 0, t4 = 0;
+  Acc t[5] = {0, 0, 0, 0, 0};
   // software pipeline: the gathers of p for the next slot and the column
   // index of the one after are issued before the block of this slot is
-  // consumed (rows past n in the last group read padding: column 0, zero
-  // blocks)
+  // consumed (padding lanes read column 0 and zero blocks)
   constexpr int W = kSpmvWaves;
   Acc pc[5] = {0, 0, 0, 0, 0};
   if (s0 < s1) {
@@ -269,27 +278,32 @@ __global__ void __launch_bounds__(kSpmvWaves * kGroup) k_spmv(
     }
     Acc a[25];
     load_slot(vals + s * (25 * kGroup), r, a);
-    t0 += a[0] * pc[0] + a[5] * pc[1] + a[10] * pc[2] + a[15] * pc[3] + a[20] * pc[4];
-    t1 += a[1] * pc[0] + a[6] * pc[1] + a[11] * pc[2] + a[16] * pc[3] + a[21] * pc[4];
-    t2 += a[2] * pc[0] + a[7] * pc[1] + a[12] * pc[2] + a[17] * pc[3] + a[22] * pc[4];
-    t3 += a[3] * pc[0] + a[8] * pc[1] + a[13] * pc[2] + a[18] * pc[3] + a[23] * pc[4];
-    t4 += a[4] * pc[0] + a[9] * pc[1] + a[14] * pc[2] + a[19] * pc[3] + a[24] * pc[4];
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      t[i] += a[i] * pc[0] + a[5 + i] * pc[1] + a[10 + i] * pc[2] + a[15 + i] * pc[3] +
+              a[20 + i] * pc[4];
 #pragma unroll
     for (int f = 0; f < 5; ++f) pc[f] = pn[f];
   }
-  part[w][0][r] = t0;
-  part[w][1][r] = t1;
-  part[w][2][r] = t2;
-  part[w][3][r] = t3;
-  part[w][4][r] = t4;
+#pragma unroll
+  for (int f = 0; f < 5; ++f) part[w][f][r] = t[f];
   __syncthreads();
-  if (w != 0 || row >= n) return;
+  if (w != 0) return;
+  const long long row = rowmap[g * kGroup + r];
+  if (row < 0) return;
+  auto rowsum = [&](int f, int rr) {
+    Acc v = part[0][f][rr];
+#pragma unroll
+    for (int k = 1; k < W; ++k) v += part[k][f][rr];
+    return (double)v;
+  };
+  const int nf = fold ? fam[g * kGroup + r] : 0;
 #pragma unroll
   for (int f = 0; f < 5; ++f) {
-    Acc v = part[0][f][r];
-#pragma unroll
-    for (int k = 1; k < W; ++k) v += part[k][f][r];
-    q[row + f * n] = (double)v;
+    double v = nf == kFamSlave ? 0.0 : rowsum(f, r);
+    if (nf > 0 && nf < kFamSlave)
+      for (int k = 1; k <= nf; ++k) v += rowsum(f, r + k);
+    q[row + f * n] = v;
   }
 }
 
@@ -300,12 +314,15 @@ template <typename T>
 __global__ void __launch_bounds__(256) k_spmv_t(const T* __restrict__ vals, const int* __restrict__ scol,
                                                 const uint32_t* __restrict__ tslot,
                                                 const long long* __restrict__ grp_slot,
+                                                const int* __restrict__ rowmap,
                                                 const double* __restrict__ x, double* __restrict__ q,
-                                                long long n) {
-  const long long row = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const long long g = row / kGroup;
-  const int r = (int)(row % kGroup);
-  if (row >= n) return;
+                                                long long n, long long ngroups) {
+  const long long at = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  const long long g = at / kGroup;
+  const int r = (int)(at % kGroup);
+  if (g >= ngroups) return;
+  const long long row = rowmap[at];
+  if (row < 0) return;
   double t[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (long long s = grp_slot[g]; s < grp_slot[g + 1]; ++s) {
     const long long i = scol[s * kGroup + r];
@@ -393,10 +410,30 @@ __global__ void k_fold_vec(double* v, const int* master, const int* ptr, const i
 // the partials are summed in a fixed order by k_finish or, for the MGS
 // chain, by every block of the next step (same code, same data: the same
 // value in every block).  No atomics, so results do not depend on timing.
+// Wavefront sum on the vector ALU (row shifts, then the two row broadcasts:
+// no LDS traffic), the same in every lane.
+template <int kCtrl, int kRows>
+__device__ inline double dpp_move(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kCtrl, kRows, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, kRows, 0xf, false);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// v of one lane (a uniform index) in every lane
+__device__ inline double from_lane(double v, int lane) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += dpp_move<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row of
+  v += dpp_move<0x112, 0xf>(v);  // 16 holds the row's sum
+  v += dpp_move<0x114, 0xf>(v);
+  v += dpp_move<0x118, 0xf>(v);
+  v += dpp_move<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v += dpp_move<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  return from_lane(v, 63);
 }
 
 __device__ inline void block_partial(double v, double* part) {
@@ -472,103 +509,316 @@ __global__ void __launch_bounds__(kRedThreads) k_dot(const double* a, const doub
   block_partial(t, part);
 }
 
-// MGS step j >= 2: u <- u - beta_{j-1} u_{j-1};  beta_j = (u, u_j).
-// beta_{j-1} is the sum of the previous step's np_prev partials.
-__global__ void __launch_bounds__(kRedThreads) k_mgs(double* u, const double* ujm1, const double* uj,
-                                                     const double* part_prev, int np_prev,
-                                                     long long n, double* part) {
-  const double beta = block_sum_partials(part_prev, np_prev);
-  const bool self = uj == u;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  constexpr int U = kUnroll / 2;
-  double v[U];
-#pragma unroll
-  for (int k = 0; k < U; ++k) v[k] = 0.0;
-  for (; i + (U - 1) * stride < n; i += U * stride) {
-    double x[U], y[U], z[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      x[k] = u[i + k * stride];
-      y[k] = ujm1[i + k * stride];
-      z[k] = self ? 0.0 : uj[i + k * stride];
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const double w = x[k] - beta * y[k];
-      u[i + k * stride] = w;
-      v[k] += w * (self ? w : z[k]);
-    }
-  }
-  for (; i < n; i += stride) {
-    const double w = u[i] - beta * ujm1[i];
-    u[i] = w;
-    v[0] += w * (self ? w : uj[i]);
-  }
-  double t = 0.0;
-#pragma unroll
-  for (int k = 0; k < U; ++k) t += v[k];
-  block_partial(t, part);
+// ---------------- Gram-Schmidt and the Hessenberg recurrence ----------------
+// One Krylov iteration after its product w = K w_i (solgmr.f:598-669), in two
+// launches and without the host: k_gs_dots, k_gs_update.
+//
+// Basis vectors stay unnormalised, u_j = w_j / n_j; the norms n_j are scalars
+// of GmDev, so no pass over memory only divides by a norm.
+//
+// The orthogonalisation is the modified Gram-Schmidt of the reference with its
+// inner products taken in one pass: with d_k = (u_k, w) of the incoming w, MGS
+// subtracts h_k u_k with
+//     h_1 = d_1,  h_k = d_k - sum_{j<k} (u_k, u_j) h_j
+// (each h_k is the product of u_k with w less the earlier directions), so one
+// pass over the basis forms every d_k and the new row (u_i, u_j) of the
+// products of the basis, a triangular substitution of at most 60 rows gives
+// the h_k, and a second pass subtracts.  Two reads of the basis per iteration
+// against MGS's i + 1 dependent steps of two reads and a write each; bound by
+// those reads from 100^3 on (128^3: 6 TB/s), by the launches below 32^3.
+// Per iteration with the norm, the scaling and the Hessenberg column, 12
+// vectors: 41 us at 64^3 (FP64; one launch per MGS step 68 us), 9 us at 4^3
+// (40 us and a wait for the host).
+//
+// Reductions: a workgroup writes its partial sums, the workgroup that arrives
+// last adds them in index order (the value does not depend on which one that
+// is) and does the scalar work of the step: the coefficients (k_gs_dots), or
+// the norm, the Givens rotations, the convergence test, at the end of a cycle
+// the back substitution, and the iteration's result to the host
+// (k_gs_update).  The partials cross the XCDs' L2 caches: they are written
+// and read with agent-scope accesses, and a wait for the writes' completion
+// stands before the arrival count.
+__device__ inline void part_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double part_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Classical Gram-Schmidt for the mixed-precision path: all dot products of
-// u with the basis in one pass, then the update u -= sum_j h_j u_j fused
-// with (u, u).  Up to kCgsMax basis vectors; partial sums per workgroup in
-// channels 0..nv-1 (dots) and nv (norm), summed in a fixed order.
-constexpr int kCgsMax = 32;
+// true in every thread of the workgroup that arrives last; its partial sums
+// have to be stored before.  The counter is zero again afterwards.
+__device__ inline bool arrive_last(unsigned* cnt) {
+  __shared__ int last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned at =
+        __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = at == gridDim.x - 1;
+    if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return last != 0;
+}
 
-__device__ inline void block_partials(double* v, int nv, double* part, long long chan_stride) {
-  __shared__ double ws[kCgsMax][kRedThreads / 64];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  // compile-time indices keep v in registers
+// Workgroups of both kernels: 16 wavefronts, at most kGsBlocks of them (two
+// per CU), so that the last one has at most 8 partials per lane and sum to
+// add, all in flight together.  Each agent-scope read goes to memory: with
+// 1024 workgroups of 4 wavefronts that read theirs one after the other the
+// tail took most of k_gs_dots at 64^3 (41 us at nv = 8).
+constexpr int kGsThreads = 1024;
+constexpr int kGsBlocks = 512;
+
+// sum of np <= kGsBlocks partials by one wavefront, in a fixed order
+__device__ inline double wave_sum_partials(const double* part, int np) {
+  const int lane = threadIdx.x & 63;
+  double v[kGsBlocks / 64];
 #pragma unroll
-  for (int j = 0; j < kCgsMax; ++j) {
+  for (int u = 0; u < kGsBlocks / 64; ++u)
+    v[u] = lane + 64 * u < np ? part_load(part + lane + 64 * u) : 0.0;
+  double s = 0.0;
+#pragma unroll
+  for (int u = 0; u < kGsBlocks / 64; ++u) s += v[u];
+  return wave_sum(s);
+}
+
+struct GsArgs {
+  double* w;             // the product, then the new basis vector
+  const double* basis;   // w_0 .. w_{nv-1}
+  long long n, kstr;     // length, stride between basis vectors (even)
+  int nv, K, minIters;   // nv: the iteration number, 1..K
+  int unit;              // w is the product of u_i, not of w_i
+  double unorm, epsnrm;  // of the cycle; the start vector has norm 1
+  double* part;          // 2 nv channels of `chan` partials
+  long long chan;
+  GmDev* gm;
+  GmHost* host;          // the iteration's slot
+  unsigned seq;          // the iteration's token for the host
+};
+
+// pairs of elements per lane and pass
+constexpr int kGsU = 2;
+
+// d_k = (w_k, w) and (w_k, w_i), raw, for the nv basis vectors.  Wavefront
+// v + 4 s of a workgroup takes the vectors v, v + 4, ... on the s-th quarter
+// of the workgroup's elements, so each holds at most kT pairs of sums (kT =
+// ceil(nv / 4)); w and w_i are read by four wavefronts together and come from
+// L1 for three of them.
+template <int kT>
+__global__ void __launch_bounds__(kGsThreads) k_gs_dots(GsArgs A) {
+  GmDev& gm = *A.gm;
+  if (A.nv > 1 && gm.done) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) gm.t1 = wall_clock64();
+  __shared__ double red[4][2 * kGmMax], D[2 * kGmMax], nr[kGmMax];
+  __shared__ double G[kGmMax * (kGmMax - 1) / 2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wv = wave & 3, quarter = wave >> 2;
+  const int nv = A.nv;
+  const long long np2 = (A.n + 1) / 2;  // pairs; the last may hold one element
+  const phg_d2* w2 = reinterpret_cast<const phg_d2*>(A.w);
+  const phg_d2* u2 = reinterpret_cast<const phg_d2*>(A.basis + (size_t)(nv - 1) * A.kstr);
+  const phg_d2* b2[kT];
+#pragma unroll
+  for (int t = 0; t < kT; ++t) {
+    const int j = wv + 4 * t;
+    b2[t] = reinterpret_cast<const phg_d2*>(A.basis + (size_t)(j < nv ? j : nv - 1) * A.kstr);
+  }
+  double a1[kT], a2[kT];
+#pragma unroll
+  for (int t = 0; t < kT; ++t) a1[t] = a2[t] = 0.0;
+  const long long step = gridDim.x * (256LL * kGsU);
+  for (long long p = (blockIdx.x * 4LL + quarter) * (64 * kGsU) + lane; p < np2; p += step) {
+    phg_d2 x[kGsU], z[kGsU];
+#pragma unroll
+    for (int u = 0; u < kGsU; ++u) {
+      const long long i = p + 64 * u;
+      const bool in = i < np2;
+      x[u] = in ? w2[i] : phg_d2{0.0, 0.0};
+      z[u] = in ? u2[i] : phg_d2{0.0, 0.0};
+      // past an odd length the pair's second element is padding
+      if (2 * i + 1 >= A.n) x[u].y = z[u].y = 0.0;
+    }
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+#pragma unroll
+      for (int u = 0; u < kGsU; ++u) {
+        const long long i = p + 64 * u;
+        phg_d2 b = b2[t][i < np2 ? i : p];
+        if (2 * i + 1 >= A.n) b.y = 0.0;
+        a1[t] += b.x * x[u].x + b.y * x[u].y;
+        a2[t] += b.x * z[u].x + b.y * z[u].y;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < kT; ++t) {
+    const int j = wv + 4 * t;
     if (j < nv) {
-      const double t = wave_sum(v[j]);
-      if (lane == 0) ws[j][wid] = t;
+      const double s1 = wave_sum(a1[t]), s2 = wave_sum(a2[t]);
+      if (lane == 0) {
+        red[quarter][2 * j] = s1;
+        red[quarter][2 * j + 1] = s2;
+      }
     }
   }
+  if ((int)threadIdx.x < nv) nr[threadIdx.x] = nv > 1 ? gm.nrm[threadIdx.x] : 1.0;
   __syncthreads();
-  if ((int)threadIdx.x < nv) {
-    double s = 0.0;
-    for (int w = 0; w < kRedThreads / 64; ++w) s += ws[threadIdx.x][w];
-    part[(size_t)threadIdx.x * chan_stride + blockIdx.x] = s;
+  if ((int)threadIdx.x < 2 * nv) {
+    const int ch = threadIdx.x;
+    const double s = red[0][ch] + red[1][ch] + red[2][ch] + red[3][ch];
+    D[ch] = s;
+    if (gridDim.x > 1) part_store(A.part + (size_t)ch * A.chan + blockIdx.x, s);
+  }
+  if (gridDim.x > 1 && !arrive_last(&gm.cnt)) return;
+  // rows 1 .. nv - 2 of the strict lower triangle, row k at k (k - 1) / 2
+  for (int e = threadIdx.x; e < (nv - 1) * (nv - 2) / 2; e += kGsThreads) G[e] = gm.G[e];
+  if (gridDim.x > 1)
+    for (int ch = wave; ch < 2 * nv; ch += kGsThreads / 64) {
+      const double s = wave_sum_partials(A.part + (size_t)ch * A.chan, gridDim.x);
+      if (lane == 0) D[ch] = s;
+    }
+  __syncthreads();
+  if (wave != 0) return;
+  // one wavefront from here: lane k holds d_k
+  const int i = nv - 1;
+  const double ni = nr[i], nk = lane < nv ? nr[lane] : 1.0, nw = A.unit ? 1.0 : ni;
+  double d = lane < nv ? D[2 * lane] / (nk * nw) : 0.0;
+  if (lane < i) {
+    const double g = D[2 * lane + 1] / (nk * ni);
+    G[i * (i - 1) / 2 + lane] = g;
+    gm.G[i * (i - 1) / 2 + lane] = g;
+  }
+  __builtin_amdgcn_wave_barrier();
+  for (int j = 0; j < i; ++j) {
+    const double hj = from_lane(d, j);
+    if (lane > j && lane < nv) d -= G[lane * (lane - 1) / 2 + j] * hj;
+  }
+  if (lane < nv) {
+    gm.h[lane] = d;
+    gm.coef[lane] = -d / nk;
+  }
+  if (lane == 0) {
+    gm.scale = 1.0 / nw;
+    if (nv == 1) {
+      gm.nrm[0] = 1.0;
+      gm.done = 0;
+      gm.e[0] = A.unorm;
+      gm.acc_spmv = gm.acc_gs = 0;
+    }
   }
 }
 
-__global__ void __launch_bounds__(kRedThreads) k_cgs_dots(const double* __restrict__ u,
-                                                          const double* __restrict__ basis, int nv,
-                                                          long long n, double* part,
-                                                          long long chan_stride) {
-  double v[kCgsMax];
-#pragma unroll
-  for (int j = 0; j < kCgsMax; ++j) v[j] = 0.0;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const double x = u[i];
-#pragma unroll
-    for (int j = 0; j < kCgsMax; ++j)
-      if (j < nv) v[j] += x * basis[(size_t)j * n + i];
-  }
-  block_partials(v, nv, part, chan_stride);
-}
-
-__global__ void __launch_bounds__(kRedThreads) k_cgs_update(double* __restrict__ u,
-                                                            const double* __restrict__ basis,
-                                                            int nv, const double* __restrict__ h,
-                                                            long long n, double* part) {
-  __shared__ double hs[kCgsMax];
-  if ((int)threadIdx.x < nv) hs[threadIdx.x] = h[threadIdx.x];
+// w <- scale w - sum_k h_k w_k / n_k (scale 1 / n_i) and its norm; then the
+// Hessenberg column's rotations (solgmr.f:645-663), the convergence test and,
+// when the cycle ends, the back substitution (solgmr.f:681-686).
+__global__ void __launch_bounds__(kGsThreads) k_gs_update(GsArgs A) {
+  GmDev& gm = *A.gm;
+  if (A.nv > 1 && gm.done) return;
+  __shared__ double cf[kGmMax], ws[kGsThreads / 64];
+  const int nv = A.nv, i = nv - 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if ((int)threadIdx.x < nv) cf[threadIdx.x] = gm.coef[threadIdx.x];
+  const double a = gm.scale;
+  // the step's scalars, loaded before the wait for the other workgroups:
+  // lane k holds row k of the column
+  double hk = wave == 0 && lane < nv ? gm.h[lane] : 0.0;
+  const double cs = wave == 0 && lane < i ? gm.cs[lane] : 0.0;
+  const double sn = wave == 0 && lane < i ? gm.sn[lane] : 0.0;
+  const double ei = gm.e[i];
   __syncthreads();
+  const long long np2 = (A.n + 1) / 2;
+  phg_d2* w2 = reinterpret_cast<phg_d2*>(A.w);
+  const phg_d2* b2 = reinterpret_cast<const phg_d2*>(A.basis);
+  const long long bs = A.kstr / 2;
   double acc = 0.0;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    double x = u[i];
-    for (int j = 0; j < nv; ++j) x -= hs[j] * basis[(size_t)j * n + i];
-    u[i] = x;
-    acc += x * x;
+  for (long long p = blockIdx.x * (long long)kGsThreads + threadIdx.x; p < np2;
+       p += gridDim.x * (long long)kGsThreads) {
+    phg_d2 x = w2[p] * a;
+    int j = 0;
+    for (; j + 4 <= nv; j += 4) {
+      phg_d2 b[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) b[t] = b2[(j + t) * bs + p];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        x.x += cf[j + t] * b[t].x;
+        x.y += cf[j + t] * b[t].y;
+      }
+    }
+    for (; j < nv; ++j) {
+      const phg_d2 b = b2[j * bs + p];
+      x.x += cf[j] * b.x;
+      x.y += cf[j] * b.y;
+    }
+    if (2 * p + 1 < A.n) {
+      w2[p] = x;
+      acc += x.x * x.x + x.y * x.y;
+    } else {
+      A.w[2 * p] = x.x;
+      acc += x.x * x.x;
+    }
   }
-  block_partial(acc, part);
+  acc = wave_sum(acc);
+  if (lane == 0) ws[wave] = acc;
+  __syncthreads();
+  double sq = wave == 0 ? wave_sum(lane < kGsThreads / 64 ? ws[lane] : 0.0) : 0.0;
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) part_store(A.part + blockIdx.x, sq);
+    if (!arrive_last(&gm.cnt)) return;
+    if (wave == 0) sq = wave_sum_partials(A.part, gridDim.x);
+  }
+  if (wave != 0) return;
+  const double nrm = sqrt(sq);
+  // rotations of the earlier columns, in order: (j, j + 1)
+  double top = from_lane(hk, 0);
+  for (int j = 0; j < i; ++j) {
+    const double c = from_lane(cs, j), s = from_lane(sn, j), lo = from_lane(hk, j + 1);
+    const double t = c * top + s * lo;
+    top = -s * top + c * lo;
+    if (lane == j) hk = t;
+  }
+  const double rho = sqrt(top * top + nrm * nrm);
+  const double c = top / rho, s = nrm / rho;
+  const double e1 = -s * ei, e0 = c * ei;
+  if (lane == i) hk = rho;
+  if (lane < nv) gm.R[(size_t)i * kGmMax + lane] = hk;
+  const double echeck = fabs(e1);
+  const bool conv = echeck <= A.epsnrm && nv >= A.minIters;
+  const bool done = conv || nv >= A.K;
+  if (lane == 0) {
+    gm.nrm[nv] = nrm;
+    gm.cs[i] = c;
+    gm.sn[i] = s;
+    gm.e[i] = e0;
+    gm.e[nv] = e1;
+  }
+  if (done) {
+    double ek = lane < i ? gm.e[lane] : (lane == i ? e0 : 0.0);
+    const double nk = lane < nv ? gm.nrm[lane] : 1.0;
+    double y = 0.0;
+    for (int j = i; j >= 0; --j) {
+      const double rj = j == i ? hk : (lane <= j ? gm.R[(size_t)j * kGmMax + lane] : 0.0);
+      const double yj = from_lane(ek, j) / from_lane(rj, j);
+      if (lane == j) y = yj;
+      if (lane < j) ek = ek - yj * rj;
+    }
+    if (lane < nv) gm.y[lane] = y / nk;
+  }
+  if (lane == 0) {
+    const long long t2 = wall_clock64();
+    const long long tp = gm.acc_spmv + gm.t1 - gm.t0, tg = gm.acc_gs + t2 - gm.t1;
+    gm.acc_spmv = tp;
+    gm.acc_gs = tg;
+    gm.iKs = nv;
+    gm.done = done ? 1 : 0;
+    GmHost* h = A.host;
+    __hip_atomic_store(&h->done, done ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&h->echeck, echeck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&h->acc_spmv, tp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&h->acc_gs, tg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&h->seq, A.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // u = src / sqrt(*sq); norm_out <- sqrt(*sq) (written by one lane)
@@ -580,16 +830,27 @@ __global__ void k_scale(double* u, const double* src, long long n, const double*
   for (; i < n; i += (long long)gridDim.x * blockDim.x) u[i] = src[i] / nrm;
 }
 
-struct Coef {
-  double c[64];
-};
-
-// dy += sum_k c_k basis_k, k ascending (solgmr.f:690-692)
-__global__ void k_combine(double* dy, const double* basis, int k, Coef cf, long long n) {
+// dy (+)= sum_k y_k u_k, k ascending (solgmr.f:690-692), over the cycle's
+// directions: the first nz from zb (network directions), the others from the
+// basis; the coefficients, each with its vector's 1/norm, as the cycle left
+// them in gm.  Two 8-byte elements per lane and four directions' loads in
+// flight.
+__global__ void __launch_bounds__(256) k_combine(double* __restrict__ dy,
+                                                 const double* __restrict__ basis, long long kstr,
+                                                 const double* __restrict__ zb, long long zstr,
+                                                 int nz, const GmDev* __restrict__ gm, long long n,
+                                                 int add) {
+  __shared__ double cf[kGmMax];
+  const int k = gm->iKs;
+  if ((int)threadIdx.x < k) cf[threadIdx.x] = gm->y[threadIdx.x];
+  __syncthreads();
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
-    double v = dy[i];
-    for (int j = 0; j < k; ++j) v = v + cf.c[j] * basis[(size_t)j * n + i];
+    double v = add ? dy[i] : 0.0;
+    int j = 0;
+    for (; j < k && j < nz; ++j) v = v + cf[j] * zb[(size_t)j * zstr + i];
+#pragma unroll 4
+    for (; j < k; ++j) v = v + cf[j] * basis[(size_t)j * kstr + i];
     dy[i] = v;
   }
 }
@@ -722,26 +983,33 @@ int launch_spsi3pre(phg_ctx* c) {
   const int g = (int)c->ngroups, nt = kPreWaves * kGroup;
   if (c->precision == PHG_MIXED)
     k_spsi3pre<float, float><<<g, nt, 0, c->stream>>>(
-        c->lhs_aos32, c->lhs32, c->slot2csr, c->scol, c->grp_slot, c->bdiag, c->nshg);
+        c->lhs_aos32, c->lhs32, c->slot2csr, c->scol, c->grp_slot, c->rowmap, c->bdiag, c->nshg);
   else
     k_spsi3pre<double, double><<<g, nt, 0, c->stream>>>(
-        c->lhs_aos, c->lhs64, c->slot2csr, c->scol, c->grp_slot, c->bdiag, c->nshg);
+        c->lhs_aos, c->lhs64, c->slot2csr, c->scol, c->grp_slot, c->rowmap, c->bdiag, c->nshg);
   PHG_HIP(hipGetLastError());
   return 0;
 }
 
-int launch_spmv(phg_ctx* c, const double* p, double* q) {
+int launch_spmv(phg_ctx* c, const double* p, double* q, bool fold, const int* gate,
+                long long* t0) {
   PHG_TRY(require_matrix(c, "SparseAp"));
   const int g = (int)((c->ngroups + 7) / 8 * 8);  // one workgroup per group, XCD-strided
   const int nt = kSpmvWaves * kGroup;
+  const int in_group = fold && c->fam_in_group ? 1 : 0;
   if (c->precision == PHG_MIXED)
-    k_spmv<float, double><<<g, nt, 0, c->stream>>>(c->lhs32, c->scolp, c->grp_slot, p, q, c->nshg,
-                                                   c->ngroups);
+    k_spmv<float, double><<<g, nt, 0, c->stream>>>(c->lhs32, c->scolp, c->grp_slot, c->rowmap,
+                                                   c->fam, p, q, c->nshg, c->ngroups, in_group,
+                                                   gate, t0);
   else
-    k_spmv<double, double><<<g, nt, 0, c->stream>>>(c->lhs64, c->scolp, c->grp_slot, p, q,
-                                                    c->nshg, c->ngroups);
+    k_spmv<double, double><<<g, nt, 0, c->stream>>>(c->lhs64, c->scolp, c->grp_slot, c->rowmap,
+                                                    c->fam, p, q, c->nshg, c->ngroups, in_group,
+                                                    gate, t0);
   PHG_HIP(hipGetLastError());
-  return 0;
+  // a family of more than kGroup rows: the rows lie in several groups.  The
+  // fold runs whatever the gate says: on a skipped product's old output it
+  // is harmless (nothing reads that vector any more)
+  return fold && !c->fam_in_group ? launch_bc3per(c, q, 5) : 0;
 }
 
 // q = K^T x for the periodic-folded operator K = F A G of the matvec:
@@ -757,13 +1025,13 @@ int launch_spmv_t(phg_ctx* c, double* x, double* q) {
                                                                   c->fold_slave, c->nfold, c->nshg);
     PHG_HIP(hipGetLastError());
   }
-  const int g = grid_for(c->nshg, 256);
+  const int g = grid_for(c->ngroups * kGroup, 256);
   if (c->precision == PHG_MIXED)
-    k_spmv_t<float><<<g, 256, 0, c->stream>>>(c->lhs32, c->scol, c->tslot, c->grp_slot, x, q,
-                                              c->nshg);
+    k_spmv_t<float><<<g, 256, 0, c->stream>>>(c->lhs32, c->scol, c->tslot, c->grp_slot, c->rowmap,
+                                              x, q, c->nshg, c->ngroups);
   else
-    k_spmv_t<double><<<g, 256, 0, c->stream>>>(c->lhs64, c->scol, c->tslot, c->grp_slot, x, q,
-                                               c->nshg);
+    k_spmv_t<double><<<g, 256, 0, c->stream>>>(c->lhs64, c->scol, c->tslot, c->grp_slot,
+                                               c->rowmap, x, q, c->nshg, c->ngroups);
   PHG_HIP(hipGetLastError());
   return launch_bc3per(c, q, 5);
 }
@@ -843,28 +1111,46 @@ int launch_dot(phg_ctx* c, const double* a, const double* b, long long n, double
   return launch_finish(c, 0, np, np, 1, out);
 }
 
-int launch_mgs_part(phg_ctx* c, double* u, const double* ujm1, const double* uj, int chan_prev,
-                    int np_prev, long long n, int chan, int* np) {
-  const int g = red_grid(c, n, kUnroll / 2);
-  k_mgs<<<g, kRedThreads, 0, c->stream>>>(u, ujm1, uj, red_chan(c, chan_prev), np_prev, n,
-                                          red_chan(c, chan));
-  PHG_HIP(hipGetLastError());
-  *np = g;
-  return 0;
-}
-
-int launch_cgs(phg_ctx* c, double* u, const double* basis, int nv, long long n, double* h) {
-  if (nv < 1 || nv > kCgsMax) {
-    phg_set_error("classical Gram-Schmidt: %d basis vectors (1..%d)", nv, kCgsMax);
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm,
+              unsigned seq) {
+  if (iK < 1 || iK >= kGmMax) {
+    phg_set_error("Gram-Schmidt: iteration %d outside 1..%d", iK, kGmMax - 1);
     return PHG_EINVAL;
   }
-  const int g = red_grid(c, n, 4);
-  k_cgs_dots<<<g, kRedThreads, 0, c->stream>>>(u, basis, nv, n, red_chan(c, 0), c->red_blocks);
+  GsArgs A{};
+  A.w = w;
+  A.basis = c->krylov;
+  A.n = 5 * c->nshg;
+  A.kstr = c->kstr;
+  A.nv = iK;
+  A.K = c->prm.Kspace;
+  A.minIters = c->prm.minIters;
+  A.unit = unit ? 1 : 0;
+  A.unorm = unorm;
+  A.epsnrm = epsnrm;
+  A.part = c->red_part;
+  A.chan = c->red_blocks;
+  A.gm = c->gm;
+  A.host = c->h_gm + iK;
+  A.seq = seq;
+  const long long np2 = (A.n + 1) / 2;
+  const int gd = (int)std::min<long long>(grid_for(np2, 256 * kGsU), kGsBlocks);
+  const int gu = (int)std::min<long long>(grid_for(np2, kGsThreads), kGsBlocks);
+  const int t = (iK + 3) / 4;
+  if (t <= 1)
+    k_gs_dots<1><<<gd, kGsThreads, 0, c->stream>>>(A);
+  else if (t == 2)
+    k_gs_dots<2><<<gd, kGsThreads, 0, c->stream>>>(A);
+  else if (t == 3)
+    k_gs_dots<3><<<gd, kGsThreads, 0, c->stream>>>(A);
+  else if (t <= 5)
+    k_gs_dots<5><<<gd, kGsThreads, 0, c->stream>>>(A);
+  else
+    k_gs_dots<15><<<gd, kGsThreads, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
-  PHG_TRY(launch_finish(c, 0, g, g, nv, h));
-  k_cgs_update<<<g, kRedThreads, 0, c->stream>>>(u, basis, nv, h, n, red_chan(c, nv));
+  k_gs_update<<<gu, kGsThreads, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
-  return launch_finish(c, nv, g, g, 1, h + nv);
+  return 0;
 }
 
 int launch_scale(phg_ctx* c, double* u, const double* src, long long n, const double* sq_ptr,
@@ -875,16 +1161,10 @@ int launch_scale(phg_ctx* c, double* u, const double* src, long long n, const do
   return 0;
 }
 
-int launch_combine(phg_ctx* c, double* dy, const double* basis, int k, const double* coef,
-                   long long n) {
-  Coef cf{};
-  if (k > 64) {
-    phg_set_error("combine: Kspace %d > 64", k);
-    return PHG_EINVAL;
-  }
-  for (int j = 0; j < k; ++j) cf.c[j] = coef[j];
+int launch_combine(phg_ctx* c, double* dy, const double* zb, int nz, bool add) {
+  const long long n = 5 * c->nshg;
   int g = (int)std::min<long long>(grid_for(n, 256), 16384);
-  k_combine<<<g, 256, 0, c->stream>>>(dy, basis, k, cf, n);
+  k_combine<<<g, 256, 0, c->stream>>>(dy, c->krylov, c->kstr, zb, n, nz, c->gm, n, add ? 1 : 0);
   PHG_HIP(hipGetLastError());
   return 0;
 }

@@ -2,6 +2,7 @@
 // matrix layout and colouring, and the host-side sequencing of the
 // SolGMRs/ElmGMRs work on one HIP stream.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -165,13 +166,49 @@ int setup(phg_ctx* c, const phg_mesh* m) {
     return PHG_ECOLOR;
   }
 
-  // ---- slot layout of the block-CSR matrix ----
-  c->ngroups = (nshg + kGroup - 1) / kGroup;
+  // ---- periodic families: slaves per master, ascending ----
+  std::vector<std::vector<int>> sl(nshg);
+  for (long long j = 0; j < nshg; ++j)
+    if (m->iBC[j] & 1024) {
+      const int i = m->iper[j] - 1;
+      if (i != j) sl[i].push_back((int)j);
+    }
+
+  // ---- slot layout of the block-CSR matrix: rows in natural order, a
+  // master's slaves pulled up behind it into its 64-row group ----
+  c->fam_in_group = true;
+  for (long long i = 0; i < nshg; ++i)
+    if ((long long)sl[i].size() + 1 > kGroup) c->fam_in_group = false;
+  std::vector<int> rowmap;
+  std::vector<uint8_t> fam;
+  rowmap.reserve(nshg + 4 * kGroup);
+  for (long long i = 0; i < nshg; ++i) {
+    const bool slave = (m->iBC[i] & 1024) && m->iper[i] - 1 != i;
+    if (c->fam_in_group && slave) continue;  // behind its master
+    const int ns = c->fam_in_group ? (int)sl[i].size() : 0;
+    if ((int)(rowmap.size() % kGroup) + ns + 1 > kGroup)
+      while (rowmap.size() % kGroup) rowmap.push_back(-1);
+    fam.resize(rowmap.size(), 0);
+    rowmap.push_back((int)i);
+    fam.push_back((uint8_t)ns);
+    for (int k = 0; k < ns; ++k) {
+      rowmap.push_back(sl[i][k]);
+      fam.push_back((uint8_t)kFamSlave);
+    }
+  }
+  while (rowmap.size() % kGroup) rowmap.push_back(-1);
+  fam.resize(rowmap.size(), 0);
+  c->ngroups = (long long)(rowmap.size() / kGroup);
+  std::vector<int> at(nshg);  // (group, lane) of a row
+  for (size_t p = 0; p < rowmap.size(); ++p)
+    if (rowmap[p] >= 0) at[rowmap[p]] = (int)p;
   c->h_grp_slot.assign(c->ngroups + 1, 0);
   for (long long g = 0; g < c->ngroups; ++g) {
     int smax = 0;
-    for (long long r = g * kGroup; r < std::min(nshg, (g + 1) * kGroup); ++r)
-      smax = std::max(smax, m->colm[r + 1] - m->colm[r]);
+    for (int r = 0; r < kGroup; ++r) {
+      const int row = rowmap[g * kGroup + r];
+      if (row >= 0) smax = std::max(smax, m->colm[row + 1] - m->colm[row]);
+    }
     c->h_grp_slot[g + 1] = c->h_grp_slot[g] + smax;
   }
   c->nslots = c->h_grp_slot[c->ngroups];
@@ -186,12 +223,12 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   for (long long g = 0; g < c->ngroups; ++g) {
     const long long S = c->h_grp_slot[g + 1] - c->h_grp_slot[g];
     for (int r = 0; r < kGroup; ++r) {
-      const long long row = g * kGroup + r;
-      const long long b0 = row < nshg ? m->colm[row] - 1 : 0;
-      const long long len = row < nshg ? m->colm[row + 1] - m->colm[row] : 0;
+      const long long row = rowmap[g * kGroup + r];
+      const long long b0 = row >= 0 ? m->colm[row] - 1 : 0;
+      const long long len = row >= 0 ? m->colm[row + 1] - m->colm[row] : 0;
       for (long long s = 0; s < S; ++s) {
         const long long q = (c->h_grp_slot[g] + s) * kGroup + r;
-        int col = row < nshg ? (int)row : 0;
+        int col = row >= 0 ? (int)row : 0;
         if (s < len) {
           col = m->rowp[b0 + s] - 1;
           c2s[b0 + s] = (uint32_t)q;
@@ -221,8 +258,9 @@ int setup(phg_ctx* c, const phg_mesh* m) {
           bad_t = 1;
           continue;
         }
-        const long long qj = (c->h_grp_slot[j / kGroup] + (f - lst)) * kGroup + j % kGroup;
-        tsl[(c->h_grp_slot[i / kGroup] + t) * kGroup + i % kGroup] = (uint32_t)qj;
+        const long long qj =
+            (c->h_grp_slot[at[j] / kGroup] + (f - lst)) * kGroup + at[j] % kGroup;
+        tsl[(c->h_grp_slot[at[i] / kGroup] + t) * kGroup + at[i] % kGroup] = (uint32_t)qj;
       }
     }
     if (bad_t) {
@@ -435,16 +473,9 @@ int setup(phg_ctx* c, const phg_mesh* m) {
     for (int a = 0; a < 4; ++a) ienbc[a * nelb + p] = m->ienb[orderb[p] + nelb * a] - 1;
 
   // ---- periodic fold lists ----
-  std::vector<std::vector<int>> sl(nshg);
   std::vector<int> masters;
-  for (long long j = 0; j < nshg; ++j)
-    if (m->iBC[j] & 1024) {
-      const int i = m->iper[j] - 1;
-      if (i == j) continue;
-      if (sl[i].empty()) masters.push_back(i);
-      sl[i].push_back((int)j);
-    }
-  std::sort(masters.begin(), masters.end());
+  for (long long i = 0; i < nshg; ++i)
+    if (!sl[i].empty()) masters.push_back((int)i);
   std::vector<int> fptr(1, 0), fsl;
   for (int mm : masters) {
     for (int s : sl[mm]) fsl.push_back(s);
@@ -501,6 +532,8 @@ int setup(phg_ctx* c, const phg_mesh* m) {
     PHG_TRY(dev_alloc(c, &c->tslot, c->nslots * kGroup));
     PHG_TRY(dev_alloc(c, &c->csr2slot, nnz));
     PHG_TRY(dev_alloc(c, &c->slot2csr, c->nslots * kGroup));
+    PHG_TRY(dev_alloc(c, &c->rowmap, rowmap.size()));
+    PHG_TRY(dev_alloc(c, &c->fam, fam.size()));
   }
   PHG_TRY(dev_alloc(c, &c->acc_res, 5 * nshg));
   if (mat && mixed)
@@ -524,11 +557,21 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_TRY(dev_alloc(c, &c->acold, 5 * nshg));
   PHG_TRY(dev_alloc(c, &c->dy, 5 * nshg));
   // K+1 basis vectors; at least 3 (the refinement loop uses 1 and 2 as scratch)
-  PHG_TRY(dev_alloc(c, &c->krylov, (size_t)(std::max(K, 2) + 1) * 5 * nshg));
+  c->kstr = (5 * nshg + 1) & ~1LL;
+  PHG_TRY(dev_alloc(c, &c->krylov, (size_t)(std::max(K, 2) + 1) * c->kstr));
   c->red_blocks = 1024;
-  PHG_TRY(dev_alloc(c, &c->red_part, (size_t)(K + 3) * c->red_blocks));
+  PHG_TRY(dev_alloc(c, &c->red_part, (size_t)(2 * (K + 2)) * c->red_blocks));
   PHG_TRY(dev_alloc(c, &c->scal, 256));
+  PHG_TRY(dev_alloc(c, &c->gm, 1));
   PHG_HIP(hipHostMalloc((void**)&c->h_scal, 256 * sizeof(double), hipHostMallocDefault));
+  PHG_HIP(hipHostMalloc((void**)&c->h_gm, kGmMax * sizeof(GmHost), hipHostMallocCoherent));
+  std::fill(c->h_gm, c->h_gm + kGmMax, GmHost{});
+  {
+    int dev = 0, khz = 0;
+    PHG_HIP(hipGetDevice(&dev));
+    PHG_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    c->clk_ms = khz > 0 ? 1.0 / (double)khz : 0.0;
+  }
 
   std::vector<double> xs(3 * nshg);
   std::copy(m->x, m->x + 3 * nshg, xs.begin());
@@ -558,6 +601,8 @@ int setup(phg_ctx* c, const phg_mesh* m) {
     PHG_TRY(upload(c, c->tslot, tsl.data(), tsl.size()));
     PHG_TRY(upload(c, c->csr2slot, c2s.data(), c2s.size()));
     PHG_TRY(upload(c, c->slot2csr, s2c.data(), s2c.size()));
+    PHG_TRY(upload(c, c->rowmap, rowmap.data(), rowmap.size()));
+    PHG_TRY(upload(c, c->fam, fam.data(), fam.size()));
     if (mixed)
       PHG_TRY(launch_fill(c, c->lhs32, sizeof(float) * 25 * kGroup * c->nslots));
     else
@@ -565,6 +610,7 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   }
   PHG_TRY(launch_fill(c, c->yold, sizeof(double) * 5 * nshg));
   PHG_TRY(launch_fill(c, c->acold, sizeof(double) * 5 * nshg));
+  PHG_TRY(launch_fill(c, c->gm, sizeof(GmDev)));
   PHG_TRY(sync(c));
   return 0;
 }
@@ -579,7 +625,7 @@ int ensure_tmp(phg_ctx* c, size_t bytes) {
   return 0;
 }
 
-double* kvec(phg_ctx* c, int k) { return c->krylov + (size_t)k * 5 * c->nshg; }
+double* kvec(phg_ctx* c, int k) { return c->krylov + (size_t)k * c->kstr; }
 
 // ElmGMRs on the resident y/ac: res, rmes(=0), BDiag, lhsK (elmgmr.f:395-610)
 // idiff 0, 1 or 3; the flux buffers are allocated when first needed
@@ -653,8 +699,10 @@ int mfg_alloc(phg_ctx* c) {
 
 // Au1MFG (au1mfg.f:56-83): w = (L^-1 Rmod(itrBC(U^-1 (ypre + e v))) - rmes) / e
 // with the forward-reduced modified residual rmes of the base point
-int mfg_apply(phg_ctx* c, const double* v, double* w) {
-  PHG_TRY(launch_mfg_point(c, c->mfg.ypre, v, c->mfg.eg, c->mfg.pack, true, true));
+// (vn: the norm that v is divided by, nullable; t0: launch_mfg_point)
+int mfg_apply(phg_ctx* c, const double* v, double* w, const double* vn = nullptr,
+              long long* t0 = nullptr) {
+  PHG_TRY(launch_mfg_point(c, c->mfg.ypre, v, c->mfg.eg, c->mfg.pack, true, true, vn, t0));
   PHG_TRY(launch_mres(c, c->mfg.pack, c->mfg.t1, false, false));
   return launch_mfg_fwd_diff(c, c->mfg.t1, c->rmes, c->mfg.eg, w);
 }
@@ -747,8 +795,28 @@ int elm_mfg(phg_ctx* c) {
   return launch_mres(c, nullptr, c->rmes, false, false);
 }
 
+// Waits until the device has written iteration iK's result (token seq) into
+// its slot.  The stream is asked now and then, so that a failed launch or a
+// fault ends the wait.
+int wait_iteration(phg_ctx* c, int iK, unsigned seq) {
+  const volatile unsigned* at = &c->h_gm[iK].seq;
+  for (unsigned spin = 1; *at != seq; ++spin) {
+    if (spin % 4096) continue;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    PHG_HIP(e);
+    if (*at != seq) {
+      phg_set_error("GMRES: the stream drained without the result of iteration %d", iK);
+      return PHG_EHIP;
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return 0;
+}
+
 // One GMRES cycle on the scaled system (solgmr.f:522-692): kvec(0) holds the
-// normalised start vector, unorm its norm.  Adds sum_k y_k u_k to c->dy.
+// normalised start vector, unorm its norm.  Leaves sum_k y_k u_k in c->dy, or
+// adds it there.
 struct CycleOut {
   int iKs = 0;
   double echeck = 0.0;
@@ -757,134 +825,104 @@ struct CycleOut {
 
 // flexible: precondition each direction with the network (FGMRES, right
 // preconditioning) and combine the preconditioned directions.
-// basis sizes the classical Gram-Schmidt kernels take (launch_cgs)
-constexpr int kCgsVectors = 32;
-
+//
+// The Hessenberg recurrence and the convergence test run on the device
+// (launch_gs); the host stays one iteration ahead of the result it has seen,
+// so the device never waits for the host between iterations.  The iteration
+// enqueued after the last one finds GmDev::done set and returns.
 int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut* out,
-                bool flexible = false) {
+                bool flexible, bool add) {
   const long long V = 5 * c->nshg;
-  auto zvec = [&](int k) { return c->mp.zbasis + (size_t)k * V; };
   const int K = c->prm.Kspace;
-  double* H = c->scal + 16;
-  int iKs = 0;
-  double echeck = 0.0;
-  std::vector<double> Hh((size_t)(K + 2) * (K + 1), 0.0), e(K + 2, 0.0), Rc(K + 2, 0.0),
-      Rs(K + 2, 0.0), yB(K + 2, 0.0);
-  auto Hm = [&](int a, int b) -> double& { return Hh[(size_t)(a - 1) + (size_t)(K + 1) * (b - 1)]; };
-  e[1] = unorm;
-  bool use_net = flexible && c->mp.use_pc >= 1;
+  auto zvec = [&](int k) { return c->mp.zbasis + (size_t)k * V; };
+  const int use_pc = flexible ? c->mp.use_pc : 0;
+  bool use_net = use_pc >= 1;
+  const unsigned base = c->gm_seq;
+  c->gm_seq += (unsigned)K + 1;
+  int last = 0;  // the last iteration whose result has been seen
   for (int iK = 1; iK <= K; ++iK) {
-    iKs = iK;
     double* w = kvec(c, iK);
     const double* dir = kvec(c, iK - 1);
-    bool have_w = false;
-    if (flexible) {
-      // the network preconditions the first use_pc directions of the cycle,
-      // the block-diagonal preconditioner (identity here) the rest
-      if (use_net && iK <= c->mp.use_pc) {
-        PHG_TRY(mp_forward(c, kvec(c, iK - 1), zvec(iK - 1), false));
-        if (iK == 1) {
-          // acceptance test, block-diagonal GMRES as the yardstick: the
-          // one-step residual min_a ||u_1 - a K z||^2 = 1 - (u_1.Kz)^2/|Kz|^2
-          // of the network's direction z = N(u_1) against that of z = u_1;
-          // the network's direction is kept unless it is larger
-          double* wp = c->mp.wplain;
-          double* sb = c->mp.sbuf + 8;
-          PHG_HIP(hipEventRecord(c->kev[0], c->stream));
-          PHG_TRY(launch_spmv(c, zvec(0), w));
-          PHG_TRY(launch_spmv(c, kvec(c, 0), wp));
-          PHG_HIP(hipEventRecord(c->kev[1], c->stream));
-          PHG_TRY(launch_bc3per(c, w, 5));
-          PHG_TRY(launch_bc3per(c, wp, 5));
-          PHG_TRY(launch_dot(c, kvec(c, 0), w, V, sb));
-          PHG_TRY(launch_dot(c, w, w, V, sb + 1));
-          PHG_TRY(launch_dot(c, kvec(c, 0), wp, V, sb + 2));
-          PHG_TRY(launch_dot(c, wp, wp, V, sb + 3));
-          double d[4] = {0.0, 0.0, 0.0, 0.0};
-          PHG_HIP(hipMemcpyAsync(d, sb, sizeof(d), hipMemcpyDeviceToHost, c->stream));
-          PHG_TRY(sync(c));
-          float a1 = 0;
-          PHG_HIP(hipEventElapsedTime(&a1, c->kev[0], c->kev[1]));
-          st->ms_spmv += a1;
-          st->n_spmv += 2;
-          const double r_net = d[1] > 0.0 ? 1.0 - d[0] * d[0] / d[1] : 1.0;
-          const double r_blk = d[3] > 0.0 ? 1.0 - d[2] * d[2] / d[3] : 1.0;
-          if (!(r_net <= r_blk)) {
-            use_net = false;
-            out->rejected = true;
-            PHG_HIP(hipMemcpyAsync(zvec(0), kvec(c, 0), sizeof(double) * V,
-                                   hipMemcpyDeviceToDevice, c->stream));
-            PHG_HIP(hipMemcpyAsync(w, wp, sizeof(double) * V, hipMemcpyDeviceToDevice,
-                                   c->stream));
-          }
-          have_w = true;
+    const bool net = use_net && iK <= use_pc;
+    // the network preconditions the first use_pc directions of the cycle,
+    // the block-diagonal preconditioner (identity here) the rest.  An
+    // iteration whose product the gate does not skip waits for the one
+    // before it
+    const int lag = net || c->mfg.on ? 0 : 1;
+    if (net) {
+      PHG_TRY(mp_forward(c, dir, zvec(iK - 1), false));
+      if (iK == 1) {
+        // acceptance test, block-diagonal GMRES as the yardstick: the
+        // one-step residual min_a ||u_1 - a K z||^2 = 1 - (u_1.Kz)^2/|Kz|^2
+        // of the network's direction z = N(u_1) against that of z = u_1;
+        // the network's direction is kept unless it is larger
+        double* wn = c->mp.wplain;
+        double* sb = c->mp.sbuf + 8;
+        PHG_HIP(hipEventRecord(c->kev[0], c->stream));
+        PHG_TRY(launch_spmv(c, zvec(0), wn, true));
+        PHG_TRY(launch_spmv(c, dir, w, true, nullptr, &c->gm->t0));
+        PHG_HIP(hipEventRecord(c->kev[1], c->stream));
+        PHG_TRY(launch_dot(c, dir, wn, V, sb));
+        PHG_TRY(launch_dot(c, wn, wn, V, sb + 1));
+        PHG_TRY(launch_dot(c, dir, w, V, sb + 2));
+        PHG_TRY(launch_dot(c, w, w, V, sb + 3));
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+        PHG_HIP(hipMemcpyAsync(d, sb, sizeof(d), hipMemcpyDeviceToHost, c->stream));
+        PHG_TRY(sync(c));
+        float a1 = 0;
+        PHG_HIP(hipEventElapsedTime(&a1, c->kev[0], c->kev[1]));
+        st->ms_spmv += 0.5 * a1;  // the second product is in the cycle's own clock
+        st->n_spmv += 1;
+        const double r_net = d[1] > 0.0 ? 1.0 - d[0] * d[0] / d[1] : 1.0;
+        const double r_blk = d[3] > 0.0 ? 1.0 - d[2] * d[2] / d[3] : 1.0;
+        if (!(r_net <= r_blk)) {
+          use_net = false;  // the plain direction's product is in w
+          out->rejected = true;
+        } else {
+          PHG_HIP(hipMemcpyAsync(w, wn, sizeof(double) * V, hipMemcpyDeviceToDevice, c->stream));
         }
       } else {
-        PHG_HIP(hipMemcpyAsync(zvec(iK - 1), kvec(c, iK - 1), sizeof(double) * V,
-                               hipMemcpyDeviceToDevice, c->stream));
+        PHG_TRY(launch_spmv(c, zvec(iK - 1), w, true, nullptr, &c->gm->t0));
       }
-      dir = zvec(iK - 1);
-    }
-    if (!have_w) {
-      PHG_HIP(hipEventRecord(c->kev[0], c->stream));
-      if (c->mfg.on) {
-        PHG_TRY(mfg_apply(c, dir, w));  // Au1MFG: bc3Res folds inside
-      } else {
-        PHG_TRY(launch_spmv(c, dir, w));
-      }
-      PHG_HIP(hipEventRecord(c->kev[1], c->stream));
-      if (!c->mfg.on) PHG_TRY(launch_bc3per(c, w, 5));
-    }
-    PHG_HIP(hipEventRecord(c->kev[2], c->stream));
-    if (c->precision == PHG_MIXED && iK <= kCgsVectors) {
-      // the mixed path orthogonalises by classical Gram-Schmidt: two passes
-      // over the basis instead of iK + 1 (its error is stated against FP64)
-      PHG_TRY(launch_cgs(c, w, kvec(c, 0), iK, V, H));
+    } else if (c->mfg.on) {
+      // Au1MFG: bc3Res folds inside
+      PHG_TRY(mfg_apply(c, dir, w, iK > 1 ? &c->gm->nrm[iK - 1] : nullptr, &c->gm->t0));
     } else {
-      // H(1..iK+1, iK) by MGS (solgmr.f:598-618): channel j-1 holds the
-      // partials of H(j, iK)
-      int np0 = 0, np = 0;
-      PHG_TRY(launch_dot_part(c, w, kvec(c, 0), V, 0, &np0));
-      int np_prev = np0;
-      for (int jK = 2; jK <= iK + 1; ++jK) {
-        PHG_TRY(launch_mgs_part(c, w, kvec(c, jK - 2), jK == iK + 1 ? w : kvec(c, jK - 1), jK - 2,
-                                np_prev, V, jK - 1, &np));
-        np_prev = np;
-      }
-      PHG_TRY(launch_finish(c, 0, np0, np, iK + 1, H));
+      PHG_TRY(launch_spmv(c, dir, w, true, iK > 1 ? &c->gm->done : nullptr, &c->gm->t0));
     }
-    PHG_HIP(hipEventRecord(c->kev[3], c->stream));
-    PHG_TRY(launch_scale(c, w, w, V, H + iK, H + iK + 1));
-    PHG_TRY(download(c, c->h_scal + 16, H, iK + 2));
+    PHG_TRY(launch_gs(c, w, iK, c->mfg.on, unorm, epsnrm, base + iK));
+    if (iK > lag) {
+      last = iK - lag;
+      PHG_TRY(wait_iteration(c, last, base + last));
+      if (c->h_gm[last].done) break;
+    }
+  }
+  if (last < K && !(last > 0 && c->h_gm[last].done)) {
+    last = K;
+    PHG_TRY(wait_iteration(c, last, base + last));
+  }
+  const GmHost& end = c->h_gm[last];
+  const int iKs = last;
+  c->ntotGM += iKs;
+  st->ms_spmv += c->clk_ms * (double)end.acc_spmv;
+  st->ms_mgs += c->clk_ms * (double)end.acc_gs;
+  st->n_spmv += iKs;
+  for (int k = 1; k <= iKs; ++k) st->n_mgs += k + 1;
+  if ((c->diag_flags & PHG_DIAG_ORTH) || (c->mp.ready && c->mp.keep_pair)) {
+    // the basis normalised: for the orthogonality check, and for the training
+    // on the cycle's Krylov vectors (phg_mpnn_train_krylov)
+    double nrm[kGmMax];
+    PHG_HIP(hipMemcpyAsync(nrm, c->gm->nrm, sizeof(nrm), hipMemcpyDeviceToHost, c->stream));
     PHG_TRY(sync(c));
-    {
-      float a1 = 0, a2 = 0;
-      if (!have_w) PHG_HIP(hipEventElapsedTime(&a1, c->kev[0], c->kev[1]));
-      PHG_HIP(hipEventElapsedTime(&a2, c->kev[2], c->kev[3]));
-      st->ms_spmv += a1;
-      st->ms_mgs += a2;
-      if (!have_w) st->n_spmv += 1;
-      st->n_mgs += iK + 1;
-    }
-    for (int jK = 1; jK <= iK; ++jK) Hm(jK, iK) = c->h_scal[16 + jK - 1];
-    Hm(iK + 1, iK) = c->h_scal[16 + iK + 1];
-    // Givens rotations on the new column (solgmr.f:645-663)
-    for (int jK = 1; jK <= iK - 1; ++jK) {
-      const double t = Rc[jK] * Hm(jK, iK) + Rs[jK] * Hm(jK + 1, iK);
-      Hm(jK + 1, iK) = -Rs[jK] * Hm(jK, iK) + Rc[jK] * Hm(jK + 1, iK);
-      Hm(jK, iK) = t;
-    }
-    const double t = std::sqrt(Hm(iK, iK) * Hm(iK, iK) + Hm(iK + 1, iK) * Hm(iK + 1, iK));
-    Rc[iK] = Hm(iK, iK) / t;
-    Rs[iK] = Hm(iK + 1, iK) / t;
-    Hm(iK, iK) = t;
-    Hm(iK + 1, iK) = 0.0;
-    const double t2 = Rc[iK] * e[iK] + Rs[iK] * e[iK + 1];
-    e[iK + 1] = -Rs[iK] * e[iK] + Rc[iK] * e[iK + 1];
-    e[iK] = t2;
-    c->ntotGM++;
-    echeck = std::fabs(e[iK + 1]);
-    if (echeck <= epsnrm && iK >= c->prm.minIters) break;
+    for (int k = 1; k <= iKs; ++k) nrm[k] = nrm[k] * nrm[k];
+    double* S = c->scal + 128;
+    PHG_HIP(hipMemcpyAsync(S, nrm, sizeof(double) * (iKs + 1), hipMemcpyHostToDevice, c->stream));
+    PHG_TRY(launch_combine(c, c->dy, c->mp.zbasis, use_net ? std::min(use_pc, iKs) : 0, add));
+    for (int k = 1; k <= iKs; ++k)
+      PHG_TRY(launch_scale(c, kvec(c, k), kvec(c, k), V, S + k, nullptr));
+    PHG_TRY(sync(c));
+  } else {
+    PHG_TRY(launch_combine(c, c->dy, c->mp.zbasis, use_net ? std::min(use_pc, iKs) : 0, add));
   }
   if (c->diag_flags & PHG_DIAG_ORTH) {
     // orthogonality of the cycle's basis u_0..u_iKs: max |u_i . u_j - delta_ij|
@@ -899,14 +937,8 @@ int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut
     }
     st->orth_loss = std::max(st->orth_loss, loss);
   }
-  // back substitution (solgmr.f:681-686), Dy += y_k u_k (solgmr.f:690-692)
-  for (int jK = iKs; jK >= 1; --jK) {
-    yB[jK] = e[jK] / Hm(jK, jK);
-    for (int lK = 1; lK <= jK - 1; ++lK) e[lK] = e[lK] - yB[jK] * Hm(lK, jK);
-  }
-  PHG_TRY(launch_combine(c, c->dy, flexible ? c->mp.zbasis : c->krylov, iKs, yB.data() + 1, V));
   out->iKs = iKs;
-  out->echeck = std::fabs(e[iKs + 1]);
+  out->echeck = end.echeck;
   return 0;
 }
 
@@ -965,7 +997,7 @@ int mfg_core(phg_ctx* c, int fdi, phg_stats* st) {
         unorm = c->h_scal[6];
       }
       CycleOut co;
-      rc = gmres_cycle(c, unorm, epsnrm, st, &co, false);
+      rc = gmres_cycle(c, unorm, epsnrm, st, &co, false, mG > 1);
       if (rc) break;
       iKs = co.iKs;
       echeck = co.echeck;
@@ -1097,8 +1129,7 @@ int sol_core(phg_ctx* c, phg_stats* st) {
         PHG_TRY(launch_sub(c, kvec(c, 2), c->rmes, kvec(c, 2), V));
         PHG_TRY(launch_i3lu(c, c->bdiag, kvec(c, 2), 1));
       } else {
-        PHG_TRY(launch_spmv(c, c->dy, kvec(c, 1)));
-        PHG_TRY(launch_bc3per(c, kvec(c, 1), 5));
+        PHG_TRY(launch_spmv(c, c->dy, kvec(c, 1), true));
         PHG_TRY(launch_sub(c, kvec(c, 2), c->res, kvec(c, 1), V));
       }
       PHG_TRY(launch_dot(c, kvec(c, 2), kvec(c, 2), V, S + 5));
@@ -1112,7 +1143,7 @@ int sol_core(phg_ctx* c, phg_stats* st) {
     if (learned) {
       // FGMRES cycle with the network; block-diagonal GMRES is its fallback and yardstick
       CycleOut co;
-      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co, true));
+      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co, true, false));
       iKs += co.iKs;
       st->refine_cycles = 1;
       PHG_TRY(true_residual(&rnorm));
@@ -1132,9 +1163,11 @@ int sol_core(phg_ctx* c, phg_stats* st) {
       }
     }
     const bool need_plain = plain_from_start || rnorm > epsnrm;
+    bool add = !plain_from_start;  // onto the learned cycle's update
     for (int cyc = 0; need_plain; ++cyc) {
       CycleOut co;
-      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co));
+      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co, false, add));
+      add = true;
       iKs += co.iKs;
       echeck = co.echeck;
       st->refine_cycles += 1;
@@ -1285,10 +1318,11 @@ extern "C" int phg_finalize(phg_ctx* c) {
                   c->acold,    c->dy,       c->krylov, c->red_part, c->scal,
                   c->tmp,      c->slot2csr, c->lhs_aos, c->lhs_aos32, c->acc_res, c->acc_bd,
                   c->nodepack, c->inc_goff, c->inc,   c->eslot,   c->qrec,    c->qnode,
-                  c->dcw,      c->mtau,     c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
+                  c->dcw,      c->mtau,     c->gm,      c->rowmap,  c->fam,     c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_scal) (void)hipHostFree(c->h_scal);
+  if (c->h_gm) (void)hipHostFree(c->h_gm);
   for (auto ev : c->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto ev : c->kev)
@@ -1543,7 +1577,7 @@ extern "C" int phg_sparse_ap(phg_ctx* c, const double* lhsK, double* p) {
     PHG_TRY(launch_csr_to_slots(c, c->tmp, c->lhs64));
   }
   PHG_TRY(upload(c, kvec(c, 0), p, 5 * n));
-  PHG_TRY(launch_spmv(c, kvec(c, 0), kvec(c, 1)));
+  PHG_TRY(launch_spmv(c, kvec(c, 0), kvec(c, 1), false));
   PHG_TRY(download(c, p, kvec(c, 1), 5 * n));
   return sync(c);
 }
@@ -1653,9 +1687,9 @@ extern "C" int phg_bc3per(phg_ctx* c, double* res, int nQs) {
 extern "C" int phg_bench_spmv(phg_ctx* c, int reps, double* ms_per_launch, double* bytes) {
   PHG_TRY(check_ctx(c));
   PHG_TRY(require_matrix(c, "phg_bench_spmv"));
-  PHG_TRY(launch_spmv(c, kvec(c, 0), kvec(c, 1)));  // warm
+  PHG_TRY(launch_spmv(c, kvec(c, 0), kvec(c, 1), false));  // warm
   PHG_HIP(hipEventRecord(c->ev[0], c->stream));
-  for (int i = 0; i < reps; ++i) PHG_TRY(launch_spmv(c, kvec(c, i & 1), kvec(c, (i + 1) & 1)));
+  for (int i = 0; i < reps; ++i) PHG_TRY(launch_spmv(c, kvec(c, i & 1), kvec(c, (i + 1) & 1), false));
   PHG_HIP(hipEventRecord(c->ev[1], c->stream));
   PHG_HIP(hipEventSynchronize(c->ev[1]));
   float ms = 0;
@@ -1674,7 +1708,7 @@ extern "C" int phg_bench_copy(phg_ctx* c, int reps, double* ms_per_launch, doubl
   PHG_TRY(check_ctx(c));
   // first half of the Krylov space -> second half
   const long long nvec = std::max(c->kcap, 2) + 1;  // vectors allocated by setup
-  const long long half = ((nvec / 2) * 5 * c->nshg) & ~1LL;
+  const long long half = (nvec / 2) * c->kstr;
   double* src = c->krylov;
   double* dst = c->krylov + half;
   PHG_TRY(launch_copy(c, dst, src, half));  // warm

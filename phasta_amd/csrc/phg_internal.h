@@ -126,6 +126,36 @@ __host__ __device__ inline uint8_t constraint_mask(int ibc) {
   return m;
 }
 
+// Longest periodic family (a master and its slaves) whose fold the matvec
+// applies itself: the family's rows have to lie in one 64-row group.
+constexpr int kFamSlave = 255;
+
+// Scalars of one GMRES cycle, on the device (k_gs_dots, k_gs_update):
+// iterations 1 .. kGmMax - 1 (Kspace is at most 60).
+constexpr int kGmMax = 64;
+struct GmDev {
+  unsigned cnt;                     // arrivals of the running reduction
+  int done, iKs;                    // the cycle has ended; iterations so far
+  long long t0, t1;                 // device clock: product begun, dots begun
+  long long acc_spmv, acc_gs;       // clock ticks of the cycle's products and
+                                    // Gram-Schmidt steps
+  double scale;                     // of the running iteration's product: 1 / n_i, or 1
+  double nrm[kGmMax];               // norms n_j of the basis vectors
+  double h[kGmMax], coef[kGmMax];   // Hessenberg column; -h_k / n_k
+  double cs[kGmMax], sn[kGmMax], e[kGmMax];  // Givens rotations, right-hand side
+  double y[kGmMax];                 // y_k / n_k, the combination's coefficients
+  double G[kGmMax * (kGmMax - 1) / 2];  // (u_k, u_j), j < k
+  double R[kGmMax * kGmMax];        // rotated columns
+};
+// An iteration's result, written by the device into its slot of pinned host
+// memory; seq last.
+struct GmHost {
+  int done;
+  double echeck;
+  long long acc_spmv, acc_gs;
+  unsigned seq;
+};
+
 // Learned preconditioner state (k_mpnn.hip); allocated by phg_mpnn_init.
 struct MpNet {
   bool ready = false;
@@ -232,8 +262,14 @@ struct phg_ctx {
   int* fold_ptr = nullptr;
   int* fold_slave = nullptr;
 
-  // block-CSR in groups of 64 rows ("slot" layout)
+  // block-CSR in groups of 64 rows ("slot" layout); a periodic master's
+  // slaves follow it in its group (fam_in_group), so that the matvec folds
+  // them.  A family of more than kGroup rows leaves the rows in natural order
+  // and the fold to k_fold_vec.
   long long ngroups = 0, nslots = 0;
+  bool fam_in_group = false;
+  int* rowmap = nullptr;           // ngroups*64 row of (group, lane), -1 padding
+  uint8_t* fam = nullptr;          // ngroups*64 slaves that follow, kFamSlave, or 0
   std::vector<long long> h_grp_slot;
   long long* grp_slot = nullptr;   // ngroups+1
   int* scol = nullptr;             // nslots*64 raw column (0-based)
@@ -269,12 +305,17 @@ struct phg_ctx {
   double* yold = nullptr;
   double* acold = nullptr;
   double* dy = nullptr;
-  double* krylov = nullptr;        // (Kspace+1) vectors of 5*nshg
+  double* krylov = nullptr;        // (Kspace+1) vectors, kstr doubles apart
+  long long kstr = 0;              // 5*nshg rounded up to even (16-byte loads)
   int kcap = 0;
 
   // reductions
   int red_blocks = 0;
-  double* red_part = nullptr;      // (kcap + 3) channels of red_blocks partials
+  double* red_part = nullptr;      // 2 (kcap + 2) channels of red_blocks partials
+  GmDev* gm = nullptr;             // the running GMRES cycle
+  GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
+  unsigned gm_seq = 0;             // token of the last iteration enqueued
+  double clk_ms = 0.0;             // ms per tick of the device clock
   double* scal = nullptr;          // device scalars (H column etc.)
   double* h_scal = nullptr;        // pinned mirror
   double reslast = 0.0;
@@ -320,8 +361,10 @@ int launch_jv(phg_ctx* c, const double* v, double* w);
 int launch_mres(phg_ctx* c, const double* yp, double* out, bool accumulate, bool iabs);
 // ypack = U^-1 (ypre + s d) per node in the local order (d may be nullptr;
 // without lu no U^-1), with itrBC's Dirichlet values and periodic copy when bc
+// dn (nullable): the norm that d is divided by; t0 (nullable): the device clock
+// at the start goes there
 int launch_mfg_point(phg_ctx* c, const double* ypre, const double* d, double s, double* ypack,
-                     bool bc, bool lu);
+                     bool bc, bool lu, const double* dn = nullptr, long long* t0 = nullptr);
 // w = (L^-1 t - rmes) / e
 int launch_mfg_fwd_diff(phg_ctx* c, const double* t, const double* rmes, double e, double* w);
 // mode 0: u = a - (u1 - u2) / h; mode 1: u = (u1 - 2 a) / h
@@ -352,7 +395,10 @@ int mp_load_pair(phg_ctx* c, int slot);
 // ---- launchers (k_solver.hip) ----
 int launch_i3lu(phg_ctx* c, double* diag, double* r, int code);
 int launch_spsi3pre(phg_ctx* c);
-int launch_spmv(phg_ctx* c, const double* p, double* q);
+// q = K p, folded (bc3per) when fold is set; skipped when *gate is set; the
+// device clock at its start into *t0 (both nullable)
+int launch_spmv(phg_ctx* c, const double* p, double* q, bool fold, const int* gate = nullptr,
+                long long* t0 = nullptr);
 int launch_sub(phg_ctx* c, double* r, const double* b, const double* q, long long n);
 // q = K^T x (x overwritten by its periodic gather); needs c->tslot
 int launch_spmv_t(phg_ctx* c, double* x, double* q);
@@ -369,17 +415,19 @@ int launch_dot(phg_ctx* c, const double* a, const double* b, long long n,
                double* out);
 int launch_dot_part(phg_ctx* c, const double* a, const double* b, long long n,
                     int chan, int* np);
-int launch_mgs_part(phg_ctx* c, double* u, const double* ujm1, const double* uj,
-                    int chan_prev, int np_prev, long long n, int chan, int* np);
 int launch_finish(phg_ctx* c, int chan0, int np0, int np, int nsums, double* out);
-// classical Gram-Schmidt of u against nv contiguous basis vectors:
-// h[0..nv-1] = (u, basis_j) of the incoming u, u -= sum h_j basis_j,
-// h[nv] = (u, u) afterwards
-int launch_cgs(phg_ctx* c, double* u, const double* basis, int nv, long long n, double* h);
+// Krylov iteration iK after its product w (of the basis vector as stored, or
+// with unit of the normalised one): orthogonalised against the iK basis
+// vectors, the Hessenberg column, its rotations and the convergence test; the
+// result goes to h_gm with the token seq.  Skipped on the device when an
+// earlier iteration ended the cycle.
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm,
+              unsigned seq);
 int launch_scale(phg_ctx* c, double* u, const double* src, long long n,
                  const double* sq_ptr, double* norm_out);
-int launch_combine(phg_ctx* c, double* dy, const double* basis, int k,
-                   const double* coef, long long n);
+// dy (+)= the cycle's combination: its first nz directions from zb (stride
+// 5*nshg), the others from the basis
+int launch_combine(phg_ctx* c, double* dy, const double* zb, int nz, bool add);
 int launch_stats(phg_ctx* c, double* out);
 int launch_csr_to_slots(phg_ctx* c, const double* ref, double* slots);
 int launch_pack_nodes(phg_ctx* c);

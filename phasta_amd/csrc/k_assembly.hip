@@ -128,6 +128,14 @@ struct QpArgs {
   PhysParams ph;
   double epsM;             // /precis/ epsM, regularises the DC norm
   int idc;                 // iDC 1, 2, 3 (only read when the kernel has kDC)
+  // wall elements, by the workgroups past the interior ones (one launch for
+  // both: 7 launches of 4 to 6 us when each wall colour had its own)
+  const int* ienb;         // 4 planes of nelb, colour order
+  double* wres;            // 5 per (wall element, face node), at wslot
+  const int* wslot;
+  long long nelb;
+  int qp_groups;           // workgroups of the interior elements
+  long long* clk;          // device clock at the start
 };
 
 __device__ inline double sel4(double v0, double v1, double v2, double v3, int i) {
@@ -587,6 +595,123 @@ __device__ inline void compact_k(const double ix[3][3], double T, double mu, dou
 template <typename S>
 constexpr int mt_stride() { return sizeof(S) == 8 ? 26 : 28; }
 
+// Wall faces: floating convective, pressure, viscous and heat fluxes
+// (iBCB = 0), residual only (iLHScond = 0).  Nodes 1..3 lie on the face,
+// ordered so (x2-x1) x (x3-x1) points outward.  The element's
+// contributions to its face nodes go to wres, a node's together and in
+// wall-colour order; k_boundary_nodes adds them in that order.
+__device__ __forceinline__ void wall_element(const QpArgs& A, long long p) {
+  const long long nelb = A.nelb;
+  if (p >= nelb) return;
+  const PhysParams& ph = A.ph;
+  double yl[4][5], xl[4][3];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const double* v = A.node + 16 * (size_t)A.ienb[a * nelb + p];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) yl[a][f] = v[f];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) xl[a][c] = v[10 + c];
+  }
+  // volume metrics for the gradients
+  double d[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) d[i][j] = 0.5 * (xl[j][i] - xl[3][i]);
+  double ix[3][3];
+  ix[0][0] = d[1][1] * d[2][2] - d[2][1] * d[1][2];
+  ix[0][1] = d[2][1] * d[0][2] - d[0][1] * d[2][2];
+  ix[0][2] = d[0][1] * d[1][2] - d[0][2] * d[1][1];
+  const double idet = 1.0 / (ix[0][0] * d[0][0] + ix[0][1] * d[1][0] + ix[0][2] * d[2][0]);
+  ix[0][0] *= idet;
+  ix[0][1] *= idet;
+  ix[0][2] *= idet;
+  ix[1][0] = (d[1][2] * d[2][0] - d[1][0] * d[2][2]) * idet;
+  ix[1][1] = (d[0][0] * d[2][2] - d[2][0] * d[0][2]) * idet;
+  ix[1][2] = (d[1][0] * d[0][2] - d[0][0] * d[1][2]) * idet;
+  ix[2][0] = (d[1][0] * d[2][1] - d[1][1] * d[2][0]) * idet;
+  ix[2][1] = (d[2][0] * d[0][1] - d[0][0] * d[2][1]) * idet;
+  ix[2][2] = (d[0][0] * d[1][1] - d[0][1] * d[1][0]) * idet;
+  double shg[4][3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    shg[0][k] = 0.5 * ix[0][k];
+    shg[1][k] = 0.5 * ix[1][k];
+    shg[2][k] = 0.5 * ix[2][k];
+    shg[3][k] = -0.5 * (ix[0][k] + ix[1][k] + ix[2][k]);
+  }
+  double g[3][5];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int f = 0; f < 5; ++f)
+      g[i][f] = shg[0][i] * yl[0][f] + shg[1][i] * yl[1][f] + shg[2][i] * yl[2][f] +
+                shg[3][i] * yl[3][f];
+  // outward unit normal and weighted area
+  double v1[3], v2[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    v1[c] = xl[1][c] - xl[0][c];
+    v2[c] = xl[2][c] - xl[0][c];
+  }
+  double nrm[3] = {v1[1] * v2[2] - v2[1] * v1[2], v2[0] * v1[2] - v1[0] * v2[2],
+                   v1[0] * v2[1] - v2[0] * v1[1]};
+  const double area2 = sqrt(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2]);
+  const double inv = 1.0 / area2;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) nrm[c] *= inv;
+  const double WdetJb = cQ.Qwtb * area2 * 0.25;
+
+  const double cp = ph.Rgas * ph.gamma / ph.gamma1;
+  const double mu = ph.mu, lam = -(2.0 / 3.0) * mu, kap = mu * cp / ph.pr;
+  const double divu = g[0][1] + g[1][2] + g[2][3];
+  // wall traction and heat flux use the volume gradients (constant)
+  double tn[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    double acc = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      acc += nrm[i] * (mu * (g[i][1 + m] + g[m][1 + i]) + (m == i ? lam * divu : 0.0));
+    tn[m] = acc;
+  }
+  const double heat = -kap * (nrm[0] * g[0][4] + nrm[1] * g[1][4] + nrm[2] * g[2][4]);
+
+  double rl[3][5];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int f = 0; f < 5; ++f) rl[a][f] = 0.0;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const double* Nq = cQ.Nb[q];
+    double Y[5];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) Y[f] = Nq[0] * yl[0][f] + Nq[1] * yl[1][f] + Nq[2] * yl[2][f];
+    const double pres = Y[0], u1 = Y[1], u2 = Y[2], u3 = Y[3], Tq = Y[4];
+    const double rk = 0.5 * (u1 * u1 + u2 * u2 + u3 * u3);
+    const double rho = pres / (ph.Rgas * Tq);
+    const double ei = Tq * (ph.Rgas / ph.gamma1);
+    const double un = nrm[0] * u1 + nrm[1] * u2 + nrm[2] * u3;
+    const double rou = rho * un;
+    double F[5];
+    F[0] = rou;
+    F[1] = rou * u1 + nrm[0] * pres - tn[0];
+    F[2] = rou * u2 + nrm[1] * pres - tn[1];
+    F[3] = rou * u3 + nrm[2] * pres - tn[2];
+    F[4] = rou * (ei + rk) + un * pres - (u1 * tn[0] + u2 * tn[1] + u3 * tn[2]) + heat;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int f = 0; f < 5; ++f) rl[a][f] += WdetJb * Nq[a] * F[f];
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int f = 0; f < 5; ++f) A.wres[(size_t)A.wslot[3 * p + a] * 5 + f] = rl[a][f];
+}
+
 // ---------------- pass 1: point states and residual ----------------
 // S: storage type of the point states and geometry (double, or float for
 // the mixed-precision path whose tangent is formed in float).  kDiff: the
@@ -598,6 +723,11 @@ constexpr int mt_stride() { return sizeof(S) == 8 ? 26 : 28; }
 // tau; W PTau is kept for the tangent pass.
 template <typename S, bool kDiff, bool kDC, bool kMT>
 __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
+  if ((int)blockIdx.x >= A.qp_groups) {
+    wall_element(A, (long long)(blockIdx.x - A.qp_groups) * 256 + threadIdx.x);
+    return;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.clk = wall_clock64();
   const long long e_raw = blockIdx.x * 64LL + threadIdx.x / 4;
   const int q = threadIdx.x & 3;
   const bool valid = e_raw < A.nel;
@@ -1299,6 +1429,7 @@ struct BlkArgs {
   long long nel, nlanes;
   int lhs_on, prec_on;
   double mu, lam, kap, cfac;
+  long long* clk;          // device clock at the start
 };
 
 // T: stored block type and arithmetic type of the per-point tangent (float
@@ -1316,6 +1447,7 @@ struct BlkArgs {
 template <typename T, typename S, bool kDC, bool kMT, bool kNd = false>
 __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
   using R = T;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.clk = wall_clock64();
   // consecutive workgroups run on different XCDs (round robin over 8): give
   // each XCD a contiguous range of lanes so its L2 sees neighbouring blocks
   const long long per = (gridDim.x + 7) / 8;
@@ -1597,6 +1729,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
 template <typename T, typename S, bool kDC, bool kMT>
 __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
   using R = T;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.clk = wall_clock64();
   const long long per = (gridDim.x + 7) / 8;
   const long long wg = (blockIdx.x % 8) * per + blockIdx.x / 8;
   const long long l = wg * 64 + threadIdx.x;
@@ -1820,175 +1953,12 @@ __global__ void __launch_bounds__(64) k_asm_pairs_dcmt(BlkArgs A) {
   asm_pairs<float, float, kDC, kMT>(A);
 }
 
-// Wall faces: floating convective, pressure, viscous and heat fluxes
-// (iBCB = 0), residual only (iLHScond = 0).  Nodes 1..3 lie on the face,
-// ordered so (x2-x1) x (x3-x1) points outward.
-struct WallArgs {
-  const int* ien;   // 4 planes of nelb, colour order
-  const double* node;
-  double* res;      // 5 per node
-  long long nshg, nelb;
-  int p0, p1;
-  PhysParams ph;
-};
-
-__global__ void __launch_bounds__(64) k_wall(WallArgs A) {
-  const int p = A.p0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= A.p1) return;
-  const long long nshg = A.nshg, nelb = A.nelb;
-  const PhysParams& ph = A.ph;
-  int nd[4];
-  double yl[4][5], xl[4][3];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    nd[a] = A.ien[a * nelb + p];
-    const double* v = A.node + 16 * (size_t)nd[a];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) yl[a][f] = v[f];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) xl[a][c] = v[10 + c];
-  }
-  // volume metrics for the gradients
-  double d[3][3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) d[i][j] = 0.5 * (xl[j][i] - xl[3][i]);
-  double ix[3][3];
-  ix[0][0] = d[1][1] * d[2][2] - d[2][1] * d[1][2];
-  ix[0][1] = d[2][1] * d[0][2] - d[0][1] * d[2][2];
-  ix[0][2] = d[0][1] * d[1][2] - d[0][2] * d[1][1];
-  const double idet = 1.0 / (ix[0][0] * d[0][0] + ix[0][1] * d[1][0] + ix[0][2] * d[2][0]);
-  ix[0][0] *= idet;
-  ix[0][1] *= idet;
-  ix[0][2] *= idet;
-  ix[1][0] = (d[1][2] * d[2][0] - d[1][0] * d[2][2]) * idet;
-  ix[1][1] = (d[0][0] * d[2][2] - d[2][0] * d[0][2]) * idet;
-  ix[1][2] = (d[1][0] * d[0][2] - d[0][0] * d[1][2]) * idet;
-  ix[2][0] = (d[1][0] * d[2][1] - d[1][1] * d[2][0]) * idet;
-  ix[2][1] = (d[2][0] * d[0][1] - d[0][0] * d[2][1]) * idet;
-  ix[2][2] = (d[0][0] * d[1][1] - d[0][1] * d[1][0]) * idet;
-  double shg[4][3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    shg[0][k] = 0.5 * ix[0][k];
-    shg[1][k] = 0.5 * ix[1][k];
-    shg[2][k] = 0.5 * ix[2][k];
-    shg[3][k] = -0.5 * (ix[0][k] + ix[1][k] + ix[2][k]);
-  }
-  double g[3][5];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int f = 0; f < 5; ++f)
-      g[i][f] = shg[0][i] * yl[0][f] + shg[1][i] * yl[1][f] + shg[2][i] * yl[2][f] +
-                shg[3][i] * yl[3][f];
-  // outward unit normal and weighted area
-  double v1[3], v2[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    v1[c] = xl[1][c] - xl[0][c];
-    v2[c] = xl[2][c] - xl[0][c];
-  }
-  double nrm[3] = {v1[1] * v2[2] - v2[1] * v1[2], v2[0] * v1[2] - v1[0] * v2[2],
-                   v1[0] * v2[1] - v2[0] * v1[1]};
-  const double area2 = sqrt(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2]);
-  const double inv = 1.0 / area2;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) nrm[c] *= inv;
-  const double WdetJb = cQ.Qwtb * area2 * 0.25;
-
-  const double cp = ph.Rgas * ph.gamma / ph.gamma1;
-  const double mu = ph.mu, lam = -(2.0 / 3.0) * mu, kap = mu * cp / ph.pr;
-  const double divu = g[0][1] + g[1][2] + g[2][3];
-  // wall traction and heat flux use the volume gradients (constant)
-  double tn[3];
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    double acc = 0.0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      acc += nrm[i] * (mu * (g[i][1 + m] + g[m][1 + i]) + (m == i ? lam * divu : 0.0));
-    tn[m] = acc;
-  }
-  const double heat = -kap * (nrm[0] * g[0][4] + nrm[1] * g[1][4] + nrm[2] * g[2][4]);
-
-  double rl[3][5];
-#pragma unroll
-  for (int a = 0; a < 3; ++a)
-#pragma unroll
-    for (int f = 0; f < 5; ++f) rl[a][f] = 0.0;
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const double* Nq = cQ.Nb[q];
-    double Y[5];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) Y[f] = Nq[0] * yl[0][f] + Nq[1] * yl[1][f] + Nq[2] * yl[2][f];
-    const double pres = Y[0], u1 = Y[1], u2 = Y[2], u3 = Y[3], Tq = Y[4];
-    const double rk = 0.5 * (u1 * u1 + u2 * u2 + u3 * u3);
-    const double rho = pres / (ph.Rgas * Tq);
-    const double ei = Tq * (ph.Rgas / ph.gamma1);
-    const double un = nrm[0] * u1 + nrm[1] * u2 + nrm[2] * u3;
-    const double rou = rho * un;
-    double F[5];
-    F[0] = rou;
-    F[1] = rou * u1 + nrm[0] * pres - tn[0];
-    F[2] = rou * u2 + nrm[1] * pres - tn[1];
-    F[3] = rou * u3 + nrm[2] * pres - tn[2];
-    F[4] = rou * (ei + rk) + un * pres - (u1 * tn[0] + u2 * tn[1] + u3 * tn[2]) + heat;
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int f = 0; f < 5; ++f) rl[a][f] += WdetJb * Nq[a] * F[f];
-  }
-#pragma unroll
-  for (int a = 0; a < 3; ++a)
-#pragma unroll
-    for (int f = 0; f < 5; ++f) A.res[5 * (size_t)nd[a] + f] += rl[a][f];
-}
-
-// Accumulation layout -> reference planes, with the Dirichlet rows of res
-// and BDiag (bc3res.f:25-153, bc3bdg.f:25-330)
-// The assembly leaves res (5) and BDiag (25) per node contiguous; a block of
-// 128 nodes stages its records through LDS (coalesced reads) and writes the
-// Dirichlet-masked values as planes.
-__global__ void __launch_bounds__(128) k_bc_nodes(const double* __restrict__ ares,
-                                                  const double* __restrict__ abd,
-                                                  double* __restrict__ res,
-                                                  double* __restrict__ bdiag,
-                                                  const uint8_t* __restrict__ bcm, long long nshg,
-                                                  int prec) {
-  __shared__ double sb[128 * 25];
-  const long long n0 = blockIdx.x * 128LL;
-  const int cnt = (int)(nshg - n0 < 128 ? nshg - n0 : 128);
-  const int t = threadIdx.x;
-  const long long n = n0 + t;
-  for (int k = t; k < 5 * cnt; k += 128) sb[k] = ares[5 * n0 + k];
-  __syncthreads();
-  const uint8_t m = t < cnt ? bcm[n] : 0;
-  if (t < cnt) {
-#pragma unroll
-    for (int f = 0; f < 5; ++f) res[n + f * nshg] = ((m >> f) & 1) ? 0.0 : sb[5 * t + f];
-  }
-  if (!prec) return;
-  __syncthreads();
-  for (int k = t; k < 25 * cnt; k += 128) sb[k] = abd[25 * n0 + k];
-  __syncthreads();
-  if (t >= cnt) return;
-#pragma unroll
-  for (int j = 0; j < 5; ++j)
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      double v = sb[25 * t + i + 5 * j];
-      if (((m >> i) & 1) || ((m >> j) & 1)) v = (i == j) ? 1.0 : 0.0;
-      bdiag[n + (i + 5 * j) * nshg] = v;
-    }
-}
 
 // y, ac (global order, planes) and x -> one 16-double line per node
 __global__ void k_pack_nodes(const double* y, const double* ac, const double* x, double* pack,
-                             long long nshg) {
+                             long long nshg, long long* clk) {
   long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (n == 0) *clk = wall_clock64();
   if (n >= nshg) return;
   double v[16];
   gather_local(y, nshg, (int)n, v);
@@ -2000,36 +1970,6 @@ __global__ void k_pack_nodes(const double* y, const double* ac, const double* x,
   double2* d = reinterpret_cast<double2*>(pack + 16 * n);
 #pragma unroll
   for (int k = 0; k < 8; ++k) d[k] = make_double2(v[2 * k], v[2 * k + 1]);
-}
-
-// Periodic fold: res(master) += res(slaves) in ascending slave order, slave
-// rows zeroed; BDiag(master) += BDiag(slaves), then slaves copy the master
-// (bc3res.f:157-163, bc3bdg.f:338-352).
-__global__ void k_fold_res_bdiag(double* res, double* bdiag, const int* master,
-                                 const int* ptr, const int* slave, int nfold,
-                                 long long nshg, int prec) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nfold) return;
-  const long long m = master[i];
-  for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const long long s = slave[k];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      res[m + f * nshg] += res[s + f * nshg];
-      res[s + f * nshg] = 0.0;
-    }
-  }
-  if (!prec) return;
-  for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const long long s = slave[k];
-#pragma unroll
-    for (int e = 0; e < 25; ++e) bdiag[m + e * nshg] += bdiag[s + e * nshg];
-  }
-  for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const long long s = slave[k];
-#pragma unroll
-    for (int e = 0; e < 25; ++e) bdiag[s + e * nshg] = bdiag[m + e * nshg];
-  }
 }
 
 // ---------------- global reconstruction of the diffusive flux ----------------
@@ -2397,7 +2337,7 @@ __global__ void __launch_bounds__(256) k_mres(MresArgs A) {
 // out (+)= the sum of the node's element contributions in element order
 // (the scatter of asires.f:91 / asimfg.f:96; read from the incidence slots
 // k_mres writes), then bc3Res's Dirichlet rows
-// (bc3res.f:25-153); the periodic fold follows (k_fold_res_bdiag)
+// (bc3res.f:25-153); the periodic fold follows (k_fold_vec)
 __global__ void __launch_bounds__(256) k_mres_nodes(const long long* __restrict__ goff,
                                                     const int* __restrict__ inc,
                                                     const double* __restrict__ resid,
@@ -2590,7 +2530,8 @@ int launch_fill(phg_ctx* c, void* p, size_t bytes) {
 
 int launch_pack_nodes(phg_ctx* c) {
   const long long n = c->nshg;
-  k_pack_nodes<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->y, c->ac, c->x, c->nodepack, n);
+  k_pack_nodes<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->y, c->ac, c->x, c->nodepack, n,
+                                                              &c->gm->ta[0]);
   PHG_HIP(hipGetLastError());
   return 0;
 }
@@ -2653,14 +2594,18 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
   Q.mtau = c->mtau;
   Q.epsM = c->prm.epsM;
   Q.idc = c->prm.idc;
-  const int g1 = (int)((c->nel + 63) / 64);
-  PHG_HIP(hipEventRecord(c->aev[0], c->stream));
+  Q.ienb = c->ienbc;
+  Q.wres = c->wres;
+  Q.wslot = c->wslot;
+  Q.nelb = c->nelb;
+  Q.qp_groups = (int)((c->nel + 63) / 64);
+  Q.clk = &c->gm->ta[1];
+  const int g1 = Q.qp_groups + (int)((c->nelb + 255) / 256);
   if (mixed)
     launch_qp<float>(g1, c->stream, Q, diff, dc, mt);
   else
     launch_qp<double>(g1, c->stream, Q, diff, dc, mt);
   PHG_HIP(hipGetLastError());
-  PHG_HIP(hipEventRecord(c->aev[1], c->stream));
   // pass 2: block owners (res, BDiag, lhsK written once)
   BlkArgs B{};
   // without lhsK only the diagonal entries' owners have work (the node's
@@ -2690,6 +2635,7 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
   B.lam = -(2.0 / 3.0) * ph.mu;
   B.kap = ph.mu * cp / ph.pr;
   B.cfac = ph.almi / ph.gami / ph.alfi * ph.Dtgl;
+  B.clk = &c->gm->ta[2];
   const int g2 = (int)(((B.nlanes + 63) / 64 + 7) / 8 * 8);  // whole XCD rounds
   if (paired && mixed && dc && mt)
     k_asm_pairs_dcmt<true, true><<<g2, 64, 0, c->stream>>>(B);
@@ -2719,23 +2665,6 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
     k_asm_blocks<double, double, true, false><<<g2, 64, 0, c->stream>>>(B);
   else
     k_asm_blocks<double, double, false, false><<<g2, 64, 0, c->stream>>>(B);
-  PHG_HIP(hipGetLastError());
-  PHG_HIP(hipEventRecord(c->aev[2], c->stream));
-  // wall faces: residual only, added colour by colour
-  WallArgs W{};
-  W.ien = c->ienbc;
-  W.node = c->nodepack;
-  W.res = c->acc_res;
-  W.nshg = c->nshg;
-  W.nelb = c->nelb;
-  W.ph = ph;
-  for (size_t k = 0; k + 1 < c->colb_off.size(); ++k) {
-    W.p0 = c->colb_off[k];
-    W.p1 = c->colb_off[k + 1];
-    int n = W.p1 - W.p0;
-    if (n <= 0) continue;
-    k_wall<<<(n + 63) / 64, 64, 0, c->stream>>>(W);
-  }
   PHG_HIP(hipGetLastError());
   return 0;
 }
@@ -2781,19 +2710,6 @@ int launch_jv(phg_ctx* c, const double* v, double* w) {
   return launch_bc3per(c, w, 5);
 }
 
-int launch_bc_res_bdiag(phg_ctx* c, bool prec) {
-  long long n = c->nshg;
-  k_bc_nodes<<<(int)((n + 127) / 128), 128, 0, c->stream>>>(c->acc_res, c->acc_bd, c->res, c->bdiag,
-                                                             c->bcm, n, prec);
-  PHG_HIP(hipGetLastError());
-  if (c->nfold > 0) {
-    k_fold_res_bdiag<<<(c->nfold + 255) / 256, 256, 0, c->stream>>>(
-        c->res, c->bdiag, c->fold_master, c->fold_ptr, c->fold_slave, c->nfold, n, prec);
-    PHG_HIP(hipGetLastError());
-  }
-  return 0;
-}
-
 // The modified residual of the variables yp (stride 8, packed by
 // launch_mfg_point; nullptr: y itself, ElmMFG) at the resident state,
 // summed into out (accumulate: added to out's values), Dirichlet rows
@@ -2829,12 +2745,7 @@ int launch_mres(phg_ctx* c, const double* yp, double* out, bool accumulate, bool
   k_mres_nodes<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->inc_goff, c->inc, c->resid,
                                                               c->bcm, out, n, accumulate ? 1 : 0);
   PHG_HIP(hipGetLastError());
-  if (c->nfold > 0) {
-    k_fold_res_bdiag<<<(c->nfold + 255) / 256, 256, 0, c->stream>>>(
-        out, nullptr, c->fold_master, c->fold_ptr, c->fold_slave, c->nfold, n, 0);
-    PHG_HIP(hipGetLastError());
-  }
-  return 0;
+  return launch_bc3per(c, out, 5);
 }
 
 int launch_mfg_point(phg_ctx* c, const double* ypre, const double* d, double s, double* ypack,

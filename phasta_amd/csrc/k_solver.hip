@@ -20,18 +20,11 @@ constexpr int kRedThreads = 256;
 
 // ---------------- block LU (i3lu.f) ----------------
 // 25 planes, D[(i + 5 j) * n + node] = Diag(node, i+1, j+1)
-__global__ void k_lu_fact(double* D, long long n) {
-  long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  double a[5][5];
-#pragma unroll
-  for (int j = 0; j < 5; ++j)
-#pragma unroll
-    for (int i = 0; i < 5; ++i) a[i][j] = D[(i + 5 * j) * n + k];
-  // Doolittle: unit-lower L, upper U with its diagonal stored inverted.
-  // As in the reference (i3lu.f:82-97) the entry U(4,5) is never reduced:
-  // row 4 of U only gets its diagonal, so (4,5) keeps the raw BDiag value
-  // and the forward/backward sweeps use it as such.
+// Doolittle: unit-lower L, upper U with its diagonal stored inverted.  As in
+// the reference (i3lu.f:82-97) the entry U(4,5) is never reduced: row 4 of U
+// only gets its diagonal, so (4,5) keeps the raw BDiag value and the
+// forward/backward sweeps use it as such.
+__device__ inline void lu_factor(double a[5][5]) {
 #pragma unroll
   for (int p = 0; p < 5; ++p) {
 #pragma unroll
@@ -51,6 +44,27 @@ __global__ void k_lu_fact(double* D, long long n) {
       a[i][p] = a[p][p] * s;
     }
   }
+}
+
+__device__ inline void lu_solve_lower(const double a[5][5], double v[5]) {
+#pragma unroll
+  for (int i = 1; i < 5; ++i) {
+    double s = v[i];
+#pragma unroll
+    for (int m = 0; m < i; ++m) s -= a[i][m] * v[m];
+    v[i] = s;
+  }
+}
+
+__global__ void k_lu_fact(double* D, long long n) {
+  long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  double a[5][5];
+#pragma unroll
+  for (int j = 0; j < 5; ++j)
+#pragma unroll
+    for (int i = 0; i < 5; ++i) a[i][j] = D[(i + 5 * j) * n + k];
+  lu_factor(a);
 #pragma unroll
   for (int j = 0; j < 5; ++j)
 #pragma unroll
@@ -60,16 +74,14 @@ __global__ void k_lu_fact(double* D, long long n) {
 __global__ void k_lu_forward(const double* D, double* r, long long n) {
   long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (k >= n) return;
-  double v[5];
+  double v[5], a[5][5];
 #pragma unroll
   for (int i = 0; i < 5; ++i) v[i] = r[i * n + k];
 #pragma unroll
-  for (int i = 1; i < 5; ++i) {
-    double s = v[i];
+  for (int i = 1; i < 5; ++i)
 #pragma unroll
-    for (int m = 0; m < i; ++m) s -= D[(i + 5 * m) * n + k] * v[m];
-    v[i] = s;
-  }
+    for (int m = 0; m < i; ++m) a[i][m] = D[(i + 5 * m) * n + k];
+  lu_solve_lower(a, v);
 #pragma unroll
   for (int i = 1; i < 5; ++i) r[i * n + k] = v[i];
 }
@@ -389,19 +401,20 @@ __global__ void k_ref_to_aos(const double* __restrict__ ref, double* __restrict_
 }
 
 
-// bc3per: master += slaves (ascending), slaves zeroed
+// bc3per: master += slaves (ascending), slaves zeroed; one lane per master
+// and plane
 __global__ void k_fold_vec(double* v, const int* master, const int* ptr, const int* slave,
-                           int nfold, long long n, int nq) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+                           int nfold, long long n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nfold) return;
+  double* p = v + (size_t)blockIdx.y * n;
   const long long m = master[i];
+  double s = p[m];
   for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const long long s = slave[k];
-    for (int f = 0; f < nq; ++f) {
-      v[m + f * n] += v[s + f * n];
-      v[s + f * n] = 0.0;
-    }
+    s += p[slave[k]];
+    p[slave[k]] = 0.0;
   }
+  p[m] = s;
 }
 
 // ---------------- deterministic reductions ----------------
@@ -588,7 +601,8 @@ struct GsArgs {
   long long n, kstr;     // length, stride between basis vectors (even)
   int nv, K, minIters;   // nv: the iteration number, 1..K
   int unit;              // w is the product of u_i, not of w_i
-  double unorm, epsnrm;  // of the cycle; the start vector has norm 1
+  double unorm, epsnrm;  // of the cycle
+  double n0;             // norm of the start vector as stored
   double* part;          // 2 nv channels of `chan` partials
   long long chan;
   GmDev* gm;
@@ -661,7 +675,7 @@ __global__ void __launch_bounds__(kGsThreads) k_gs_dots(GsArgs A) {
       }
     }
   }
-  if ((int)threadIdx.x < nv) nr[threadIdx.x] = nv > 1 ? gm.nrm[threadIdx.x] : 1.0;
+  if ((int)threadIdx.x < nv) nr[threadIdx.x] = nv > 1 ? gm.nrm[threadIdx.x] : A.n0;
   __syncthreads();
   if ((int)threadIdx.x < 2 * nv) {
     const int ch = threadIdx.x;
@@ -700,7 +714,7 @@ __global__ void __launch_bounds__(kGsThreads) k_gs_dots(GsArgs A) {
   if (lane == 0) {
     gm.scale = 1.0 / nw;
     if (nv == 1) {
-      gm.nrm[0] = 1.0;
+      gm.nrm[0] = A.n0;
       gm.done = 0;
       gm.e[0] = A.unorm;
       gm.acc_spmv = gm.acc_gs = 0;
@@ -855,15 +869,226 @@ __global__ void __launch_bounds__(256) k_combine(double* __restrict__ dy,
   }
 }
 
-// stats: [sum res^2, sum rmes^2, nan/large counts of res, BDiag]
-__global__ void __launch_bounds__(kRedThreads) k_stat_bad(const double* a, long long n, double* part) {
-  double v = 0.0;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const double x = a[i];
-    if (x != x || fabs(x) > 1.0e10) v += 1.0;
+// ---------------- nodal work after the assembly ----------------
+// The assembly leaves res (5) and BDiag (25) per node contiguous and the wall
+// elements' contributions apart.  Per node: wall contributions, the Dirichlet
+// rows and columns (bc3res.f:25-153, bc3bdg.f:25-330) and the periodic fold
+// (res: master += slaves ascending, slaves zero, bc3res.f:157-163; BDiag:
+// master += slaves, slaves copy it, bc3bdg.f:338-352).  With kSolve also what
+// SolGMRs does per node before its Krylov loop: tnanq's count on res and
+// BDiag, rmes, the LU factors, L^-1 res (also into the start vector) and the
+// two sums of squares (solgmr.f:459-490), so each node's 30 values are read
+// once and its 40 written once.
+//
+// k_boundary_nodes forms the sums of the few nodes with several sources (a
+// periodic family, wall faces) with one lane per value, so that their chains
+// of dependent loads run side by side; in k_nodes' own lanes they held up
+// nearly every wavefront of a box (27.9 us at 4^3, 557 us at 128^3 against
+// 15 and 310 us for both kernels).  k_nodes is bound by its bytes (0.5
+// KB per node) from 64^3 on, by launches below.
+constexpr int kNodeThreads = 256;
+constexpr int kNodeBlocks = 1024;
+
+struct NodeArgs {
+  const double* ares;      // 5 per node
+  const double* abd;       // 25 per node
+  const double* wres;      // 5 per contribution
+  int nspec;
+  const int* sptr;         // members of a boundary group
+  const int* smem;
+  const int* wptr;         // wall contributions of a member
+  double* ssum;            // 32 per group: BDiag (25), res (5)
+  const int2* info;        // boundary group, family (-1 without)
+  const uint8_t* bcm;
+  double* res;
+  double* rmes;
+  double* start;
+  double* bdiag;
+  double* raw;             // BDiag before factorisation, nullable
+  long long n;
+  int prec;
+  double* part;            // 3 channels of kNodeBlocks partials
+  GmDev* gm;
+  SolveHost* host;
+  unsigned seq;
+};
+
+// value e of a node after the Dirichlet rows and columns: e < 25 BDiag (row
+// e % 5, column e / 5), else res
+__device__ inline double masked(double v, int e, uint8_t m) {
+  if (e >= 25) return (m >> (e - 25)) & 1 ? 0.0 : v;
+  const int i = e % 5, j = e / 5;
+  return ((m >> i) & 1) || ((m >> j) & 1) ? (i == j ? 1.0 : 0.0) : v;
+}
+
+// one lane per (group, value)
+__global__ void __launch_bounds__(256) k_boundary_nodes(NodeArgs A) {
+  const long long at = blockIdx.x * 256LL + threadIdx.x;
+  const int g = (int)(at >> 5), e = (int)(at & 31);
+  if (g >= A.nspec || e >= 30 || (e < 25 && !A.prec)) return;
+  double s = 0.0;
+  for (int q = A.sptr[g]; q < A.sptr[g + 1]; ++q) {
+    const long long k = A.smem[q];
+    double v = e < 25 ? A.abd[25 * k + e] : A.ares[5 * k + e - 25];
+    if (e >= 25) {
+      const int w1 = A.wptr[q + 1];
+#pragma unroll 4
+      for (int w = A.wptr[q]; w < w1; ++w) v += A.wres[5 * (size_t)w + e - 25];
+    }
+    s += masked(v, e, A.bcm[k]);
   }
-  block_partial(v, part);
+  A.ssum[32 * (size_t)g + e] = s;
+}
+
+__device__ inline double is_bad(double x) { return x != x || fabs(x) > 1.0e10 ? 1.0 : 0.0; }
+
+template <bool kSolve>
+__global__ void __launch_bounds__(kNodeThreads) k_nodes(NodeArgs A) {
+  const int t = threadIdx.x;
+  const long long n = A.n;
+  // agent scope: the last workgroup reads it, perhaps from another XCD
+  if (blockIdx.x == 0 && t == 0)
+    __hip_atomic_store(&A.gm->ta[3], wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double s_res = 0.0, s_rmes = 0.0, bad = 0.0;
+  for (long long k = blockIdx.x * (long long)kNodeThreads + t; k < n;
+       k += gridDim.x * (long long)kNodeThreads) {
+    const int2 in = A.info[k];
+    const uint8_t m = A.bcm[k];
+    const bool sp = in.x >= 0;
+    const double* rr = sp ? A.ssum + 32 * (size_t)in.x + 25 : A.ares + 5 * k;
+    const double* rb = sp ? A.ssum + 32 * (size_t)in.x : A.abd + 25 * k;
+    // a family's sums belong to its master; the slaves' res is zero
+    const bool slave = in.y >= 0 && A.smem[A.sptr[in.x]] != k;
+    double r[5], a[5][5];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) r[f] = rr[f];
+    if (A.prec) {
+#pragma unroll
+      for (int j = 0; j < 5; ++j)
+#pragma unroll
+        for (int i = 0; i < 5; ++i) a[i][j] = rb[i + 5 * j];
+    }
+    if (!sp && m) {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) r[f] = masked(r[f], 25 + f, m);
+      if (A.prec) {
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) a[i][j] = masked(a[i][j], i + 5 * j, m);
+      }
+    }
+    if (slave) {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) r[f] = 0.0;
+    }
+    if constexpr (kSolve) {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) {
+        A.rmes[k + f * n] = r[f];
+        bad += is_bad(r[f]);
+        s_rmes += r[f] * r[f];
+      }
+      if (A.prec) {
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) {
+            bad += is_bad(a[i][j]);
+            if (A.raw) A.raw[k + (i + 5 * j) * n] = a[i][j];
+          }
+        lu_factor(a);
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) A.bdiag[k + (i + 5 * j) * n] = a[i][j];
+      } else {
+        // the factors of an earlier call (solgmr.f:471)
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) {
+            a[i][j] = A.bdiag[k + (i + 5 * j) * n];
+            bad += is_bad(a[i][j]);
+          }
+      }
+      lu_solve_lower(a, r);
+#pragma unroll
+      for (int f = 0; f < 5; ++f) {
+        A.res[k + f * n] = r[f];
+        A.start[k + f * n] = r[f];
+        s_res += r[f] * r[f];
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) A.res[k + f * n] = r[f];
+      if (A.prec) {
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) A.bdiag[k + (i + 5 * j) * n] = a[i][j];
+      }
+    }
+  }
+  if constexpr (kSolve) {
+    __shared__ double ws[3][kNodeThreads / 64];
+    auto block_sums = [&](double out[3]) {
+      s_res = wave_sum(s_res);
+      s_rmes = wave_sum(s_rmes);
+      bad = wave_sum(bad);
+      if ((t & 63) == 0) {
+        ws[0][t >> 6] = s_res;
+        ws[1][t >> 6] = s_rmes;
+        ws[2][t >> 6] = bad;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < 3; ++c) out[c] = ws[c][0] + ws[c][1] + ws[c][2] + ws[c][3];
+    };
+    double sum[3];
+    block_sums(sum);
+    if (t == 0) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) part_store(A.part + c * kNodeBlocks + blockIdx.x, sum[c]);
+    }
+    if (!arrive_last(&A.gm->cnt)) return;
+    double v[3][kNodeBlocks / kNodeThreads];
+#pragma unroll
+    for (int u = 0; u < kNodeBlocks / kNodeThreads; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const int b = t + kNodeThreads * u;
+        v[c][u] = b < (int)gridDim.x ? part_load(A.part + c * kNodeBlocks + b) : 0.0;
+      }
+    s_res = s_rmes = bad = 0.0;
+#pragma unroll
+    for (int u = 0; u < kNodeBlocks / kNodeThreads; ++u) {
+      s_res += v[0][u];
+      s_rmes += v[1][u];
+      bad += v[2][u];
+    }
+    block_sums(sum);
+    if (t != 0) return;
+    SolveHost* h = A.host;
+    const long long now = wall_clock64();
+    const long long ta3 =
+        __hip_atomic_load(&A.gm->ta[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const long long ta[5] = {A.gm->ta[0], A.gm->ta[1], A.gm->ta[2], ta3, now};
+    __hip_atomic_store(&h->sumsq, sum[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&h->sumsq_m, sum[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&h->bad, sum[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      __hip_atomic_store(&h->ta[k], ta[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&h->seq, A.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+__global__ void k_end_mark(SolveHost* h, unsigned seq) {
+  __hip_atomic_store(&h->end, wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __hip_atomic_store(&h->end_seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------- layout conversion ----------------
@@ -887,69 +1112,77 @@ __global__ void k_slots_to_csr(const T* slots, double* ref, const uint32_t* c2s,
   for (int e = 0; e < 25; ++e) ref[k * 25 + e] = (double)src[slot_pos<T>(e, (int)(qs & 63))];
 }
 
-// ---------------- itrPredict / itrCorrect / itrBC ----------------
-// itrPredict, same-velocity predictor (itrPC.f:67-73): y = yold,
-// ac = acold (1 - almi/gami)
-__global__ void k_predict(const double* yold, const double* acold, double* y, double* ac,
-                          long long n5, double fac) {
-  long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n5) return;
-  y[i] = yold[i];
-  ac[i] = acold[i] * fac;
-}
+// ---------------- itrPredict / itrCorrect / itrUpdate / itrBC ----------------
+// One lane per node forms the node's new (y, ac), sets the Dirichlet values
+// on y (temperature, no-slip velocity, pressure; itrbc.f:60-139) and writes
+// them; a periodic master writes its slaves' too (itrbc.f:141-178: they copy
+// y and ac), so a slave's own lane writes nothing.
+struct StateArgs {
+  double* y;
+  double* ac;
+  const double* yold;
+  const double* acold;
+  const double* dy;
+  const uint8_t* bcm;
+  const double* BC;
+  const int2* info;
+  const int* fmaster;
+  const int* fptr;
+  const int* fslave;
+  long long n;
+  double f1, f2;
+};
 
-__global__ void k_correct(double* y, double* ac, const double* yold, const double* acold,
-                          const double* dy, long long n, double fct1, double fct2) {
-  long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+// kMode 0: itrPredict, same-velocity predictor (itrPC.f:67-73): y = yold,
+//          ac = acold f1
+//       1: itrCorrect (itrPC.f:128-148): y -= Dy, ac = acold f1 + (y - yold) f2
+//       2: itrUpdate (itrPC.f:204-207) of (y, ac) = the old state towards
+//          (yold, acold) = the new one: ac += (acold - ac) f1, y += (yold - y) f2
+template <int kMode>
+__global__ void k_state(StateArgs A) {
+  const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  const long long n = A.n;
   if (k >= n) return;
-  // y(:,1:3) -= Dy(:,2:4); y(:,4) -= Dy(:,1); y(:,5) -= Dy(:,5)
-  const int from[5] = {1, 2, 3, 0, 4};
+  const int fam = A.info[k].y;
+  if (fam >= 0 && A.fmaster[fam] != k) return;
+  double v[5], a[5];
+  const int from[5] = {1, 2, 3, 0, 4};  // Dy is in equation order
 #pragma unroll
   for (int f = 0; f < 5; ++f) {
-    const double v = y[k + f * n] - dy[k + from[f] * n];
-    y[k + f * n] = v;
-    ac[k + f * n] = acold[k + f * n] * fct1 + (v - yold[k + f * n]) * fct2;
-  }
-}
-
-// Dirichlet values on y (temperature, no-slip velocity, pressure)
-__global__ void k_bc_y(double* y, const uint8_t* bcm, const double* BC, long long n) {
-  long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const uint8_t m = bcm[k];
-  if (!m) return;
-  if (m & 16) y[k + 4 * n] = BC[k + n];
-  if (m & 2) {
-    y[k] = BC[k + 2 * n];
-    y[k + n] = BC[k + 3 * n];
-    y[k + 2 * n] = BC[k + 4 * n];
-  }
-  if (m & 1) y[k + 3 * n] = BC[k];
-}
-
-// periodic copy y(slave) = y(master), ac likewise
-__global__ void k_per_copy(double* y, double* ac, const int* master, const int* ptr,
-                           const int* slave, int nfold, long long n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nfold) return;
-  const long long m = master[i];
-  for (int k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const long long s = slave[k];
-#pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      y[s + f * n] = y[m + f * n];
-      ac[s + f * n] = ac[m + f * n];
+    const long long i = k + f * n;
+    if constexpr (kMode == 0) {
+      v[f] = A.yold[i];
+      a[f] = A.acold[i] * A.f1;
+    } else if constexpr (kMode == 1) {
+      v[f] = A.y[i] - A.dy[k + from[f] * n];
+      a[f] = A.acold[i] * A.f1 + (v[f] - A.yold[i]) * A.f2;
+    } else {
+      a[f] = A.ac[i] + (A.acold[i] - A.ac[i]) * A.f1;
+      v[f] = A.y[i] + (A.yold[i] - A.y[i]) * A.f2;
     }
   }
-}
-
-// itrUpdate (itrPC.f:204-207): acold += (ac-acold)/almi, yold += (y-yold)/alfi
-__global__ void k_update(double* yold, double* acold, const double* y, const double* ac,
-                         long long n5, double fct2, double fct3) {
-  long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n5) return;
-  acold[i] = acold[i] + (ac[i] - acold[i]) * fct2;
-  yold[i] = yold[i] + (y[i] - yold[i]) * fct3;
+  const uint8_t m = A.bcm[k];
+  if (m & 16) v[4] = A.BC[k + n];
+  if (m & 2) {
+    v[0] = A.BC[k + 2 * n];
+    v[1] = A.BC[k + 3 * n];
+    v[2] = A.BC[k + 4 * n];
+  }
+  if (m & 1) v[3] = A.BC[k];
+#pragma unroll
+  for (int f = 0; f < 5; ++f) {
+    A.y[k + f * n] = v[f];
+    A.ac[k + f * n] = a[f];
+  }
+  if (fam < 0) return;
+  for (int q = A.fptr[fam]; q < A.fptr[fam + 1]; ++q) {
+    const long long s = A.fslave[q];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) {
+      A.y[s + f * n] = v[f];
+      A.ac[s + f * n] = a[f];
+    }
+  }
 }
 
 inline int grid_for(long long n, int threads) {
@@ -1075,8 +1308,8 @@ int launch_ref_to_aos(phg_ctx* c, const double* ref) {
 
 int launch_bc3per(phg_ctx* c, double* v, int nq) {
   if (c->nfold <= 0) return 0;
-  k_fold_vec<<<(c->nfold + 255) / 256, 256, 0, c->stream>>>(v, c->fold_master, c->fold_ptr,
-                                                            c->fold_slave, c->nfold, c->nshg, nq);
+  k_fold_vec<<<dim3((c->nfold + 255) / 256, nq), 256, 0, c->stream>>>(
+      v, c->fold_master, c->fold_ptr, c->fold_slave, c->nfold, c->nshg);
   PHG_HIP(hipGetLastError());
   return 0;
 }
@@ -1111,7 +1344,7 @@ int launch_dot(phg_ctx* c, const double* a, const double* b, long long n, double
   return launch_finish(c, 0, np, np, 1, out);
 }
 
-int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm,
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm, double n0,
               unsigned seq) {
   if (iK < 1 || iK >= kGmMax) {
     phg_set_error("Gram-Schmidt: iteration %d outside 1..%d", iK, kGmMax - 1);
@@ -1128,6 +1361,7 @@ int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double eps
   A.unit = unit ? 1 : 0;
   A.unorm = unorm;
   A.epsnrm = epsnrm;
+  A.n0 = n0;
   A.part = c->red_part;
   A.chan = c->red_blocks;
   A.gm = c->gm;
@@ -1169,16 +1403,47 @@ int launch_combine(phg_ctx* c, double* dy, const double* zb, int nz, bool add) {
   return 0;
 }
 
-// out[0] = sum res^2, out[1] = bad entries of res, out[2] = bad entries of BDiag
-int launch_stats(phg_ctx* c, double* out) {
-  const long long n5 = 5 * c->nshg;
-  int np = 0;
-  PHG_TRY(launch_dot_part(c, c->res, c->res, n5, 0, &np));
-  PHG_TRY(launch_finish(c, 0, np, np, 1, out));
-  k_stat_bad<<<c->red_blocks, kRedThreads, 0, c->stream>>>(c->res, n5, red_chan(c, 1));
-  k_stat_bad<<<c->red_blocks, kRedThreads, 0, c->stream>>>(c->bdiag, 5 * n5, red_chan(c, 2));
+int launch_nodes(phg_ctx* c, bool prec, bool solve, double* raw, double* start) {
+  NodeArgs A{};
+  A.ares = c->acc_res;
+  A.abd = c->acc_bd;
+  A.wres = c->wres;
+  A.nspec = c->nspec;
+  A.sptr = c->sptr;
+  A.smem = c->smem;
+  A.wptr = c->wptr;
+  A.ssum = c->ssum;
+  A.info = c->ninfo;
+  A.bcm = c->bcm;
+  A.res = c->res;
+  A.rmes = c->rmes;
+  A.start = start;
+  A.bdiag = c->bdiag;
+  A.raw = raw;
+  A.n = c->nshg;
+  A.prec = prec ? 1 : 0;
+  A.part = c->red_part;
+  A.gm = c->gm;
+  A.host = c->h_sol;
+  if (c->nspec > 0) {
+    k_boundary_nodes<<<grid_for(32LL * c->nspec, 256), 256, 0, c->stream>>>(A);
+    PHG_HIP(hipGetLastError());
+  }
+  const int g = std::min(grid_for(c->nshg, kNodeThreads), kNodeBlocks);
+  if (solve) {
+    A.seq = ++c->sol_seq;
+    k_nodes<true><<<g, kNodeThreads, 0, c->stream>>>(A);
+  } else {
+    k_nodes<false><<<g, kNodeThreads, 0, c->stream>>>(A);
+  }
   PHG_HIP(hipGetLastError());
-  return launch_finish(c, 1, c->red_blocks, c->red_blocks, 2, out + 1);
+  return 0;
+}
+
+int launch_end_mark(phg_ctx* c) {
+  k_end_mark<<<1, 1, 0, c->stream>>>(c->h_sol, c->sol_seq);
+  PHG_HIP(hipGetLastError());
+  return 0;
 }
 
 int launch_csr_to_slots(phg_ctx* c, const double* ref, double* slots) {
@@ -1202,6 +1467,23 @@ int launch_slots_to_csr32(phg_ctx* c, const float* slots, double* ref) {
   return 0;
 }
 
+static StateArgs state_args(const phg_ctx* c, double* y, double* ac, const double* yold,
+                            const double* acold) {
+  StateArgs A{};
+  A.y = y;
+  A.ac = ac;
+  A.yold = yold;
+  A.acold = acold;
+  A.bcm = c->bcm;
+  A.BC = c->BCv;
+  A.info = c->ninfo;
+  A.fmaster = c->fold_master;
+  A.fptr = c->fold_ptr;
+  A.fslave = c->fold_slave;
+  A.n = c->nshg;
+  return A;
+}
+
 int launch_predict(phg_ctx* c) {
   // The reference's other predictors (ipred 2-4, itrPC.f:75-119) call
   // itrBC with iBC, BC, iper and ilwork undeclared in itrPredict, so they
@@ -1212,39 +1494,29 @@ int launch_predict(phg_ctx* c) {
                   "itrPC.f:67-73) has a defined result in the reference", c->prm.ipred);
     return PHG_EINVAL;
   }
-  const long long n5 = 5 * c->nshg;
-  const double fac = 1.0 - c->prm.almi / c->prm.gami;
-  k_predict<<<grid_for(n5, 256), 256, 0, c->stream>>>(c->yold, c->acold, c->y, c->ac, n5, fac);
+  StateArgs A = state_args(c, c->y, c->ac, c->yold, c->acold);
+  A.f1 = 1.0 - c->prm.almi / c->prm.gami;
+  k_state<0><<<grid_for(c->nshg, 256), 256, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
-  return launch_itrbc(c, c->y, c->ac);
+  return 0;
 }
 
 int launch_correct(phg_ctx* c) {
-  const double fct1 = 1.0 - c->prm.almi / c->prm.gami;
-  const double fct2 = c->prm.almi * c->prm.Dtgl / c->prm.gami / c->prm.alfi;
-  k_correct<<<grid_for(c->nshg, 256), 256, 0, c->stream>>>(c->y, c->ac, c->yold, c->acold, c->dy,
-                                                           c->nshg, fct1, fct2);
+  StateArgs A = state_args(c, c->y, c->ac, c->yold, c->acold);
+  A.dy = c->dy;
+  A.f1 = 1.0 - c->prm.almi / c->prm.gami;
+  A.f2 = c->prm.almi * c->prm.Dtgl / c->prm.gami / c->prm.alfi;
+  k_state<1><<<grid_for(c->nshg, 256), 256, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
-  return launch_itrbc(c, c->y, c->ac);
+  return 0;
 }
 
 int launch_update(phg_ctx* c) {
-  const long long n5 = 5 * c->nshg;
-  k_update<<<grid_for(n5, 256), 256, 0, c->stream>>>(c->yold, c->acold, c->y, c->ac, n5,
-                                                     1.0 / c->prm.almi, 1.0 / c->prm.alfi);
+  StateArgs A = state_args(c, c->yold, c->acold, c->y, c->ac);
+  A.f1 = 1.0 / c->prm.almi;
+  A.f2 = 1.0 / c->prm.alfi;
+  k_state<2><<<grid_for(c->nshg, 256), 256, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
-  return launch_itrbc(c, c->yold, c->acold);
-}
-
-int launch_itrbc(phg_ctx* c, double* y, double* ac) {
-  k_bc_y<<<grid_for(c->nshg, 256), 256, 0, c->stream>>>(y, c->bcm, c->BCv, c->nshg);
-  PHG_HIP(hipGetLastError());
-  if (c->nfold > 0) {
-    k_per_copy<<<(c->nfold + 255) / 256, 256, 0, c->stream>>>(y, ac, c->fold_master,
-                                                              c->fold_ptr, c->fold_slave, c->nfold,
-                                                              c->nshg);
-    PHG_HIP(hipGetLastError());
-  }
   return 0;
 }
 

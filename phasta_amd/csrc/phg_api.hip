@@ -483,6 +483,39 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   }
   c->nfold = (int)masters.size();
 
+  // ---- boundary groups (periodic families, then single wall nodes) and the
+  // members' wall contributions, in wall colour order ----
+  std::vector<int2> ninfo(nshg, make_int2(-1, -1));
+  std::vector<int> sptr(1, 0), smem;
+  for (size_t k = 0; k < masters.size(); ++k) {
+    ninfo[masters[k]] = make_int2((int)k, (int)k);
+    smem.push_back(masters[k]);
+    for (int q = fptr[k]; q < fptr[k + 1]; ++q) {
+      ninfo[fsl[q]] = make_int2((int)k, (int)k);
+      smem.push_back(fsl[q]);
+    }
+    sptr.push_back((int)smem.size());
+  }
+  for (long long p = 0; p < nelb; ++p)
+    for (int a = 0; a < 3; ++a) {
+      const int node = ienbc[a * nelb + p];
+      if (ninfo[node].x >= 0) continue;
+      ninfo[node].x = (int)sptr.size() - 1;
+      smem.push_back(node);
+      sptr.push_back((int)smem.size());
+    }
+  c->nspec = (int)sptr.size() - 1;
+  std::vector<int> wptr(smem.size() + 1, 0), wslot(3 * nelb), place(nshg, -1);
+  for (size_t q = 0; q < smem.size(); ++q) place[smem[q]] = (int)q;
+  for (long long p = 0; p < nelb; ++p)
+    for (int a = 0; a < 3; ++a) wptr[place[ienbc[a * nelb + p]] + 1]++;
+  for (size_t q = 0; q < smem.size(); ++q) wptr[q + 1] += wptr[q];
+  {
+    std::vector<int> next(wptr.begin(), wptr.end() - 1);
+    for (long long p = 0; p < nelb; ++p)
+      for (int a = 0; a < 3; ++a) wslot[3 * p + a] = next[place[ienbc[a * nelb + p]]]++;
+  }
+
   std::vector<uint8_t> bcm(nshg);
   std::vector<int> iper0(nshg);
   for (long long n = 0; n < nshg; ++n) {
@@ -519,6 +552,13 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_TRY(dev_alloc(c, &c->resid, (size_t)std::max<long long>(nel * 4, goff[ngq]) * 5));
   PHG_TRY(dev_alloc(c, &c->eslot, (size_t)nel * 4));
   PHG_TRY(dev_alloc(c, &c->ienbc, ienbc.size()));
+  PHG_TRY(dev_alloc(c, &c->wres, (size_t)nelb * 15));
+  PHG_TRY(dev_alloc(c, &c->wslot, wslot.size()));
+  PHG_TRY(dev_alloc(c, &c->sptr, sptr.size()));
+  PHG_TRY(dev_alloc(c, &c->smem, smem.size()));
+  PHG_TRY(dev_alloc(c, &c->wptr, wptr.size()));
+  PHG_TRY(dev_alloc(c, &c->ssum, (size_t)32 * c->nspec));
+  PHG_TRY(dev_alloc(c, &c->ninfo, nshg));
   PHG_TRY(dev_alloc(c, &c->bcm, nshg));
   PHG_TRY(dev_alloc(c, &c->iper, nshg));
   PHG_TRY(dev_alloc(c, &c->BCv, (size_t)nshg * m->ndofBC));
@@ -560,12 +600,15 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   c->kstr = (5 * nshg + 1) & ~1LL;
   PHG_TRY(dev_alloc(c, &c->krylov, (size_t)(std::max(K, 2) + 1) * c->kstr));
   c->red_blocks = 1024;
-  PHG_TRY(dev_alloc(c, &c->red_part, (size_t)(2 * (K + 2)) * c->red_blocks));
+  // Gram-Schmidt: 2 K channels; the nodal kernel: 3 of twice the length
+  PHG_TRY(dev_alloc(c, &c->red_part, (size_t)(2 * (K + 3)) * c->red_blocks));
   PHG_TRY(dev_alloc(c, &c->scal, 256));
   PHG_TRY(dev_alloc(c, &c->gm, 1));
   PHG_HIP(hipHostMalloc((void**)&c->h_scal, 256 * sizeof(double), hipHostMallocDefault));
   PHG_HIP(hipHostMalloc((void**)&c->h_gm, kGmMax * sizeof(GmHost), hipHostMallocCoherent));
   std::fill(c->h_gm, c->h_gm + kGmMax, GmHost{});
+  PHG_HIP(hipHostMalloc((void**)&c->h_sol, sizeof(SolveHost), hipHostMallocCoherent));
+  *c->h_sol = SolveHost{};
   {
     int dev = 0, khz = 0;
     PHG_HIP(hipGetDevice(&dev));
@@ -586,6 +629,11 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_TRY(upload(c, c->lanes_diag, lanes_diag.data(), lanes_diag.size()));
   PHG_TRY(upload(c, c->blocks, blk_lane.data(), blk_lane.size()));
   PHG_TRY(upload(c, c->ienbc, ienbc.data(), ienbc.size()));
+  PHG_TRY(upload(c, c->wslot, wslot.data(), wslot.size()));
+  PHG_TRY(upload(c, c->sptr, sptr.data(), sptr.size()));
+  PHG_TRY(upload(c, c->smem, smem.data(), smem.size()));
+  PHG_TRY(upload(c, c->wptr, wptr.data(), wptr.size()));
+  PHG_TRY(upload(c, c->ninfo, ninfo.data(), ninfo.size()));
   PHG_TRY(upload(c, c->bcm, bcm.data(), bcm.size()));
   PHG_TRY(upload(c, c->iper, iper0.data(), iper0.size()));
   PHG_TRY(upload(c, c->BCv, m->BC, (size_t)nshg * m->ndofBC));
@@ -676,14 +724,31 @@ int check_idiff(phg_ctx* c) {
   return 0;
 }
 
-int elm_core(phg_ctx* c) {
-  const long long n = c->nshg;
+// solve: with SolGMRs' nodal work (launch_nodes)
+int elm_core(phg_ctx* c, bool solve = false, double* raw = nullptr, double* start = nullptr) {
   const bool lhs = c->prm.lhs == 1, prec = c->prm.iprec != 0;
   PHG_TRY(check_idiff(c));
   // every node owns its diagonal block and every CSR entry has an owner, so
   // the assembly stores res, BDiag and lhsK completely: no clearing
   PHG_TRY(launch_assembly(c, lhs, prec));
-  PHG_TRY(launch_bc_res_bdiag(c, prec));
+  return launch_nodes(c, prec, solve, raw, start);
+}
+
+// Waits until the device has written the token seq to *at (pinned memory) and
+// with it the result beside it.  The stream is asked now and then, so that a
+// failed launch or a fault ends the wait.
+int wait_token(phg_ctx* c, const volatile unsigned* at, unsigned seq, const char* what) {
+  for (unsigned spin = 1; *at != seq; ++spin) {
+    if (spin % 4096) continue;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    PHG_HIP(e);
+    if (*at != seq) {
+      phg_set_error("the stream drained without the result of %s", what);
+      return PHG_EHIP;
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
   return 0;
 }
 
@@ -791,32 +856,13 @@ int elm_mfg(phg_ctx* c) {
   PHG_TRY(mfg_check(c));
   PHG_TRY(mfg_alloc(c));
   PHG_TRY(launch_assembly(c, false, prec));
-  PHG_TRY(launch_bc_res_bdiag(c, prec));
+  PHG_TRY(launch_nodes(c, prec, false, nullptr, nullptr));
   return launch_mres(c, nullptr, c->rmes, false, false);
 }
 
-// Waits until the device has written iteration iK's result (token seq) into
-// its slot.  The stream is asked now and then, so that a failed launch or a
-// fault ends the wait.
-int wait_iteration(phg_ctx* c, int iK, unsigned seq) {
-  const volatile unsigned* at = &c->h_gm[iK].seq;
-  for (unsigned spin = 1; *at != seq; ++spin) {
-    if (spin % 4096) continue;
-    const hipError_t e = hipStreamQuery(c->stream);
-    if (e == hipErrorNotReady) continue;
-    PHG_HIP(e);
-    if (*at != seq) {
-      phg_set_error("GMRES: the stream drained without the result of iteration %d", iK);
-      return PHG_EHIP;
-    }
-  }
-  std::atomic_thread_fence(std::memory_order_acquire);
-  return 0;
-}
-
 // One GMRES cycle on the scaled system (solgmr.f:522-692): kvec(0) holds the
-// normalised start vector, unorm its norm.  Leaves sum_k y_k u_k in c->dy, or
-// adds it there.
+// start vector, n0 its norm as stored, unorm the residual norm that it stands
+// for.  Leaves sum_k y_k u_k in c->dy, or adds it there.
 struct CycleOut {
   int iKs = 0;
   double echeck = 0.0;
@@ -830,7 +876,7 @@ struct CycleOut {
 // (launch_gs); the host stays one iteration ahead of the result it has seen,
 // so the device never waits for the host between iterations.  The iteration
 // enqueued after the last one finds GmDev::done set and returns.
-int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut* out,
+int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, double n0, phg_stats* st, CycleOut* out,
                 bool flexible, bool add) {
   const long long V = 5 * c->nshg;
   const int K = c->prm.Kspace;
@@ -873,8 +919,9 @@ int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut
         PHG_HIP(hipEventElapsedTime(&a1, c->kev[0], c->kev[1]));
         st->ms_spmv += 0.5 * a1;  // the second product is in the cycle's own clock
         st->n_spmv += 1;
-        const double r_net = d[1] > 0.0 ? 1.0 - d[0] * d[0] / d[1] : 1.0;
-        const double r_blk = d[3] > 0.0 ? 1.0 - d[2] * d[2] / d[3] : 1.0;
+        const double n2 = n0 * n0;  // u_1 = dir / n0
+        const double r_net = d[1] > 0.0 ? 1.0 - d[0] * d[0] / d[1] / n2 : 1.0;
+        const double r_blk = d[3] > 0.0 ? 1.0 - d[2] * d[2] / d[3] / n2 : 1.0;
         if (!(r_net <= r_blk)) {
           use_net = false;  // the plain direction's product is in w
           out->rejected = true;
@@ -890,16 +937,16 @@ int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut
     } else {
       PHG_TRY(launch_spmv(c, dir, w, true, iK > 1 ? &c->gm->done : nullptr, &c->gm->t0));
     }
-    PHG_TRY(launch_gs(c, w, iK, c->mfg.on, unorm, epsnrm, base + iK));
+    PHG_TRY(launch_gs(c, w, iK, c->mfg.on, unorm, epsnrm, n0, base + iK));
     if (iK > lag) {
       last = iK - lag;
-      PHG_TRY(wait_iteration(c, last, base + last));
+      PHG_TRY(wait_token(c, &c->h_gm[last].seq, base + last, "a Krylov iteration"));
       if (c->h_gm[last].done) break;
     }
   }
   if (last < K && !(last > 0 && c->h_gm[last].done)) {
     last = K;
-    PHG_TRY(wait_iteration(c, last, base + last));
+    PHG_TRY(wait_token(c, &c->h_gm[last].seq, base + last, "a Krylov iteration"));
   }
   const GmHost& end = c->h_gm[last];
   const int iKs = last;
@@ -914,11 +961,11 @@ int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, phg_stats* st, CycleOut
     double nrm[kGmMax];
     PHG_HIP(hipMemcpyAsync(nrm, c->gm->nrm, sizeof(nrm), hipMemcpyDeviceToHost, c->stream));
     PHG_TRY(sync(c));
-    for (int k = 1; k <= iKs; ++k) nrm[k] = nrm[k] * nrm[k];
+    for (int k = 0; k <= iKs; ++k) nrm[k] = nrm[k] * nrm[k];
     double* S = c->scal + 128;
     PHG_HIP(hipMemcpyAsync(S, nrm, sizeof(double) * (iKs + 1), hipMemcpyHostToDevice, c->stream));
     PHG_TRY(launch_combine(c, c->dy, c->mp.zbasis, use_net ? std::min(use_pc, iKs) : 0, add));
-    for (int k = 1; k <= iKs; ++k)
+    for (int k = 0; k <= iKs; ++k)
       PHG_TRY(launch_scale(c, kvec(c, k), kvec(c, k), V, S + k, nullptr));
     PHG_TRY(sync(c));
   } else {
@@ -997,7 +1044,7 @@ int mfg_core(phg_ctx* c, int fdi, phg_stats* st) {
         unorm = c->h_scal[6];
       }
       CycleOut co;
-      rc = gmres_cycle(c, unorm, epsnrm, st, &co, false, mG > 1);
+      rc = gmres_cycle(c, unorm, epsnrm, 1.0, st, &co, false, mG > 1);
       if (rc) break;
       iKs = co.iKs;
       echeck = co.echeck;
@@ -1025,11 +1072,11 @@ int mfg_core(phg_ctx* c, int fdi, phg_stats* st) {
   PHG_HIP(hipEventElapsedTime(&ms2, c->ev[1], c->ev[2]));
   st->ms_assembly = ms1;
   st->ms_solve = ms2;
-  float ma = 0, mb = 0;
-  PHG_HIP(hipEventElapsedTime(&ma, c->aev[0], c->aev[1]));
-  PHG_HIP(hipEventElapsedTime(&mb, c->aev[1], c->aev[2]));
-  st->ms_point = ma;
-  st->ms_blocks = mb;
+  long long ta[4];
+  PHG_HIP(hipMemcpyAsync(ta, c->gm->ta, sizeof(ta), hipMemcpyDeviceToHost, c->stream));
+  PHG_TRY(sync(c));
+  st->ms_point = c->clk_ms * (double)(ta[2] - ta[1]);
+  st->ms_blocks = c->clk_ms * (double)(ta[3] - ta[2]);
   st->ms_total = ms1 + ms2;
   return 0;
 }
@@ -1045,7 +1092,8 @@ constexpr int kMaxRefine = 4;
 // the FP64 tangent (launch_jv) and its norm is tested against the same
 // epsnrm as the FP64 path; cycles restart from that residual until it
 // passes (at most kMaxRefine cycles).
-int sol_core(phg_ctx* c, phg_stats* st) {
+// correct: itrCorrect + itrBC on the state afterwards.
+int sol_core(phg_ctx* c, phg_stats* st, bool correct = false) {
   const long long n = c->nshg, V = 5 * n;
   const int K = c->prm.Kspace;
   const bool mixed = c->precision == PHG_MIXED;
@@ -1057,40 +1105,31 @@ int sol_core(phg_ctx* c, phg_stats* st) {
     phg_set_error("nGMRES must be 1 (restart branch of solgmr.f:526 is inactive)");
     return PHG_EINVAL;
   }
-  PHG_HIP(hipEventRecord(c->ev[0], c->stream));
-  PHG_TRY(elm_core(c));
-  PHG_HIP(hipEventRecord(c->ev[1], c->stream));
-  PHG_HIP(hipMemcpyAsync(c->rmes, c->res, sizeof(double) * V, hipMemcpyDeviceToDevice, c->stream));
-  double* S = c->scal;  // [0] sum res^2 (after forward), [1],[2] bad counts, [3] unorm, [4] sum rmes^2
-  // tnanq on res and BDiag before factorisation (solgmr.f:459-460)
-  PHG_TRY(launch_stats(c, S));  // S[0] provisional, overwritten below
   const bool set_aside = c->mp.in_step && c->mp.step_off;
   const bool learned = c->mp.ready && c->mp.use_pc > 0 && !set_aside;
+  double* raw = nullptr;
   if ((learned || c->mp.keep_pair) && c->mp.ready) {
     // the network's BDiag input is the block diagonal before factorisation:
     // a call with iprec = 0 reuses the factored BDiag of an earlier call
     // (solgmr.f:471), so the raw copy of that call is kept
     if (c->prm.iprec != 0) {
-      PHG_HIP(hipMemcpyAsync(c->mp.bd_raw, c->bdiag, sizeof(double) * 25 * n,
-                             hipMemcpyDeviceToDevice, c->stream));
-      c->mp.bd_raw_ok = true;
+      raw = c->mp.bd_raw;
     } else if (!c->mp.bd_raw_ok) {
       phg_set_error("learned preconditioner with iprec = 0: no earlier call formed BDiag");
       return PHG_EINVAL;
     }
   }
-  if (c->prm.iprec != 0) PHG_TRY(launch_i3lu(c, c->bdiag, nullptr, 0));
-  PHG_TRY(launch_i3lu(c, c->bdiag, c->res, 1));
-  PHG_TRY(launch_dot(c, c->res, c->res, V, S));
-  PHG_TRY(launch_dot(c, c->rmes, c->rmes, V, S + 4));
-  PHG_TRY(launch_fill(c, c->dy, sizeof(double) * V));
+  // assembly; tnanq on res and BDiag, factorisation, forward reduction and the
+  // sums (solgmr.f:459-490) in the nodal kernel, the start vector in kvec(0)
+  PHG_TRY(elm_core(c, true, raw, kvec(c, 0)));
+  if (raw) c->mp.bd_raw_ok = true;
+  const unsigned seq = c->sol_seq;
   if (c->prm.lhs == 1) PHG_TRY(launch_spsi3pre(c));
-  PHG_TRY(launch_scale(c, kvec(c, 0), c->res, V, S, S + 3));
-  PHG_TRY(download(c, c->h_scal, S, 8));
-  PHG_TRY(sync(c));
-  const double sumsq = c->h_scal[0];
+  double* S = c->scal;
+  PHG_TRY(wait_token(c, &c->h_sol->seq, seq, "the assembly"));
+  const double sumsq = c->h_sol->sumsq, sumsq_m = c->h_sol->sumsq_m;
   st->nnan = 0;
-  st->nlarge = (long long)(c->h_scal[1] + c->h_scal[2]);
+  st->nlarge = (long long)c->h_sol->bad;
   if (st->nlarge > 0) {
     phg_set_error("tnanq: %lld NaN/large entries in res/BDiag", st->nlarge);
     return PHG_ENAN;
@@ -1102,7 +1141,7 @@ int sol_core(phg_ctx* c, phg_stats* st) {
     return PHG_EDIVERGE;
   }
   c->reslast = totres_chk;
-  const double unorm = c->h_scal[3];
+  const double unorm = std::sqrt(sumsq);
   st->unorm0 = unorm;
   const double epsnrm = c->prm.etol * unorm;
   st->epsnrm = epsnrm;
@@ -1114,7 +1153,7 @@ int sol_core(phg_ctx* c, phg_stats* st) {
   double echeck = 0.0;
   st->pc_fallback = set_aside && c->mp.ready && c->mp.use_pc > 0 ? 4 : 0;
   if (!(unorm < 100. * c->prm.epsM * c->prm.epsM)) {
-    double rnorm = unorm;
+    double rnorm = unorm, n0 = unorm;  // residual norm, kvec(0)'s norm as stored
     // true residual of the scaled system, r = b - K dy, normalised into
     // kvec(0); returns its norm.  FP64 path: the stored (FP64) matrix.
     // Mixed path: the FP64 tangent without the stored float matrix,
@@ -1137,13 +1176,14 @@ int sol_core(phg_ctx* c, phg_stats* st) {
       PHG_TRY(download(c, c->h_scal + 5, S + 5, 2));
       PHG_TRY(sync(c));
       *norm = c->h_scal[6];
+      n0 = 1.0;
       return 0;
     };
     bool plain_from_start = !learned;
     if (learned) {
       // FGMRES cycle with the network; block-diagonal GMRES is its fallback and yardstick
       CycleOut co;
-      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co, true, false));
+      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, n0, st, &co, true, false));
       iKs += co.iKs;
       st->refine_cycles = 1;
       PHG_TRY(true_residual(&rnorm));
@@ -1154,9 +1194,9 @@ int sol_core(phg_ctx* c, phg_stats* st) {
       } else if (!(rnorm < unorm)) {
         // no reduction: discard and solve with block-diagonal GMRES
         st->pc_fallback = 1;
-        PHG_TRY(launch_fill(c, c->dy, sizeof(double) * V));
-        PHG_TRY(launch_scale(c, kvec(c, 0), c->res, V, S, S + 3));
-        rnorm = unorm;
+        PHG_HIP(hipMemcpyAsync(kvec(c, 0), c->res, sizeof(double) * V, hipMemcpyDeviceToDevice,
+                               c->stream));
+        rnorm = n0 = unorm;
         plain_from_start = true;
       } else if (rnorm > epsnrm) {
         st->pc_fallback = 2;  // reduced, finished by block-diagonal cycles
@@ -1166,7 +1206,7 @@ int sol_core(phg_ctx* c, phg_stats* st) {
     bool add = !plain_from_start;  // onto the learned cycle's update
     for (int cyc = 0; need_plain; ++cyc) {
       CycleOut co;
-      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, st, &co, false, add));
+      PHG_TRY(gmres_cycle(c, rnorm, epsnrm, n0, st, &co, false, add));
       add = true;
       iKs += co.iKs;
       echeck = co.echeck;
@@ -1176,34 +1216,31 @@ int sol_core(phg_ctx* c, phg_stats* st) {
       echeck = rnorm;
       if (rnorm <= epsnrm || cyc + 1 >= kMaxRefine) break;
     }
+  } else {
+    PHG_TRY(launch_fill(c, c->dy, sizeof(double) * V));  // no cycle ran
   }
   if (c->mp.ready && c->mp.keep_pair)
     PHG_HIP(hipMemcpyAsync(c->mp.zhat, c->dy, sizeof(double) * V, hipMemcpyDeviceToDevice,
                            c->stream));
   PHG_TRY(launch_i3lu(c, c->bdiag, c->dy, 2));
-  PHG_HIP(hipEventRecord(c->ev[2], c->stream));
-  PHG_TRY(download(c, c->h_scal + 4, S + 4, 1));
-  PHG_TRY(sync(c));
+  if (correct) PHG_TRY(launch_correct(c));
+  PHG_TRY(launch_end_mark(c));
+  PHG_TRY(wait_token(c, &c->h_sol->end_seq, seq, "the solve"));
   // rstat.f:95-116
   st->totres[0] = std::sqrt(sumsq) / (double)(float)n;
-  st->totres[1] = std::sqrt(c->h_scal[4]) / (double)(float)n;
+  st->totres[1] = std::sqrt(sumsq_m) / (double)(float)n;
   st->iKs = iKs;
   st->lGMRES = 0;
   st->ntotGM = c->ntotGM;
   st->echeck = echeck;
   st->converged = echeck <= epsnrm;
   st->reslast = c->reslast;
-  float ms1 = 0, ms2 = 0;
-  PHG_HIP(hipEventElapsedTime(&ms1, c->ev[0], c->ev[1]));
-  PHG_HIP(hipEventElapsedTime(&ms2, c->ev[1], c->ev[2]));
-  st->ms_assembly = ms1;
-  st->ms_solve = ms2;
-  float ma = 0, mb = 0;
-  PHG_HIP(hipEventElapsedTime(&ma, c->aev[0], c->aev[1]));
-  PHG_HIP(hipEventElapsedTime(&mb, c->aev[1], c->aev[2]));
-  st->ms_point = ma;
-  st->ms_blocks = mb;
-  st->ms_total = ms1 + ms2;
+  const SolveHost& h = *c->h_sol;
+  st->ms_assembly = c->clk_ms * (double)(h.ta[4] - h.ta[0]);
+  st->ms_point = c->clk_ms * (double)(h.ta[2] - h.ta[1]);
+  st->ms_blocks = c->clk_ms * (double)(h.ta[3] - h.ta[2]);
+  st->ms_solve = c->clk_ms * (double)(h.end - h.ta[4]);
+  st->ms_total = st->ms_assembly + st->ms_solve;
   return 0;
 }
 
@@ -1281,17 +1318,12 @@ extern "C" int phg_init(const phg_mesh* mesh, const phg_params* prm, int precisi
   for (auto& ev : c->kev) {
     if (hipEventCreate(&ev) != hipSuccess) ev = nullptr;
   }
-  for (auto& ev : c->aev) {
-    if (hipEventCreate(&ev) != hipSuccess) ev = nullptr;
-  }
   int rc = setup(c, mesh);
   if (rc == 0) rc = scratch_address(&c->scratch);
   if (rc == 0) {
     for (auto ev : c->ev)
       if (!ev) rc = PHG_EHIP;
     for (auto ev : c->kev)
-      if (!ev) rc = PHG_EHIP;
-    for (auto ev : c->aev)
       if (!ev) rc = PHG_EHIP;
     if (rc) phg_set_error("hipEventCreate failed");
   }
@@ -1318,16 +1350,16 @@ extern "C" int phg_finalize(phg_ctx* c) {
                   c->acold,    c->dy,       c->krylov, c->red_part, c->scal,
                   c->tmp,      c->slot2csr, c->lhs_aos, c->lhs_aos32, c->acc_res, c->acc_bd,
                   c->nodepack, c->inc_goff, c->inc,   c->eslot,   c->qrec,    c->qnode,
-                  c->dcw,      c->mtau,     c->gm,      c->rowmap,  c->fam,     c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
+                  c->dcw,      c->mtau,     c->gm,      c->rowmap,  c->fam,     c->wres,
+                  c->wptr,     c->wslot,    c->sptr,    c->smem,    c->ssum,    c->ninfo,   c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_scal) (void)hipHostFree(c->h_scal);
   if (c->h_gm) (void)hipHostFree(c->h_gm);
+  if (c->h_sol) (void)hipHostFree(c->h_sol);
   for (auto ev : c->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto ev : c->kev)
-    if (ev) (void)hipEventDestroy(ev);
-  for (auto ev : c->aev)
     if (ev) (void)hipEventDestroy(ev);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1460,9 +1492,7 @@ extern "C" int phg_newton_iteration(phg_ctx* c, phg_stats* st) {
   phg_stats local{};
   if (!st) st = &local;
   c->prm.iter += 1;  // itrdrv.f:434
-  PHG_TRY(sol_core(c, st));
-  PHG_TRY(launch_correct(c));
-  return 0;
+  return sol_core(c, st, true);
 }
 
 extern "C" int phg_update(phg_ctx* c) {

@@ -136,6 +136,8 @@ constexpr int kGmMax = 64;
 struct GmDev {
   unsigned cnt;                     // arrivals of the running reduction
   int done, iKs;                    // the cycle has ended; iterations so far
+  long long ta[4];                  // device clock: nodes packed, point pass, block
+                                    // pass, nodal kernel begun
   long long t0, t1;                 // device clock: product begun, dots begun
   long long acc_spmv, acc_gs;       // clock ticks of the cycle's products and
                                     // Gram-Schmidt steps
@@ -154,6 +156,15 @@ struct GmHost {
   double echeck;
   long long acc_spmv, acc_gs;
   unsigned seq;
+};
+
+// What the nodal kernel and the end of a solve report, likewise.
+struct SolveHost {
+  double sumsq, sumsq_m;            // sum (L^-1 res)^2, sum res^2
+  double bad;                       // NaN / large entries of res and BDiag
+  long long ta[5];                  // GmDev::ta and the nodal kernel's end
+  long long end;                    // the solve's end
+  unsigned seq, end_seq;
 };
 
 // Learned preconditioner state (k_mpnn.hip); allocated by phg_mpnn_init.
@@ -251,6 +262,18 @@ struct phg_ctx {
   size_t dcw_len = 0;           // doubles allocated in dcw
   void* mtau = nullptr;         // nel*4 W PTau per point (itau = 10), the tangent's type
   int* ienbc = nullptr;         // 4 planes of nelb, colour order, 0-based
+  double* wres = nullptr;       // 5 per (wall element, face node), the face nodes'
+                                // contributions together in wall-colour order
+  int* wslot = nullptr;         // place of (wall element, face node) in wres
+  // boundary groups: a periodic family (master first, slaves ascending) or a
+  // single node with wall faces; their sums after the assembly
+  int nspec = 0;
+  int* sptr = nullptr;          // members of group g: smem[sptr[g] .. sptr[g+1])
+  int* smem = nullptr;
+  int* wptr = nullptr;          // contributions of member q: wres[wptr[q] .. wptr[q+1])
+  double* ssum = nullptr;       // 32 per group: res (5) at 25, BDiag (25)
+  int2* ninfo = nullptr;        // per node: boundary group, periodic family (in
+                                // fold_ptr); -1 without
   uint8_t* bcm = nullptr;       // constraint mask per node
   int* iper = nullptr;          // 0-based master
   double* BCv = nullptr;        // (nshg, ndofBC)
@@ -315,6 +338,8 @@ struct phg_ctx {
   GmDev* gm = nullptr;             // the running GMRES cycle
   GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
   unsigned gm_seq = 0;             // token of the last iteration enqueued
+  SolveHost* h_sol = nullptr;      // pinned
+  unsigned sol_seq = 0;            // token of the last solve enqueued
   double clk_ms = 0.0;             // ms per tick of the device clock
   double* scal = nullptr;          // device scalars (H column etc.)
   double* h_scal = nullptr;        // pinned mirror
@@ -341,14 +366,12 @@ struct phg_ctx {
   // timing events on the library stream, created once
   hipEvent_t ev[3] = {};
   hipEvent_t kev[4] = {};
-  hipEvent_t aev[3] = {};  // assembly: before pass 1, after pass 1, after pass 2
 };
 
 // ---- launchers (k_assembly.hip) ----
 int launch_fill(phg_ctx* c, void* p, size_t bytes);
 int launch_assembly(phg_ctx* c, bool lhs, bool prec);
 int launch_diffusive_flux(phg_ctx* c);
-int launch_bc_res_bdiag(phg_ctx* c, bool prec);
 // w = A v with A the FP64 assembled tangent (after bc3LHS) of the state of
 // the last assembly, v read at the periodic masters and w folded (bc3per):
 // the operator of SparseAp + bc3per before the two-sided scaling.  Uses
@@ -421,14 +444,19 @@ int launch_finish(phg_ctx* c, int chan0, int np0, int np, int nsums, double* out
 // vectors, the Hessenberg column, its rotations and the convergence test; the
 // result goes to h_gm with the token seq.  Skipped on the device when an
 // earlier iteration ended the cycle.
-int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm,
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm, double n0,
               unsigned seq);
 int launch_scale(phg_ctx* c, double* u, const double* src, long long n,
                  const double* sq_ptr, double* norm_out);
 // dy (+)= the cycle's combination: its first nz directions from zb (stride
 // 5*nshg), the others from the basis
 int launch_combine(phg_ctx* c, double* dy, const double* zb, int nz, bool add);
-int launch_stats(phg_ctx* c, double* out);
+// After the assembly: res and BDiag (prec) after bc3Res / bc3BDg.  solve: also
+// rmes, BDiag factored (its values before into raw, nullable), res forward
+// reduced and copied to start, the sums and counts to h_sol with sol_seq.
+int launch_nodes(phg_ctx* c, bool prec, bool solve, double* raw, double* start);
+// the device clock into h_sol->end, with sol_seq
+int launch_end_mark(phg_ctx* c);
 int launch_csr_to_slots(phg_ctx* c, const double* ref, double* slots);
 int launch_pack_nodes(phg_ctx* c);
 int launch_slots_to_csr(phg_ctx* c, const double* slots, double* ref);
@@ -436,6 +464,5 @@ int launch_slots_to_csr32(phg_ctx* c, const float* slots, double* ref);
 int launch_predict(phg_ctx* c);
 int launch_correct(phg_ctx* c);
 int launch_update(phg_ctx* c);
-int launch_itrbc(phg_ctx* c, double* y, double* ac);
 // yshuffle of 5-plane vectors (src and dst may be the same)
 int launch_yshuffle(phg_ctx* c, const double* src, double* dst, bool new2old);

@@ -7,7 +7,7 @@
 //
 //  k_asm_qp      four lanes per element, lane q = quadrature point q: the
 //                element metrics, the interpolated state, thermodynamics and
-//                tau at q (12 values, kept for the tangent pass) and q's
+//                tau at q (kept for the tangent pass) and q's
 //                residual contribution to the element's four nodes, summed
 //                over q across the four lanes and written per (element,
 //                node).
@@ -54,27 +54,40 @@ struct Quad {
 
 __constant__ Quad cQ;
 
-// Geometry records of 13 values (shape gradients (4 x 3) and WdetJ), padded
-// so that a record is read with 16-byte loads: 14 doubles or 16 floats.
+// What the tangent pass reads of an element: per node a row (shape gradient,
+// WdetJ), per point a record.
+// Double: the rows in geo (16 values), the records of 8 values in qps:
+//   0..2 u, 3 rho, 4 drdp, 5 e3p (Franca's tau: WdetJ tau_2), 6, 7 WdetJ tau_0, 1
+// (the tangent pass builds P scaled by WdetJ); with k the kinetic energy, drdT =
+// -R rho drdp, e1p = (cp/R - 1) + drdp k, e4p = drdT k (ideal gas, e3mtrx.f),
+// tau_2 is a constant times tau_1 (Shakib) or stored, e3p then from rho h =
+// (cp/R) rho / drdp.
+// Float: 64 values per element in qps, the four rows and then 12 values per
+// point, each rounded once from double (formed from 8 floats they would carry two
+// to four roundings):
+//   0..2 u, 3 rho, 4 drdp, 5 drdT, 6 e1p, 7 e3p, 8 e4p, 9..11 WdetJ tau
+// So an element's points are 256 bytes, two cache lines, in either type.
 template <typename S>
-constexpr int rec_stride() { return sizeof(S) == 8 ? 14 : 16; }
+constexpr int pt_vals() { return sizeof(S) == 8 ? 8 : 12; }
 
-// Point records of 12 values, what the tangent pass needs at a point:
-//   0..2 u, 3 rho, 4 drdp, 5 drdT, 6 e1p, 7 e3p, 8 e4p (e2p = e1p + 1),
-//   9..11 WdetJ tau (the tangent pass builds P scaled by WdetJ)
-// read with three 16-byte loads in float (six in double).  The pass is
-// bound by the vector-memory address path (one tag lookup per lane and
-// load instruction), so the record is kept to the values it needs.
-template <typename S>
-constexpr int pt_stride() { return 12; }
-enum PtField { kPtRho = 3, kPtDrdp, kPtDrdT, kPtE1p, kPtE3p, kPtE4p, kPtT0, kPtT1, kPtT2 };
+// Constants of a point record's decoding
+template <typename R>
+struct PtConst {
+  R Rg, e1c, cpR, kt2;
+  bool franca;
+};
+
+template <typename R>
+struct Pt {
+  R u[3], rho, drdp, drdT, e1p, e3p, e4p, t0, t1, t2;
+};
 
 template <typename S>
-__device__ inline void load_pt(const S* p, S v[12]) {
+__device__ inline void load_vals(const S* p, S* v, int count) {
   if constexpr (sizeof(S) == 8) {
     const double2* q = reinterpret_cast<const double2*>(p);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < count / 2; ++i) {
       const double2 t = q[i];
       v[2 * i] = t.x;
       v[2 * i + 1] = t.y;
@@ -82,7 +95,7 @@ __device__ inline void load_pt(const S* p, S v[12]) {
   } else {
     const float4* q = reinterpret_cast<const float4*>(p);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < count / 4; ++i) {
       const float4 t = q[i];
       v[4 * i] = t.x;
       v[4 * i + 1] = t.y;
@@ -92,35 +105,339 @@ __device__ inline void load_pt(const S* p, S v[12]) {
   }
 }
 
-template <typename S>
-__device__ inline void load_rec(const S* p, S v[16]) {
-  if constexpr (sizeof(S) == 8) {
-    const double2* q = reinterpret_cast<const double2*>(p);
-#pragma unroll
-    for (int i = 0; i < 7; ++i) {
-      const double2 t = q[i];
-      v[2 * i] = t.x;
-      v[2 * i + 1] = t.y;
-    }
+template <typename R, typename S>
+__device__ __forceinline__ Pt<R> decode_pt(const S v[pt_vals<S>()], const PtConst<R>& C) {
+  Pt<R> t;
+  t.u[0] = (R)v[0];
+  t.u[1] = (R)v[1];
+  t.u[2] = (R)v[2];
+  t.rho = (R)v[3];
+  t.drdp = (R)v[4];
+  if constexpr (sizeof(S) == 4) {
+    t.drdT = (R)v[5];
+    t.e1p = (R)v[6];
+    t.e3p = (R)v[7];
+    t.e4p = (R)v[8];
+    t.t0 = (R)v[9];
+    t.t1 = (R)v[10];
+    t.t2 = (R)v[11];
   } else {
-    const float4* q = reinterpret_cast<const float4*>(p);
+    const R k = (R)0.5 * (t.u[0] * t.u[0] + t.u[1] * t.u[1] + t.u[2] * t.u[2]);
+    t.drdT = -(C.Rg * t.drdp) * t.rho;
+    t.e1p = C.e1c + t.drdp * k;
+    t.e4p = t.drdT * k;
+    t.t0 = (R)v[6];
+    t.t1 = (R)v[7];
+    if (C.franca) {
+      t.t2 = (R)v[5];
+      t.e3p = C.cpR * t.rho / t.drdp + t.rho * k;
+    } else {
+      t.t2 = C.kt2 * t.t1;
+      t.e3p = (R)v[5];
+    }
+  }
+  return t;
+}
+
+template <typename S>
+__device__ inline void store_vals(S* p, const S* v, int count) {
+  if constexpr (sizeof(S) == 8) {
+    double2* q = reinterpret_cast<double2*>(p);
+#pragma unroll
+    for (int i = 0; i < count / 2; ++i) q[i] = make_double2(v[2 * i], v[2 * i + 1]);
+  } else {
+    float4* q = reinterpret_cast<float4*>(p);
+#pragma unroll
+    for (int i = 0; i < count / 4; ++i)
+      q[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+  }
+}
+
+// where element e's row a and point record q are
+template <typename S>
+__device__ __forceinline__ S* row_at(S* qps, S* geo, long long e, int a) {
+  if constexpr (sizeof(S) == 8)
+    return geo + 16 * e + 4 * a;
+  else
+    return qps + 64 * e + 4 * a;
+}
+template <typename S>
+__device__ __forceinline__ S* pt_at(S* qps, long long e, int q) {
+  if constexpr (sizeof(S) == 8)
+    return qps + 32 * e + 8 * q;
+  else
+    return qps + 64 * e + 16 + 12 * q;
+}
+
+// ---- element records through LDS ----
+// Loads whose 64 lanes go to 64 different records bounded the block pass: the
+// texture addresser takes such an instruction a lane per cycle, and every
+// 16-byte piece looks its cache line up again (addresser busy 83 % of the
+// cycles in float, vector ALU 51 %).  So the eight lanes of an octet load their
+// eight records together, straight into LDS: load i takes a line of 128 bytes
+// of the octet's lane i, a piece of 16 bytes per lane, and each lane then reads
+// its own pieces.  A cache line is asked for once, and no register holds a
+// record in flight, so lines are asked for two to three points ahead.  At 128^3
+// hexes of six tets (2.1 M nodes, 12.6 M elements), the whole pass: 7.79 -> 5.79
+// ms in float, 12.5 -> 8.36 ms in double; vector ALU 70 % busy in float, the
+// addresser 68 %, a third of it the blocks' stores.  Of that 7.7 and 10.2 ms came
+// with the shorter records and DiagPt's algebra, loaded lane by lane; quads of
+// lanes and 64-byte pieces in the same scheme gave 7.6 and 9.2 ms (each cache
+// line asked for twice, the second time while it was on its way).
+//
+// An element is in float two lines (four rows, point 0 and the first piece of
+// point 1; the rest), in double two lines of two points each and a line of rows,
+// of which the two that the block needs are loaded by a quad of lanes.  LDS per
+// wavefront: 16.7 KB in float (two lines per lane), 12.9 KB in double (one line,
+// points 0 and 1 and then points 2 and 3, and the two rows).
+//
+// Load i of the octet puts piece p of its lane i at 16-byte place 64 i + 8
+// octet + (p ^ i), a quad's load i at 64 i + 4 quad + (p ^ i): the sixteen lanes
+// that one LDS cycle serves read sixteen different places modulo 256 bytes.
+//
+// Every lane of the wavefront takes part, with an element that may be read; one
+// wavefront per workgroup, so a wait of its own is the only synchronisation.
+typedef int phg_i4 __attribute__((ext_vector_type(4)));
+// two doubles at an 8-byte boundary
+typedef double phg_d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// the next lane's value (zero in lane 63)
+template <typename T>
+__device__ __forceinline__ T next_lane(T v) {
+  if constexpr (sizeof(T) == 8) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, ((long long)hi << 32) | (unsigned)lo);
+  } else {
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
+  }
+}
+
+template <typename S>
+__device__ __forceinline__ S piece(const phg_i4 A[4], int k) {
+  if constexpr (sizeof(S) == 8) {
+    const unsigned lo = (unsigned)A[k / 2][2 * (k & 1)];
+    const long long v = ((long long)A[k / 2][2 * (k & 1) + 1] << 32) | lo;
+    return __builtin_bit_cast(double, v);
+  } else {
+    const int w = A[k / 4][k & 3];
+    return __builtin_bit_cast(float, w);
+  }
+}
+
+// one read of LDS that direct loads have written, complete when it returns
+__device__ __forceinline__ phg_i4 lds_i4(unsigned at) {
+  phg_i4 v;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");
+  return v;
+}
+__device__ __forceinline__ int lds_int(unsigned at) {
+  int v;
+  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");
+  return v;
+}
+template <int kLater>
+__device__ __forceinline__ void loads_but() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLater) : "memory");
+}
+
+template <typename R, typename S>
+struct Pipe {
+  static constexpr bool kDbl = sizeof(S) == 8;
+  static constexpr int kLine = 512;                            // pieces: 128 bytes per lane
+  static constexpr int kRows = kDbl ? kLine : 0;               // slots: double's two rows,
+  static constexpr int kCode = kDbl ? kLine + 256 : 2 * kLine;  // block codes (double: two slots),
+  static constexpr int kN = kCode + (kDbl ? 32 : 16);          // N(node, point)
+  static constexpr int kPieces = kN + 8;
+
+  typedef __attribute__((address_space(3))) phg_i4* lp;
+  typedef const __attribute__((address_space(1))) void* gp;
+  const S* qps;
+  const S* geo;
+  const int* blk;   // the block codes (e * 16 + a * 4 + b); the lane's are
+  int first, last;  // blk[first .. last], none if last < first
+  lp lds;
+  unsigned at;      // LDS address of piece 0 of this lane's line
+
+  __device__ __forceinline__ Pipe(const S* q, const S* g, const int* b, int f, int cnt,
+                                  phg_i4* l)
+      : qps(q), geo(g), blk(b), first(f), last(f + cnt - 1), lds((lp)l) {
+    const int i = threadIdx.x & 7;
+    at = addr(0) + 16 * (64 * i + (threadIdx.x & 56) + i);
+    if (threadIdx.x < 16)
+      reinterpret_cast<__attribute__((address_space(3))) R*>(lds + kN)[threadIdx.x] =
+          (R)cQ.N[threadIdx.x & 3][threadIdx.x >> 2];
+  }
+  __device__ __forceinline__ unsigned addr(int piece) const {
+    return (unsigned)(size_t)(lds + piece);
+  }
+  __device__ __forceinline__ static int codes(int k) { return kDbl ? kCode + 16 * (k & 1) : kCode; }
+  __device__ __forceinline__ int code_at(int k) const {
+    return first <= last ? blk[min(first + k, last)] : 0;
+  }
+  // starts the load of block k's code
+  __device__ __forceinline__ void start_code(int k) const {
+    __builtin_amdgcn_global_load_lds((gp)(blk + max(min(first + k, last), 0)), lds + codes(k), 4,
+                                     0, 0);
+  }
+  // starts the loads of 128-byte line `line` of the octet's elements of block k
+  // (from qps, 256 bytes per element) into the line slot at `slot`
+  __device__ __forceinline__ void start_line(int k, int line, int slot) const {
+    const unsigned c = addr(codes(k)) + 4 * (threadIdx.x & 56);
+    const phg_i4 lo = lds_i4(c), hi = lds_i4(c + 16);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int code = i < 4 ? lo[i & 3] : hi[i & 3];
+      const unsigned p = (unsigned)(code & ~15) + 8 * line + ((threadIdx.x & 7) ^ i);
+      __builtin_amdgcn_global_load_lds((gp)(reinterpret_cast<const phg_i4*>(qps) + p),
+                                       lds + slot + 64 * i, 16, 0, 0);
+    }
+  }
+  // double: starts the loads of the rows of nodes a and b of block k
+  __device__ __forceinline__ void start_rows(int k) const {
+    const phg_i4 c = lds_i4(addr(codes(k)) + 4 * (threadIdx.x & 60));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float4 t = q[i];
-      v[4 * i] = t.x;
-      v[4 * i + 1] = t.y;
-      v[4 * i + 2] = t.z;
-      v[4 * i + 3] = t.w;
+      const int p = (threadIdx.x & 3) ^ i;
+      const unsigned nd = p & 2 ? c[i] & 3 : (c[i] >> 2) & 3;
+      const unsigned at = (unsigned)(c[i] >> 4) * 8 + 2 * nd + (p & 1);
+      __builtin_amdgcn_global_load_lds((gp)(reinterpret_cast<const phg_i4*>(geo) + at),
+                                       lds + kRows + 64 * i, 16, 0, 0);
     }
   }
-}
+  // the loads of the first block (code: the lane's)
+  __device__ __forceinline__ void start(int code) const {
+    reinterpret_cast<__attribute__((address_space(3))) int*>(lds + codes(0))[threadIdx.x] = code;
+    if constexpr (kDbl) {
+      start_rows(0);
+      start_line(0, 0, 0);
+    } else {
+      start_line(0, 0, 0);
+      start_line(0, 1, kLine);
+    }
+    start_code(1);
+  }
+  // Vector memory loads end in order, so a slot is full once no more loads are
+  // outstanding than were started after its own.  The order for a block, without
+  // the starts in brackets for the wavefront's last:
+  //   float:  rows and point 0 read (line 0: 9 later loads, line 1 and a code) |
+  //     point 1 read (line 1 and the code: none later) [line 0 of the next] |
+  //     point 2 | point 3 read [line 1 of the next, the code after it]
+  //   double: rows read (9 later: points 0, 1 and a code) | point 0 read (none
+  //     later) | point 1 read, points 2 and 3 started [rows of the next] |
+  //     point 2 read (4 later, or none) | point 3 read [points 0 and 1 of the
+  //     next, the code after it]
+  //
+  // the shape gradients of nodes a and b; returns WdetJ
+  __device__ __forceinline__ R rows(int code, R sa[3], R sb[3]) const {
+    loads_but<9>();
+    if constexpr (kDbl) {
+      const int i = threadIdx.x & 3;
+      const unsigned r = addr(kRows) + 16 * ((64 * i + (threadIdx.x & 60)) | i);
+      phg_i4 A[4];
+      asm volatile(
+          "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+          "ds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(A[0]), "=&v"(A[1]), "=&v"(A[2]), "=&v"(A[3])
+          : "v"(r), "v"(r ^ 16), "v"(r ^ 32), "v"(r ^ 48)
+          : "memory");
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        sa[c] = (R)piece<S>(A, c);
+        sb[c] = (R)piece<S>(A, 4 + c);
+      }
+      return (R)piece<S>(A, 3);
+    } else {
+      phg_i4 A[4];
+      asm volatile(
+          "ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(A[0]), "=&v"(A[1])
+          : "v"(at ^ ((code & 12) << 2)), "v"(at ^ ((code & 3) << 4))
+          : "memory");
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        sa[c] = (R)piece<S>(A, c);
+        sb[c] = (R)piece<S>(A, 4 + c);
+      }
+      return (R)piece<S>(A, 3);
+    }
+  }
+  // point q's record of block k and the shape functions of nodes a and b there;
+  // more: some lane of the wavefront has a block k + 1.  next: its code, from
+  // point 1 on
+  __device__ __forceinline__ void point(int q, int k, bool more, int code, int& next,
+                                        S v[pt_vals<S>()], R& Na, R& Nb) const {
+    if constexpr (kDbl) {
+      if (q == 0 || (q == 2 && !more)) loads_but<0>();
+      if (q == 2) loads_but<4>();
+    } else {
+      if (q == 1) loads_but<0>();
+    }
+    const unsigned n = addr(kN) + (int)sizeof(R) * q;
+    const unsigned na = n + (int)sizeof(R) * (code & 12);
+    const unsigned nb = n + (int)sizeof(R) * ((code << 2) & 12);
+    phg_i4 A[4];
+    if constexpr (sizeof(R) == 8)
+      asm volatile(
+          "ds_read_b64 %0, %2\n\tds_read_b64 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(Na), "=&v"(Nb)
+          : "v"(na), "v"(nb)
+          : "memory");
+    else
+      asm volatile(
+          "ds_read_b32 %0, %2\n\tds_read_b32 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(Na), "=&v"(Nb)
+          : "v"(na), "v"(nb)
+          : "memory");
+    if constexpr (kDbl) {
+      const unsigned s = at ^ ((q & 1) << 6);
+      asm volatile(
+          "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+          "ds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(A[0]), "=&v"(A[1]), "=&v"(A[2]), "=&v"(A[3])
+          : "v"(s), "v"(s ^ 16), "v"(s ^ 32), "v"(s ^ 48)
+          : "memory");
+    } else {
+      const int p = 4 + 3 * q;  // the record's first piece of the element's 16
+      asm volatile(
+          "ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\tds_read_b128 %2, %5\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(A[0]), "=&v"(A[1]), "=&v"(A[2])
+          : "v"(piece_at(p)), "v"(piece_at(p + 1)), "v"(piece_at(p + 2))
+          : "memory");
+    }
+#pragma unroll
+    for (int k = 0; k < pt_vals<S>(); ++k) v[k] = piece<S>(A, k);
+    if (q == 1) {
+      if constexpr (kDbl) start_line(k, 1, 0);
+      next = lds_int(addr(codes(k + 1)) + 4 * threadIdx.x);
+      if (more) {
+        if constexpr (kDbl)
+          start_rows(k + 1);
+        else
+          start_line(k + 1, 0, 0);
+      }
+    }
+    if (q == 3 && more) {
+      start_line(k + 1, kDbl ? 0 : 1, kDbl ? 0 : kLine);
+      start_code(k + 2);
+    }
+  }
+  __device__ __forceinline__ unsigned piece_at(int p) const {
+    return (at ^ ((p & 7) << 4)) + 16 * kLine * (p >> 3);
+  }
+  // no load may write to LDS that the wavefront has given back
+  __device__ __forceinline__ void finish() const { loads_but<0>(); }
+};
 
 struct QpArgs {
   const int* ien;          // 4 planes of nel (0-based)
   const double* node;      // 16 per node: y (p,u,v,w,T), ac (same order), x
   const double* qnode;     // 16 per node: reconstructed diffusive flux (12)
-  void* qps;               // (nel*4) x 12 point states (S)
-  void* geo;               // nel x 13 (S), padded to 16 floats / 14 doubles
+  void* qps;               // (nel*4) point records (S)
+  void* geo;               // nel x 16 rows (double; float: in qps)
   double* resid;           // (nel*4) x 5 residual of element e at its node a
   double* dcw;             // nel*4 discontinuity-capturing factor per point (iDC != 0)
   void* mtau;              // nel*4 x mt_stride W PTau per point (itau = 10), S
@@ -756,13 +1073,14 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   tet_shg(ix, shg);
   double G[6], trG, GG;
   tet_metric_tensor(ix, G, trG, GG);
-  if (valid && q == 0) {
-    S* go = reinterpret_cast<S*>(A.geo) + (size_t)e * rec_stride<S>();
+  if (valid) {
+    // lane q stores node q's row
+    S* go = row_at<S>(reinterpret_cast<S*>(A.qps), reinterpret_cast<S*>(A.geo), e, q);
+    S g4[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) go[3 * k + c] = (S)shg[k][c];
-    go[12] = (S)WdetJ;
+    for (int c = 0; c < 3; ++c) g4[c] = (S)sel4(shg[0][c], shg[1][c], shg[2][c], shg[3][c], q);
+    g4[3] = (S)WdetJ;
+    store_vals<S>(go, g4, 4);
   }
 
   // nodal y and ac streamed into the point values and the (element-
@@ -805,29 +1123,26 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   double ei, rk;
   point_thermo(Y, ph, G, trG, GG, t, ei, rk);
   if (valid) {
-    S v[12];
+    S v[pt_vals<S>()];
     v[0] = (S)t.u[0];
     v[1] = (S)t.u[1];
     v[2] = (S)t.u[2];
-    v[kPtRho] = (S)t.rho;
-    v[kPtDrdp] = (S)t.drdp;
-    v[kPtDrdT] = (S)t.drdT;
-    v[kPtE1p] = (S)t.e1p;
-    v[kPtE3p] = (S)t.e3p;
-    v[kPtE4p] = (S)t.e4p;
-    v[kPtT0] = (S)(WdetJ * t.tau[0]);
-    v[kPtT1] = (S)(WdetJ * t.tau[1]);
-    v[kPtT2] = (S)(WdetJ * t.tau[2]);
-    S* o = reinterpret_cast<S*>(A.qps) + ((size_t)e * 4 + q) * pt_stride<S>();
-    if constexpr (sizeof(S) == 8) {
-      double2* o2 = reinterpret_cast<double2*>(o);
-#pragma unroll
-      for (int i = 0; i < 6; ++i) o2[i] = make_double2(v[2 * i], v[2 * i + 1]);
+    v[3] = (S)t.rho;
+    v[4] = (S)t.drdp;
+    if constexpr (sizeof(S) == 4) {
+      v[5] = (S)t.drdT;
+      v[6] = (S)t.e1p;
+      v[7] = (S)t.e3p;
+      v[8] = (S)t.e4p;
+      v[9] = (S)(WdetJ * t.tau[0]);
+      v[10] = (S)(WdetJ * t.tau[1]);
+      v[11] = (S)(WdetJ * t.tau[2]);
     } else {
-      float4* o4 = reinterpret_cast<float4*>(o);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) o4[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+      v[5] = ph.itau == 1 ? WdetJ * t.tau[2] : t.e3p;
+      v[6] = WdetJ * t.tau[0];
+      v[7] = WdetJ * t.tau[1];
     }
+    store_vals<S>(pt_at<S>(reinterpret_cast<S*>(A.qps), e, q), v, pt_vals<S>());
   }
   double PT[5][5], ixr[3][3];
   if constexpr (kMT) {
@@ -1208,95 +1523,128 @@ __global__ void __launch_bounds__(256) k_jv_nodes(const long long* __restrict__ 
 }
 
 // ---------------- pass 2: block owners ----------------
-// One point's WdetJ P Q with Shakib's diagonal tau, added to ac (row + 5
-// column): P = A(sP) diag(W tau) + NaP I (NaP = WdetJ N_a), Q = A(sQ) +
-// c NbQ A0 (NbQ = N_b).  With the products of the state with W tau, P's
-// row 0 is v + N_a e_0, v = (W t0 drdp una, W t1 rho s, W t2 drdT una);
-// rows 1+k are u_k v + (W t0 s_k) e_0 + dg e_{1+k}, dg = W t1 rho una + N_a;
-// row 4 is (W t0 e2p una, W t1 e3p s + (W t1 rho una) u, W t2 e4p una +
-// N_a).  Q's rows 1+k are u_k Q0 + r_k e_0 + rho w e_{1+k} (Q0 its row 0,
-// r = sQ, w = u.r + c N_b), so with vQ = v Q
-//   (P Q)(0)   = vQ + N_a Q0
-//   (P Q)(1+k) = u_k (vQ + dg Q0) + (W t0 s_k) Q0 + dg r_k e_0 + dg rho w e_{1+k}
-// and row 4 through the same factored Q.
+// WdetJ P Q with a diagonal tau (Shakib's or Franca's), P = A(sP) diag(W tau) +
+// NaP I, Q = A(sQ) + c NbQ A0, in terms of the point's scalars and u alone.
+// With a = u.sP, b = u.sQ, w = b + c N_b, t_i = W tau_i, beta = t_1 rho, and
+//   Q0 = (drdp w, rho sQ, drdT w),  Q4 = (q40, e3p sQ + rho w u, e4p w),
+//   Qk = u_k Q0 + sQ_k e_0 + rho w e_k
+// the rows of P Q are
+//   row 0: R = al Q0 + beta (st e_0 + rho w sP) + p04 Q4
+//   row k: u_k (R + ba Q0) + t_0 sP_k Q0 + dg (sQ_k e_0 + rho w e_k)
+//   row 4: ga Q0 + t_1 e3p (st e_0 + rho w sP) + ba (b e_0 + rho w u) + p44 Q4
+// with st = sP.sQ, ba = beta a, dg = ba + N_a, al = t_0 drdp a + dg, p04 = t_2
+// drdT a, ga = a (t_0 e2p + t_1 e3p + 2 beta k), p44 = t_2 e4p a + N_a.  sP and
+// sQ do not depend on the point, so the terms that are a scalar times one of
+// them (or times their outer product) are summed over the points as scalars
+// (DiagSums) and applied once per element: 65 operations per block and point
+// and 25 per block and element beside the shared scalars, against 132 per
+// block and point when every term went to its entry at once.
 template <typename R>
-__device__ __forceinline__ void shakib_pq(const R uq[3], R rho, R drdp, R drdT, R e1p, R e3p,
-                                          R e4p, R t0, R wt1, R wt2, R cfacR, const R sP[3],
-                                          const R sQ[3], R NaP, R NbQ, R ac[25]) {
-  const R u0 = uq[0], u1 = uq[1], u2 = uq[2];
-  const R e2p = e1p + (R)1;
-  const R una = u0 * sP[0] + u1 * sP[1] + u2 * sP[2];
-  const R unb = u0 * sQ[0] + u1 * sQ[1] + u2 * sQ[2];
-  const R w = unb + cfacR * NbQ;
-  const R q00 = drdp * w, q04 = drdT * w, rw = rho * w;
-  R q0[3], q4[3];
+struct DiagPt {  // one point, shared by all blocks
+  R u[3], rho, e3p, e1p, drdp, drdT, e2p, e4p, t0, beta, betae, t0drdp, t2drdT, t2e4p, g0;
+  __device__ __forceinline__ explicit DiagPt(const Pt<R>& p)
+      : u{p.u[0], p.u[1], p.u[2]}, rho(p.rho), e3p(p.e3p), e1p(p.e1p), drdp(p.drdp),
+        drdT(p.drdT), e2p(p.e1p + (R)1), e4p(p.e4p), t0(p.t0), beta(p.t1 * p.rho),
+        betae(p.t1 * p.e3p), t0drdp(p.t0 * p.drdp), t2drdT(p.t2 * p.drdT), t2e4p(p.t2 * p.e4p) {
+    const R uu = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+    g0 = t0 * e2p + betae + beta * uu;
+  }
+};
+
+template <typename R>
+struct DiagRow {  // the row's node at the point (WN = WdetJ N)
+  R ba, dg, al, p04, ga, p44;
+  __device__ __forceinline__ DiagRow(const DiagPt<R>& p, R a, R WN)
+      : ba(p.beta * a), dg(ba + WN), al(p.t0drdp * a + dg), p04(p.t2drdT * a), ga(p.g0 * a),
+        p44(p.t2e4p * a + WN) {}
+};
+
+template <typename R>
+struct DiagCol {  // the column's node at the point (cN = c N)
+  R a, dw, Tw, rw, q40, q44;
+  __device__ __forceinline__ DiagCol(const DiagPt<R>& p, R a, R cN)
+      : a(a), dw(p.drdp * (a + cN)), Tw(p.drdT * (a + cN)), rw(p.rho * (a + cN)),
+        q40(p.e2p * a + cN * p.e1p), q44(p.e4p * (a + cN)) {}
+};
+
+template <typename R>
+struct DiagSums {  // of one block, over the element's points
+  R tdw = 0, tTw = 0, dg = 0, dgrw = 0, D = 0, E = 0;
+};
+
+// one point of the block (row node P, column node Q) into ac and S
+template <typename R>
+__device__ __forceinline__ void diag_point(const DiagPt<R>& p, const DiagRow<R>& P,
+                                           const DiagCol<R>& Q, R st, const R sP[3],
+                                           const R sQ[3], R ac[25], DiagSums<R>& S) {
+  R Z[5];
+  const R r0 = P.al * Q.dw + P.p04 * Q.q40 + p.beta * st;
+  const R r4 = P.al * Q.Tw + P.p04 * Q.q44;
+  ac[0] += r0;
+  ac[20] += r4;
+  Z[0] = r0 + P.ba * Q.dw;
+  Z[4] = r4 + P.ba * Q.Tw;
+  const R A = P.al * p.rho + P.p04 * p.e3p, X = P.ba * p.rho;
+  const R B = p.beta * Q.rw, C = P.p04 * Q.rw;
 #pragma unroll
   for (int n = 0; n < 3; ++n) {
-    q0[n] = rho * sQ[n];
-    q4[n] = e3p * sQ[n] + rw * uq[n];
+    const R e = A * sQ[n] + B * sP[n] + C * p.u[n];
+    ac[5 * (1 + n)] += e;
+    Z[1 + n] = e + X * sQ[n];
   }
-  const R q40 = e2p * unb + cfacR * NbQ * e1p, q44 = e4p * w;
-  const R rt1 = wt1 * rho, pt0 = t0 * drdp, tt2 = wt2 * drdT;
-  const R et0 = t0 * e2p, et1 = wt1 * e3p, et2 = wt2 * e4p;
-  const R a0 = pt0 * una, r1 = rt1 * una, p04 = tt2 * una, dg = r1 + NaP;
-  const R v1[3] = {rt1 * sP[0], rt1 * sP[1], rt1 * sP[2]};
-  const R Q0[5] = {q00, q0[0], q0[1], q0[2], q04};
-  const R sg = a0 + (v1[0] * u0 + v1[1] * u1 + v1[2] * u2);
-  const R rg = v1[0] * sQ[0] + v1[1] * sQ[1] + v1[2] * sQ[2];
-  R vQ[5];
-  vQ[0] = sg * q00 + rg + p04 * q40;
 #pragma unroll
-  for (int n = 0; n < 3; ++n) vQ[1 + n] = sg * q0[n] + rw * v1[n] + p04 * q4[n];
-  vQ[4] = sg * q04 + p04 * q44;
-  // row 0
+  for (int c = 0; c < 5; ++c)
 #pragma unroll
-  for (int c = 0; c < 5; ++c) ac[5 * c] += vQ[c] + NaP * Q0[c];
-  // rows 1..3
-  R Z[5];
+    for (int k = 0; k < 3; ++k) ac[(1 + k) + 5 * c] += p.u[k] * Z[c];
+  S.tdw += p.t0 * Q.dw;
+  S.tTw += p.t0 * Q.Tw;
+  S.dg += P.dg;
+  S.dgrw += P.dg * Q.rw;
+  // (summed first, then added: in float every addition to a sum over points and
+  // elements rounds at the size of that sum)
+  ac[4] += P.ga * Q.dw + P.ba * Q.a + P.p44 * Q.q40;
+  S.D += P.ga * p.rho + P.p44 * p.e3p;
+  S.E += p.betae * Q.rw;
+  const R F = (P.ba + P.p44) * Q.rw;
 #pragma unroll
-  for (int c = 0; c < 5; ++c) Z[c] = vQ[c] + dg * Q0[c];
-  const R dgrw = dg * rw;
+  for (int n = 0; n < 3; ++n) ac[4 + 5 * (1 + n)] += F * p.u[n];
+  ac[24] += P.ga * Q.Tw + P.p44 * Q.q44;
+}
+
+// the element's sums of a block; be = sum_q t_1 e3p (t_0 rho sP sQ^T goes with
+// the viscous block's outer product, visc_add)
+template <typename R>
+__device__ __forceinline__ void diag_element(const DiagSums<R>& S, R be, R st, const R sP[3],
+                                             const R sQ[3], R ac[25]) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const R ts = t0 * sP[k];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      R& ck = ac[(1 + k) + 5 * c];
-      ck += uq[k] * Z[c];
-      ck += ts * Q0[c];
-    }
-    ac[1 + k] += dg * sQ[k];
-    ac[(1 + k) + 5 * (1 + k)] += dgrw;
+    ac[1 + k] += S.tdw * sP[k] + S.dg * sQ[k];
+    ac[(1 + k) + 20] += S.tTw * sP[k];
+    ac[(1 + k) + 5 * (1 + k)] += S.dgrw;
+    ac[4 + 5 * (1 + k)] += S.D * sQ[k] + S.E * sP[k];
   }
-  // row 4
-  const R p40 = et0 * una, p44 = et2 * una + NaP;
-  R p4[3];
-#pragma unroll
-  for (int n = 0; n < 3; ++n) p4[n] = et1 * sP[n] + r1 * uq[n];
-  const R s4 = p40 + (p4[0] * u0 + p4[1] * u1 + p4[2] * u2);
-  ac[4] += s4 * q00 + (p4[0] * sQ[0] + p4[1] * sQ[1] + p4[2] * sQ[2]) + p44 * q40;
-#pragma unroll
-  for (int n = 0; n < 3; ++n) ac[4 + 5 * (1 + n)] += s4 * q0[n] + rw * p4[n] + p44 * q4[n];
-  ac[24] += s4 * q04 + p44 * q44;
+  ac[4] += be * st;
 }
 
 // sum_q WdetJ K_ab of one element block (e3visc.f's stiffness through
 // e3wmlt): the momentum rows and the conduction term do not depend on the
 // point (4 equal weights), the energy row only through the velocity,
-// linearly (ub = the sum of the point velocities)
+// linearly (ub = the sum of the point velocities).  outer: another multiple
+// of sP sQ^T for the momentum rows.
 template <typename R>
 __device__ __forceinline__ void visc_add(R W, const R sP[3], const R sQ[3], const R ub[3],
-                                         R muR, R lamR, R kapR, R ac[25]) {
+                                         R muR, R lamR, R kapR, R outer, R ac[25]) {
   const R W4 = (R)4 * W;
   const R st = sP[0] * sQ[0] + sP[1] * sQ[1] + sP[2] * sQ[2];
   const R ubs = ub[0] * sP[0] + ub[1] * sP[1] + ub[2] * sP[2];
   const R ubr = ub[0] * sQ[0] + ub[1] * sQ[1] + ub[2] * sQ[2];
+  const R Wm = W4 * muR, Wl = W4 * lamR + outer, Ws = Wm * st;
 #pragma unroll
   for (int m = 0; m < 3; ++m)
 #pragma unroll
     for (int n = 0; n < 3; ++n)
       ac[(1 + m) + 5 * (1 + n)] +=
-          W4 * (muR * ((m == n ? st : (R)0) + sP[n] * sQ[m]) + lamR * sP[m] * sQ[n]);
+          (m == n ? Ws : (R)0) + (Wm * sQ[m]) * sP[n] + (Wl * sP[m]) * sQ[n];
 #pragma unroll
   for (int n = 0; n < 3; ++n)
     ac[4 + 5 * (1 + n)] += W * (muR * (st * ub[n] + sP[n] * ubr) + lamR * ubs * sQ[n]);
@@ -1304,8 +1652,8 @@ __device__ __forceinline__ void visc_add(R W, const R sP[3], const R sQ[3], cons
 }
 
 // One point's WdetJ P Q with the matrix tau, added to ac (row + 5
-// column): P = A(sP) (W PTau) + NaP I, Q = A(sQ) + c NbQ A0 in the factored
-// form of shakib_pq (Q's rows 0 and 4 and rho w; with pu = sum_k P(m,k) u_k
+// column): P = A(sP) (W PTau) + NaP I, Q = A(sQ) + c NbQ A0 in factored
+// form (Q's rows 0 and 4 and rho w; with pu = sum_k P(m,k) u_k
 // and Sm = P(m,0) + pu, row m of P Q is
 //   column 0:    Sm q00 + sum_k P(m,k) r_k + P(m,4) q40
 //   column 1+n:  Sm q0n + rho w P(m,1+n) + P(m,4) q4n
@@ -1429,8 +1777,15 @@ struct BlkArgs {
   long long nel, nlanes;
   int lhs_on, prec_on;
   double mu, lam, kap, cfac;
+  double Rg, e1c, cpR, kt2;  // PtConst
+  int franca;
   long long* clk;          // device clock at the start
 };
+
+template <typename R>
+__device__ __forceinline__ PtConst<R> pt_const(const BlkArgs& A) {
+  return PtConst<R>{(R)A.Rg, (R)A.e1c, (R)A.cpR, (R)A.kt2, A.franca != 0};
+}
 
 // T: stored block type and arithmetic type of the per-point tangent (float
 // on the mixed path); S: storage type of the point states.  Sums over
@@ -1455,6 +1810,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
   const long long l = wg * 64 + threadIdx.x;
   int4 L = make_int4(0, 0, 0, 0);
   if (l < A.nlanes) L = A.lanes[l];
+  __shared__ phg_i4 lds[Pipe<T, S>::kPieces];
   const bool diag = (L.w >> 1) & 1;
   const int cnt = (A.lhs_on || diag) ? L.z : 0;
   // block sums in the tangent's type (float accumulation on the mixed
@@ -1466,23 +1822,33 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
   const S* qps = reinterpret_cast<const S*>(A.qps);
   const S* geo = reinterpret_cast<const S*>(A.geo);
   const R muR = (R)A.mu, lamR = (R)A.lam, kapR = (R)A.kap, cfacR = (R)A.cfac;
-  for (int k = 0; k < cnt; ++k) {
-    const int code = A.blocks[L.x + k];
+  const PtConst<R> pc = pt_const<R>(A);
+  // a wavefront walks its longest lane's blocks.  Lanes past theirs load with
+  // their quad, their own last block again, and add zeros: every term has a
+  // shape gradient or WdetJ N, which they set to zero
+  Pipe<R, S> pipe(qps, geo, A.blocks, L.x, cnt, lds);
+  int code = pipe.code_at(0);
+  const bool any = __ballot(cnt > 0);
+  if (any) pipe.start(code);
+  // (tested at its end: the compiler does not turn a loop whose test is a vote,
+  // and kept a copy of the sums for the exit)
+  for (int k = 0; any;) {
+    const bool on = k < cnt, more = __ballot(k + 1 < cnt);
     const long long e = code >> 4;
     const int a = (code >> 2) & 3, b = code & 3;
-    // the two shape gradients and WdetJ of the element's geometry record
-    // the element's geometry record with 16-byte loads, then the two rows
-    S g16[16];
-    load_rec<S>(geo + (size_t)e * rec_stride<S>(), g16);
     R sR[3], rR[3];
+    int next = 0;
+    R W = pipe.rows(code, sR, rR);
+    if (!on) {
+      W = (R)0;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      sR[c] = (R)sel4t(g16[c], g16[3 + c], g16[6 + c], g16[9 + c], a);
-      rR[c] = (R)sel4t(g16[c], g16[3 + c], g16[6 + c], g16[9 + c], b);
+      for (int c = 0; c < 3; ++c) sR[c] = rR[c] = (R)0;
     }
-    const R W = (R)g16[12];
     // acc += WdetJ [P Q] per point: the stored tau is WdetJ tau and N_a is
     // scaled here, so P's rows come out multiplied by WdetJ
+    const R st = sR[0] * rR[0] + sR[1] * rR[1] + sR[2] * rR[2];
+    DiagSums<R> S1;
+    R be = (R)0, outer = (R)0;
     R ub[3] = {(R)0, (R)0, (R)0};  // sum of the point velocities
     // kDC: sum_q DC_q A0(q) through its distinct entries: drdp, drdT,
     // drdp u (3), drdT u (3), rho, rho u (3), e1p, e4p
@@ -1491,21 +1857,18 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
 #pragma unroll
       for (int i = 0; i < 14; ++i) dA[i] = (R)0;
     }
-    const S* qrec = qps + (size_t)e * 4 * pt_stride<S>();
-    // float: unrolled so the four points' record loads issue together
-    // (2.6% at 128^3); double: the unrolled body spills
-    constexpr int kPtUnroll = sizeof(S) == 4 ? 4 : 1;
-#pragma unroll kPtUnroll
+#pragma unroll 1
     for (int q = 0; q < 4; ++q) {
-      S o[12];
-      load_pt<S>(qrec + q * pt_stride<S>(), o);
-      const R u0 = (R)o[0], u1 = (R)o[1], u2 = (R)o[2];
-      const R uq[3] = {u0, u1, u2};
-      ub[0] += u0;
-      ub[1] += u1;
-      ub[2] += u2;
-      const R rho = (R)o[kPtRho], drdp = (R)o[kPtDrdp], drdT = (R)o[kPtDrdT];
-      const R e1p = (R)o[kPtE1p], e2p = e1p + (R)1, e3p = (R)o[kPtE3p], e4p = (R)o[kPtE4p];
+      S v[pt_vals<S>()];
+      R Nqa, Nqb;
+      pipe.point(q, k, more, code, next, v, Nqa, Nqb);
+      const Pt<R> pt = decode_pt<R, S>(v, pc);
+      const R uq[3] = {pt.u[0], pt.u[1], pt.u[2]};
+      ub[0] += uq[0];
+      ub[1] += uq[1];
+      ub[2] += uq[2];
+      const R rho = pt.rho, drdp = pt.drdp, drdT = pt.drdT;
+      const R e1p = pt.e1p, e2p = e1p + (R)1, e3p = pt.e3p, e4p = pt.e4p;
       if constexpr (kDC) {
         // weight of the point's A0: DC (the element's giju is applied after
         // the loop), or with the matrix tau s_a . (DC giju_q) s_b of the
@@ -1523,15 +1886,13 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
         }
         dc_point<R>(dq, drdp, drdT, rho, uq, e1p, e4p, dA);
       }
-      const R Na = W * (R)sel4(cQ.N[q][0], cQ.N[q][1], cQ.N[q][2], cQ.N[q][3], a);
-      const R Nb = (R)sel4(cQ.N[q][0], cQ.N[q][1], cQ.N[q][2], cQ.N[q][3], b);
       if constexpr (kMT) {
         // rows of P = A(s_a) W PTau + N_a I from the point's W PTau
         R WPT[25];
         const S* mp = reinterpret_cast<const S*>(A.mtau) + ((size_t)e * 4 + q) * mt_stride<S>();
 #pragma unroll
         for (int k = 0; k < 25; ++k) WPT[k] = (R)mp[k];
-        mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, sR, rR, Na, Nb, acc);
+        mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, sR, rR, W * Nqa, Nqb, acc);
         if constexpr (kNd) {
           // row m of A_k (the flux Jacobian along x_k, pressure-primitive)
           auto arow = [&](int k, int m, R r[5]) {
@@ -1608,21 +1969,31 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
           acc[4 + 10] += s2 * ((Wt[1][4] - Wt[3][4]) * r4[2]);
         }
       } else {
-        shakib_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, (R)o[kPtT0], (R)o[kPtT1],
-                     (R)o[kPtT2], cfacR, sR, rR, Na, Nb, acc);
+        const DiagPt<R> dp(pt);
+        const R ua = uq[0] * sR[0] + uq[1] * sR[1] + uq[2] * sR[2];
+        const R ub_ = uq[0] * rR[0] + uq[1] * rR[1] + uq[2] * rR[2];
+        diag_point<R>(dp, DiagRow<R>(dp, ua, W * Nqa), DiagCol<R>(dp, ub_, cfacR * Nqb), st, sR,
+                      rR, acc, S1);
+        be += dp.betae;
+        outer += dp.t0 * dp.rho;
       }
     }
     // viscous part sum_q WdetJ K_ab
-    visc_add<R>(W, sR, rR, ub, muR, lamR, kapR, acc);
+    visc_add<R>(W, sR, rR, ub, muR, lamR, kapR, outer, acc);
+    if constexpr (!kMT) diag_element<R>(S1, be, st, sR, rR, acc);
     if constexpr (kDC) {
       R sab = (R)1;
       if constexpr (!kMT) {
         // giju of the element from dxi/dx = 2 (shape gradients of nodes 1..3)
         R ix[3][3], G[6], trG, GG, gu[6];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < 3; ++k) {
+          const S* rk = row_at<const S>(qps, geo, e, k);
 #pragma unroll
-          for (int c = 0; c < 3; ++c) ix[k][c] = (R)2 * (R)g16[3 * k + c];
+          for (int c = 0; c < 3; ++c) ix[k][c] = (R)rk[c];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) ix[k][c] *= (R)2;
+        }
         tet_metric_tensor(ix, G, trG, GG);
         metric_inverse(G, gu);
         sab = (R)0;
@@ -1633,14 +2004,23 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
       }
       dc_block<R>(W * sab, dA, acc);
     }
+    code = next;
+    ++k;
+    if (!more) break;
   }
+  pipe.finish();
   // the node's residual: element residuals of the diagonal blocks' elements
   if (diag) {
     for (int k = 0; k < cnt; ++k) {
       const int code = A.blocks[L.x + k];
       const double* ro = A.resid + ((size_t)(code >> 4) * 4 + ((code >> 2) & 3)) * 5;
-#pragma unroll
-      for (int f = 0; f < 5; ++f) racc[f] += ro[f];
+      const phg_d2u r01 = *reinterpret_cast<const phg_d2u*>(ro);
+      const phg_d2u r23 = *reinterpret_cast<const phg_d2u*>(ro + 2);
+      racc[0] += r01.x;
+      racc[1] += r01.y;
+      racc[2] += r23.x;
+      racc[3] += r23.y;
+      racc[4] += ro[4];
     }
   }
   // combine the chunks of one block in lane order: the leader adds the
@@ -1719,28 +2099,17 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
 
 // The block pass with lhsK: the entries (A,B) and (B,A) come from the same
 // element blocks with a and b exchanged, so one lane forms both from one
-// read of the point records (the pass is bound by those per-lane reads).
+// read of the point records.
 // Diagonal entries run in wavefronts of their own, so every lane of a
 // wavefront forms the same number of blocks.  Same arithmetic per block as
 // k_asm_blocks; with DC (kDC) the point weights and s_a.giju s_b are
 // symmetric in a and b and serve both blocks; the matrix tau (kMT) through
 // mtau_pq.  Used for every flag set in float, for Shakib's or Franca's tau
 // without DC in double (the other double variants exceed the registers).
-template <typename T, typename S, bool kDC, bool kMT>
-__device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
+template <typename T, typename S, bool kDC, bool kMT, bool kPair>
+__device__ __forceinline__ void asm_pairs_wave(const BlkArgs& A, const int4 L, const int k2,
+                                               phg_i4* lds) {
   using R = T;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *A.clk = wall_clock64();
-  const long long per = (gridDim.x + 7) / 8;
-  const long long wg = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  const long long l = wg * 64 + threadIdx.x;
-  int4 L = make_int4(0, 0, 0, 0);
-  int k2 = -1;
-  if (l < A.nlanes) {
-    L = A.lanes[l];
-    k2 = A.lanes_k2[l];
-  }
-  const bool diag = (L.w >> 1) & 1;
-  const bool pair = k2 >= 0;
   const int cnt = L.z;
   R acc[25], acc2[25];
 #pragma unroll
@@ -1749,43 +2118,50 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
   const S* qps = reinterpret_cast<const S*>(A.qps);
   const S* geo = reinterpret_cast<const S*>(A.geo);
   const R muR = (R)A.mu, lamR = (R)A.lam, kapR = (R)A.kap, cfacR = (R)A.cfac;
-  for (int k = 0; k < cnt; ++k) {
-    const int code = A.blocks[L.x + k];
+  const PtConst<R> pc = pt_const<R>(A);
+  // a wavefront walks its longest lane's blocks.  Lanes past theirs load with
+  // their quad, their own last block again, and add zeros: every term has a
+  // shape gradient or WdetJ N, which they set to zero
+  Pipe<R, S> pipe(qps, geo, A.blocks, L.x, cnt, lds);
+  int code = pipe.code_at(0);
+  const bool any = __ballot(cnt > 0);
+  if (any) pipe.start(code);
+  // (tested at its end: the compiler does not turn a loop whose test is a vote,
+  // and kept a copy of the sums for the exit)
+  for (int k = 0; any;) {
+    const bool on = k < cnt, more = __ballot(k + 1 < cnt);
     const long long e = code >> 4;
     const int a = (code >> 2) & 3, b = code & 3;
-    S g16[16];
-    load_rec<S>(geo + (size_t)e * rec_stride<S>(), g16);
     R sR[3], rR[3];
+    int next = 0;
+    R W = pipe.rows(code, sR, rR);
+    if (!on) W = (R)0;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      sR[c] = (R)sel4t(g16[c], g16[3 + c], g16[6 + c], g16[9 + c], a);
-      rR[c] = (R)sel4t(g16[c], g16[3 + c], g16[6 + c], g16[9 + c], b);
+      if (!on) sR[c] = rR[c] = (R)0;
+      if constexpr (!kPair) rR[c] = sR[c];  // a diagonal entry's blocks have a = b
     }
-    const R W = (R)g16[12];
+    const R st = sR[0] * rR[0] + sR[1] * rR[1] + sR[2] * rR[2];
+    DiagSums<R> S1, S2;
+    R be = (R)0, outer = (R)0;
     R ub[3] = {(R)0, (R)0, (R)0};
     R dA[14];
     if constexpr (kDC) {
 #pragma unroll
       for (int i = 0; i < 14; ++i) dA[i] = (R)0;
     }
-    const S* qrec = qps + (size_t)e * 4 * pt_stride<S>();
-    // float: two points' record loads in flight (136 VGPRs, three
-    // wavefronts per SIMD: 8.23 ms at 128^3 against 8.51 not unrolled);
-    // double and the DC / matrix-tau variants: not unrolled (registers)
-    constexpr int kPairUnroll = (sizeof(S) == 4 && !kDC && !kMT) ? 2 : 1;
-#pragma unroll kPairUnroll
+#pragma unroll 1
     for (int q = 0; q < 4; ++q) {
-      S o[12];
-      load_pt<S>(qrec + q * pt_stride<S>(), o);
-      const R uq[3] = {(R)o[0], (R)o[1], (R)o[2]};
+      S v[pt_vals<S>()];
+      R Nqa, Nqb;
+      pipe.point(q, k, more, code, next, v, Nqa, Nqb);
+      const Pt<R> pt = decode_pt<R, S>(v, pc);
+      const R uq[3] = {pt.u[0], pt.u[1], pt.u[2]};
       ub[0] += uq[0];
       ub[1] += uq[1];
       ub[2] += uq[2];
-      const R rho = (R)o[kPtRho], drdp = (R)o[kPtDrdp], drdT = (R)o[kPtDrdT];
-      const R e1p = (R)o[kPtE1p], e3p = (R)o[kPtE3p], e4p = (R)o[kPtE4p];
-      const R t0 = (R)o[kPtT0], wt1 = (R)o[kPtT1], wt2 = (R)o[kPtT2];
-      const R Nqa = (R)sel4(cQ.N[q][0], cQ.N[q][1], cQ.N[q][2], cQ.N[q][3], a);
-      const R Nqb = (R)sel4(cQ.N[q][0], cQ.N[q][1], cQ.N[q][2], cQ.N[q][3], b);
+      const R rho = pt.rho, drdp = pt.drdp, drdT = pt.drdT;
+      const R e1p = pt.e1p, e3p = pt.e3p, e4p = pt.e4p;
       if constexpr (kDC) {
         R dq;
         if constexpr (kMT) {
@@ -1807,28 +2183,47 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
 #pragma unroll
         for (int k = 0; k < 25; ++k) WPT[k] = (R)mp[k];
         mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, sR, rR, W * Nqa, Nqb, acc);
-        if (pair)
+        if constexpr (kPair)
           mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, rR, sR, W * Nqb, Nqa,
                      acc2);
       } else {
-        shakib_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, t0, wt1, wt2, cfacR, sR, rR, W * Nqa,
-                     Nqb, acc);
-        if (pair)
-          shakib_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, t0, wt1, wt2, cfacR, rR, sR,
-                       W * Nqb, Nqa, acc2);
+        const DiagPt<R> dp(pt);
+        const R ua = uq[0] * sR[0] + uq[1] * sR[1] + uq[2] * sR[2];
+        if constexpr (kPair) {
+          const R ub_ = uq[0] * rR[0] + uq[1] * rR[1] + uq[2] * rR[2];
+          diag_point<R>(dp, DiagRow<R>(dp, ua, W * Nqa), DiagCol<R>(dp, ub_, cfacR * Nqb), st,
+                        sR, rR, acc, S1);
+          // (one block after the other: the second's scalars would not fit beside the first's)
+          if constexpr (sizeof(R) == 8) __builtin_amdgcn_sched_barrier(0);
+          diag_point<R>(dp, DiagRow<R>(dp, ub_, W * Nqb), DiagCol<R>(dp, ua, cfacR * Nqa), st,
+                        rR, sR, acc2, S2);
+        } else {
+          diag_point<R>(dp, DiagRow<R>(dp, ua, W * Nqa), DiagCol<R>(dp, ua, cfacR * Nqa), st,
+                        sR, sR, acc, S1);
+        }
+        be += dp.betae;
+        outer += dp.t0 * dp.rho;
       }
     }
-    visc_add<R>(W, sR, rR, ub, muR, lamR, kapR, acc);
-    if (pair) visc_add<R>(W, rR, sR, ub, muR, lamR, kapR, acc2);
+    visc_add<R>(W, sR, rR, ub, muR, lamR, kapR, outer, acc);
+    if constexpr (!kMT) diag_element<R>(S1, be, st, sR, rR, acc);
+    if constexpr (kPair) {
+      visc_add<R>(W, rR, sR, ub, muR, lamR, kapR, outer, acc2);
+      if constexpr (!kMT) diag_element<R>(S2, be, st, rR, sR, acc2);
+    }
     if constexpr (kDC) {
       R sab = (R)1;
       if constexpr (!kMT) {
         // giju of the element from dxi/dx = 2 (shape gradients of nodes 1..3)
         R ix[3][3], G[6], trG, GG, gu[6];
 #pragma unroll
-        for (int kk = 0; kk < 3; ++kk)
+        for (int kk = 0; kk < 3; ++kk) {
+          const S* rk = row_at<const S>(qps, geo, e, kk);
 #pragma unroll
-          for (int c = 0; c < 3; ++c) ix[kk][c] = (R)2 * (R)g16[3 * kk + c];
+          for (int c = 0; c < 3; ++c) ix[kk][c] = (R)rk[c];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) ix[kk][c] *= (R)2;
+        }
         tet_metric_tensor(ix, G, trG, GG);
         metric_inverse(G, gu);
         sab = (R)0;
@@ -1838,49 +2233,59 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
           for (int j = 0; j < 3; ++j) sab += sR[i] * gu[gu_idx(i, j)] * rR[j];
       }
       dc_block<R>(W * sab, dA, acc);
-      if (pair) dc_block<R>(W * sab, dA, acc2);
+      if constexpr (kPair) dc_block<R>(W * sab, dA, acc2);
     }
+    code = next;
+    ++k;
+    if (!more) break;
   }
-  if (diag) {
+  pipe.finish();
+  if constexpr (!kPair) {
     for (int k = 0; k < cnt; ++k) {
       const int code = A.blocks[L.x + k];
       const double* ro = A.resid + ((size_t)(code >> 4) * 4 + ((code >> 2) & 3)) * 5;
-#pragma unroll
-      for (int f = 0; f < 5; ++f) racc[f] += ro[f];
+      const phg_d2u r01 = *reinterpret_cast<const phg_d2u*>(ro);
+      const phg_d2u r23 = *reinterpret_cast<const phg_d2u*>(ro + 2);
+      racc[0] += r01.x;
+      racc[1] += r01.y;
+      racc[2] += r23.x;
+      racc[3] += r23.y;
+      racc[4] += ro[4];
     }
   }
-  // chunk combine as in k_asm_blocks, one block at a time (the second one's
-  // partials move only in wavefronts of pairs, wavefront-uniform: padding
-  // lanes hold zeros), each stored by the leader before the next
-  const bool leader = (L.w & 1) && l < A.nlanes;
+  // chunk combine as in k_asm_blocks, one block at a time, each stored by the
+  // leader before the next
+  const bool leader = L.w & 1;
   const int nch = (L.w >> 8) & 0xff;
   const int total = L.w >> 16;
-  int mx = nch, wp = pair ? 1 : 0;
+  int mx = nch;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    mx = max(mx, __shfl_xor(mx, o, 64));
-    wp = max(wp, __shfl_xor(wp, o, 64));
-  }
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
   R csum[25];
-  auto combine = [&](const R* ac) {
+  auto combine = [&](R* ac) {
 #pragma unroll
     for (int i = 0; i < 25; ++i) csum[i] = ac[i];
     for (int c = 1; c < mx; ++c) {
 #pragma unroll
       for (int i = 0; i < 25; ++i) {
-        const R v = __shfl_down(ac[i], c, 64);
-        if (c < nch) csum[i] += v;
+        ac[i] = next_lane(ac[i]);
+        if (c < nch) csum[i] += ac[i];
       }
     }
   };
-  if (!wp) {
+  if constexpr (!kPair) {
+    double rsum[5];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) rsum[f] = racc[f];
     for (int c = 1; c < mx; ++c) {
 #pragma unroll
       for (int f = 0; f < 5; ++f) {
-        const double v = __shfl_down(racc[f], c, 64);
-        if (c < nch) racc[f] += v;
+        racc[f] = next_lane(racc[f]);
+        if (c < nch) rsum[f] += racc[f];
       }
     }
+#pragma unroll
+    for (int f = 0; f < 5; ++f) racc[f] = rsum[f];
   }
   int v = 0, wcol = 0;
   uint8_t ma = 0, mb = 0;
@@ -1895,7 +2300,8 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
     mb = A.bcm[wcol];
   }
   // bc3LHS and the store of one block: rows masked by mr, columns by mc
-  auto store = [&](long long entry, uint8_t mr, uint8_t mc, bool dg) {
+  auto store = [&](long long entry, uint8_t mr, uint8_t mc) {
+    constexpr bool dg = !kPair;
     double sum[25];
 #pragma unroll
     for (int i = 0; i < 25; ++i) sum[i] = (double)csum[i];
@@ -1929,21 +2335,42 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
   };
   combine(acc);
   if (leader) {
-    if (diag) {
+    if constexpr (!kPair) {
 #pragma unroll
       for (int f = 0; f < 5; ++f) A.res[5 * (size_t)v + f] = racc[f];
     }
-    store(L.y, ma, mb, diag);
+    store(L.y, ma, mb);
   }
-  if (wp) {
+  if constexpr (kPair) {
     combine(acc2);
-    if (leader && pair) store(k2, mb, ma, false);
+    if (leader) store(k2, mb, ma);
   }
+}
+
+template <typename T, typename S, bool kDC, bool kMT>
+__device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.clk = wall_clock64();
+  const long long per = (gridDim.x + 7) / 8;
+  const long long wg = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  const long long l = wg * 64 + threadIdx.x;
+  int4 L = make_int4(0, 0, 0, 0);
+  int k2 = -1;
+  if (l < A.nlanes) {
+    L = A.lanes[l];
+    k2 = A.lanes_k2[l];
+  }
+  // a wavefront holds pairs or diagonal entries, padding lanes (no blocks, no
+  // leader) behind them
+  __shared__ phg_i4 lds[Pipe<T, S>::kPieces];
+  if (__builtin_amdgcn_readfirstlane(k2) >= 0)
+    asm_pairs_wave<T, S, kDC, kMT, true>(A, L, k2, lds);
+  else
+    asm_pairs_wave<T, S, kDC, kMT, false>(A, L, k2, lds);
 }
 
 // Shakib's or Franca's tau without DC, float or double
 template <typename T, typename S>
-__global__ void __launch_bounds__(64) k_asm_pairs(BlkArgs A) {
+__global__ void __launch_bounds__(64, 2) k_asm_pairs(BlkArgs A) {
   asm_pairs<T, S, false, false>(A);
 }
 
@@ -2216,29 +2643,34 @@ __global__ void __launch_bounds__(256) k_mres(MresArgs A) {
   for (int k = 0; k < 4; ++k) nd[k] = A.ien[k * nel + e];
   // the state's point values, thermodynamics and W tau, and the element's
   // shape gradients and WdetJ, as the point pass stored them at this state
-  double rec[12], g16[16];
-  load_pt<double>(A.qps + ((size_t)e * 4 + q) * pt_stride<double>(), rec);
-  load_rec<double>(A.geo + (size_t)e * rec_stride<double>(), g16);
-  const double WdetJ = g16[12];
+  double g16[16];
+  load_vals<double>(A.geo + 16 * (size_t)e, g16, 16);
+  double rec[8];
+  load_vals<double>(pt_at<const double>(A.qps, e, q), rec, 8);
+  const double WdetJ = g16[3];
   double shg[4][3];
 #pragma unroll
   for (int k = 0; k < 4; ++k)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) shg[k][c] = g16[3 * k + c];
+    for (int c = 0; c < 3; ++c) shg[k][c] = g16[4 * k + c];
+  const double cpR = ph.gamma / ph.gamma1;
+  const PtConst<double> pc{ph.Rgas, cpR - 1.0, cpR, ph.temper / (ph.Rgas / ph.gamma1),
+                           ph.itau == 1};
+  const Pt<double> pt = decode_pt<double, double>(rec, pc);
   Thermo t;
-  t.u[0] = rec[0];
-  t.u[1] = rec[1];
-  t.u[2] = rec[2];
-  t.rho = rec[kPtRho];
-  t.drdp = rec[kPtDrdp];
-  t.drdT = rec[kPtDrdT];
-  t.e1p = rec[kPtE1p];
+  t.u[0] = pt.u[0];
+  t.u[1] = pt.u[1];
+  t.u[2] = pt.u[2];
+  t.rho = pt.rho;
+  t.drdp = pt.drdp;
+  t.drdT = pt.drdT;
+  t.e1p = pt.e1p;
   t.e2p = t.e1p + 1.0;
-  t.e3p = rec[kPtE3p];
-  t.e4p = rec[kPtE4p];
-  t.tau[0] = rec[kPtT0] / WdetJ;
-  t.tau[1] = rec[kPtT1] / WdetJ;
-  t.tau[2] = rec[kPtT2] / WdetJ;
+  t.e3p = pt.e3p;
+  t.e4p = pt.e4p;
+  t.tau[0] = pt.t0 / WdetJ;
+  t.tau[1] = pt.t1 / WdetJ;
+  t.tau[2] = pt.t2 / WdetJ;
   double Nq[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) Nq[k] = sel4(cQ.N[0][k], cQ.N[1][k], cQ.N[2][k], cQ.N[3][k], q);
@@ -2576,7 +3008,7 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
   Q.node = c->nodepack;
   Q.qnode = c->qnode;
   Q.qps = mixed ? (void*)c->qps32 : (void*)c->qps;
-  Q.geo = mixed ? (void*)c->geo32 : (void*)c->geo;
+  Q.geo = c->geo;
   Q.resid = c->resid;
   Q.nel = c->nel;
   Q.ph = ph;
@@ -2635,6 +3067,11 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
   B.lam = -(2.0 / 3.0) * ph.mu;
   B.kap = ph.mu * cp / ph.pr;
   B.cfac = ph.almi / ph.gami / ph.alfi * ph.Dtgl;
+  B.Rg = ph.Rgas;
+  B.cpR = ph.gamma / ph.gamma1;
+  B.e1c = B.cpR - 1.0;
+  B.kt2 = ph.temper / (ph.Rgas / ph.gamma1);
+  B.franca = ph.itau == 1 ? 1 : 0;
   B.clk = &c->gm->ta[2];
   const int g2 = (int)(((B.nlanes + 63) / 64 + 7) / 8 * 8);  // whole XCD rounds
   if (paired && mixed && dc && mt)

@@ -538,14 +538,12 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   if (mat) PHG_TRY(dev_alloc(c, &c->lanes_k2, c->nlanes_pair));
   PHG_TRY(dev_alloc(c, &c->lanes_diag, c->nlanes_diag));
   PHG_TRY(dev_alloc(c, &c->blocks, 16 * nel));
-  // point records: 12 values per point; geometry: 13 values padded to 16
-  // floats or 14 doubles (16-byte loads)
+  // point records: 8 doubles, geometry 16; in float 16 values for both
   if (mixed) {
-    PHG_TRY(dev_alloc(c, &c->qps32, (size_t)nel * 4 * 12));
-    PHG_TRY(dev_alloc(c, &c->geo32, (size_t)nel * 16));
+    PHG_TRY(dev_alloc(c, &c->qps32, (size_t)nel * 4 * 16));
   } else {
-    PHG_TRY(dev_alloc(c, &c->qps, (size_t)nel * 4 * 12));
-    PHG_TRY(dev_alloc(c, &c->geo, (size_t)nel * 14));
+    PHG_TRY(dev_alloc(c, &c->qps, (size_t)nel * 4 * 8));
+    PHG_TRY(dev_alloc(c, &c->geo, (size_t)nel * 16));
   }
   // element residuals (element order), then the element products in the
   // incidence slots (k_jv, k_mres)
@@ -1343,7 +1341,7 @@ extern "C" int phg_finalize(phg_ctx* c) {
   mp_free(c);
   void* ptrs[] = {c->x,        c->ienc,     c->lanes,  c->lanes_diag, c->lanes_pair,
                   c->lanes_k2, c->blocks, c->qps, c->qps32, c->geo,
-                  c->geo32,    c->resid,    c->tslot,    c->ienbc,  c->bcm,       c->iper,
+                  c->resid,    c->tslot,    c->ienbc,  c->bcm,       c->iper,
                   c->BCv,      c->fold_master, c->fold_ptr, c->fold_slave, c->grp_slot,
                   c->scol,     c->scolp,    c->csr2slot, c->lhs64, c->lhs32,     c->res,
                   c->rmes,     c->bdiag,    c->bdiag32, c->y,      c->ac,        c->yold,

@@ -250,10 +250,9 @@ struct phg_ctx {
   int* blocks = nullptr;        // e*16 + a*4 + b, grouped per owner lane
   void* scratch = nullptr;      // this device's address of the library's
                                 // static staging array (phg_spsi3pre_noalloc)
-  double* qps = nullptr;        // (nel*4) x 12 point records (FP64 path)
-  float* qps32 = nullptr;       // (nel*4) x 12, mixed path
-  double* geo = nullptr;        // nel x 14: shape gradients, WdetJ (+ pad)
-  float* geo32 = nullptr;       // nel x 16
+  double* qps = nullptr;        // (nel*4) x 8 point records (FP64 path)
+  float* qps32 = nullptr;       // (nel*4) x 16, mixed path: point record and node row
+  double* geo = nullptr;        // nel x 16: per node shape gradient and WdetJ
   double* resid = nullptr;      // (nel*4) x 5 element residual per node (element
                                 // order), then the element products of k_jv and
                                 // k_mres in the incidence slots

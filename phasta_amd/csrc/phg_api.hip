@@ -8,9 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <initializer_list>
 #include <numeric>
-#include <type_traits>
 
 #include "phg_internal.h"
 
@@ -65,79 +63,13 @@ int dev_alloc(phg_ctx* c, T** p, size_t count) {
   return 0;
 }
 
-// ---- host arrays to the device and back ----
-// hipMemcpyAsync on ordinary host memory waits for the copy, 10 to 15 us for
-// each array however small.  So arrays of kStageBytes / 2 together and less go
-// through a pinned buffer: an upload does not wait, a download waits once for
-// all its arrays (a time step of 125 nodes: two arrays in and three out, 341 ->
-// 311 us).  The runtime's staging is as fast from some 400 KB on (4913 nodes:
-// 1.41 ms that way, 1.43 through a pinned ring).
-struct HostArray {
-  char* dev;
-  char* host;
-  size_t bytes;
-  template <typename D, typename H>
-  HostArray(D* d, H* h, size_t count) : dev((char*)d), host((char*)h), bytes(count * sizeof(D)) {
-    static_assert(std::is_same_v<std::remove_const_t<D>, std::remove_const_t<H>>);
-  }
-  size_t place() const { return (bytes + 63) & ~(size_t)63; }
-};
-
-size_t place_of(std::initializer_list<HostArray> list) {
-  size_t n = 0;
-  for (const HostArray& a : list)
-    if (a.host) n += a.place();
-  return n;
-}
-
-int upload(phg_ctx* c, std::initializer_list<HostArray> list) {
-  const size_t n = place_of(list);
-  bool small = n <= kStageBytes / 2;
-  for (const HostArray& a : list) small = small && a.host;  // a missing one is the runtime's error
-  if (small && c->stage_fill + n > kStageBytes) {
-    PHG_HIP(hipStreamSynchronize(c->stream));
-    c->stage_fill = 0;
-  }
-  for (const HostArray& a : list) {
-    if (a.bytes == 0) continue;
-    const char* from = a.host;
-    if (small) {
-      from = c->stage + c->stage_fill;
-      std::memcpy(c->stage + c->stage_fill, a.host, a.bytes);
-      c->stage_fill += a.place();
-    }
-    PHG_HIP(hipMemcpyAsync(a.dev, from, a.bytes, hipMemcpyHostToDevice, c->stream));
-  }
-  return 0;
-}
-
 template <typename T>
 int upload(phg_ctx* c, T* dst, const T* src, size_t count) {
-  return upload(c, {HostArray(dst, src, count)});
-}
-
-// complete when it returns; arrays without a host array are left out
-int download(phg_ctx* c, std::initializer_list<HostArray> list) {
-  const bool small = place_of(list) <= kStageBytes / 2;
-  size_t at = 0;  // (uploads from the buffer end before in the stream)
-  for (const HostArray& a : list) {
-    if (!a.host || a.bytes == 0) continue;
-    PHG_HIP(hipMemcpyAsync(small ? c->stage + at : a.host, a.dev, a.bytes, hipMemcpyDeviceToHost,
-                           c->stream));
-    at += a.place();
-  }
-  PHG_HIP(hipStreamSynchronize(c->stream));
-  c->stage_fill = 0;
-  at = 0;
-  for (const HostArray& a : list) {
-    if (!small || !a.host) continue;
-    std::memcpy(a.host, c->stage + at, a.bytes);
-    at += a.place();
-  }
+  if (count == 0) return 0;
+  PHG_HIP(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
   return 0;
 }
 
-// one array, which has to be there; the caller synchronises
 template <typename T>
 int download(phg_ctx* c, T* dst, const T* src, size_t count) {
   if (count == 0) return 0;
@@ -674,7 +606,6 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_HIP(hipHostMalloc((void**)&c->h_gm, kGmMax * sizeof(GmHost), hipHostMallocCoherent));
   std::fill(c->h_gm, c->h_gm + kGmMax, GmHost{});
   PHG_HIP(hipHostMalloc((void**)&c->h_sol, sizeof(SolveHost), hipHostMallocCoherent));
-  PHG_HIP(hipHostMalloc((void**)&c->stage, kStageBytes, hipHostMallocDefault));
   *c->h_sol = SolveHost{};
   {
     int dev = 0, khz = 0;
@@ -1424,7 +1355,6 @@ extern "C" int phg_finalize(phg_ctx* c) {
   if (c->h_scal) (void)hipHostFree(c->h_scal);
   if (c->h_gm) (void)hipHostFree(c->h_gm);
   if (c->h_sol) (void)hipHostFree(c->h_sol);
-  if (c->stage) (void)hipHostFree(c->stage);
   for (auto ev : c->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto ev : c->kev)
@@ -1477,7 +1407,8 @@ extern "C" int phg_elmgmrs(phg_ctx* c, const double* y, const double* ac, double
                            double* BDiag, double* lhsK) {
   PHG_TRY(check_ctx(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   PHG_TRY(elm_core(c));
   PHG_TRY(download(c, res, c->res, 5 * n));
   if (rmes) std::memset(rmes, 0, sizeof(double) * 5 * n);  // elmgmr.f:400
@@ -1497,10 +1428,13 @@ extern "C" int phg_solgmrs(phg_ctx* c, const double* y, const double* ac, double
   phg_stats local{};
   if (!st) st = &local;
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   PHG_TRY(sol_core(c, st));
-  PHG_TRY(download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
-                       HostArray(c->bdiag, BDiag, 25 * n), HostArray(c->dy, Dy, 5 * n)}));
+  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
+  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
+  if (BDiag) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
+  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * n));
   if (lhsK) {
     PHG_TRY(ensure_tmp(c, sizeof(double) * 25 * c->nnz));
     if (c->precision == PHG_MIXED)
@@ -1514,28 +1448,31 @@ extern "C" int phg_solgmrs(phg_ctx* c, const double* y, const double* ac, double
 
 extern "C" int phg_state_upload(phg_ctx* c, const double* yold, const double* acold) {
   PHG_TRY(check_ctx(c));
-  const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->yold, yold, 5 * n), HostArray(c->acold, acold, 5 * n)}));
+  PHG_TRY(upload(c, c->yold, yold, 5 * c->nshg));
+  PHG_TRY(upload(c, c->acold, acold, 5 * c->nshg));
   return sync(c);
 }
 
 extern "C" int phg_state_download(phg_ctx* c, double* y, double* ac, double* Dy) {
   PHG_TRY(check_ctx(c));
-  const long long n = c->nshg;
-  return download(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n),
-                      HostArray(c->dy, Dy, 5 * n)});
+  if (y) PHG_TRY(download(c, y, c->y, 5 * c->nshg));
+  if (ac) PHG_TRY(download(c, ac, c->ac, 5 * c->nshg));
+  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * c->nshg));
+  return sync(c);
 }
 
 extern "C" int phg_state_upload_cur(phg_ctx* c, const double* y, const double* ac) {
   PHG_TRY(check_ctx(c));
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * c->nshg), HostArray(c->ac, ac, 5 * c->nshg)}));
+  PHG_TRY(upload(c, c->y, y, 5 * c->nshg));
+  PHG_TRY(upload(c, c->ac, ac, 5 * c->nshg));
   return sync(c);
 }
 
 extern "C" int phg_state_download_old(phg_ctx* c, double* yold, double* acold) {
   PHG_TRY(check_ctx(c));
-  const long long n = c->nshg;
-  return download(c, {HostArray(c->yold, yold, 5 * n), HostArray(c->acold, acold, 5 * n)});
+  if (yold) PHG_TRY(download(c, yold, c->yold, 5 * c->nshg));
+  if (acold) PHG_TRY(download(c, acold, c->acold, 5 * c->nshg));
+  return sync(c);
 }
 
 extern "C" int phg_predict(phg_ctx* c) {
@@ -1569,10 +1506,13 @@ extern "C" int phg_elmmfg(phg_ctx* c, const double* y, const double* ac, double*
                           double* BDiag) {
   PHG_TRY(check_ctx(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   PHG_TRY(elm_mfg(c));
-  return download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
-                      HostArray(c->bdiag, c->prm.iprec != 0 ? BDiag : nullptr, 25 * n)});
+  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
+  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
+  if (BDiag && c->prm.iprec != 0) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
+  return sync(c);
 }
 
 extern "C" int phg_itrres(phg_ctx* c, const double* yp, const double* yc, const double* ac,
@@ -1581,7 +1521,8 @@ extern "C" int phg_itrres(phg_ctx* c, const double* yp, const double* yc, const 
   PHG_TRY(mfg_check(c));
   PHG_TRY(mfg_alloc(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, yc, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, yc, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   PHG_TRY(launch_pack_nodes(c));
   // the state's point records (and W PTau with the matrix tau), which the
   // modified residual reads
@@ -1605,7 +1546,8 @@ extern "C" int phg_au1mfg(phg_ctx* c, const double* ypre, const double* y, const
     return PHG_EINVAL;
   }
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   PHG_TRY(launch_pack_nodes(c));
   PHG_TRY(launch_assembly(c, false, false));  // the state's point records
   PHG_TRY(upload(c, c->bdiag, BDiag, 25 * n));
@@ -1627,12 +1569,15 @@ extern "C" int phg_solmfg(phg_ctx* c, const double* y, const double* ac, double*
   phg_stats local{};
   if (!st) st = &local;
   const long long n = c->nshg;
-  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
+  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, c->ac, ac, 5 * n));
   if (eGMRES) c->mfg.eg = *eGMRES;
   PHG_TRY(mfg_core(c, fdi, st));
   if (eGMRES) *eGMRES = c->mfg.eg;
-  PHG_TRY(download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
-                       HostArray(c->bdiag, BDiag, 25 * n), HostArray(c->dy, Dy, 5 * n)}));
+  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
+  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
+  if (BDiag) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
+  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * n));
   return sync(c);
 }
 

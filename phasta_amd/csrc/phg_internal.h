@@ -227,8 +227,6 @@ struct MpNet {
   int ds_cap = 0;
 };
 
-constexpr size_t kStageBytes = 256 << 10;
-
 struct phg_ctx {
   long long nshg = 0, nel = 0, nelb = 0, nnz = 0;
   int ndofBC = 0;
@@ -340,8 +338,6 @@ struct phg_ctx {
   GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
   unsigned gm_seq = 0;             // token of the last iteration enqueued
   SolveHost* h_sol = nullptr;      // pinned
-  char* stage = nullptr;           // pinned, kStageBytes: small host arrays on their way
-  size_t stage_fill = 0;           // bytes of uploads that may still be read
   unsigned sol_seq = 0;            // token of the last solve enqueued
   double clk_ms = 0.0;             // ms per tick of the device clock
   double* scal = nullptr;          // device scalars (H column etc.)

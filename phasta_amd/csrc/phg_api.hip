@@ -8,7 +8,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <numeric>
+#include <type_traits>
 
 #include "phg_internal.h"
 
@@ -63,18 +65,130 @@ int dev_alloc(phg_ctx* c, T** p, size_t count) {
   return 0;
 }
 
-template <typename T>
-int upload(phg_ctx* c, T* dst, const T* src, size_t count) {
-  if (count == 0) return 0;
-  PHG_HIP(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
+// ---- host arrays to the device and back ----
+// hipMemcpyAsync on ordinary host memory waits for the copy, 10 to 15 us for
+// each array however small, and moves large results piece after piece through
+// one buffer.  So results move over the bus into a ring of kStageSlots pinned
+// slots while the calling thread copies from it: three arrays of 85.9 MB into
+// new memory 25.1 -> 19.4 ms (12 of them the first touch), of 11.0 MB 2.4 -> 1.2
+// ms (with arrays that are not zeroed first), of 5.6 MB 1.2 -> 0.63.  Small
+// arrays go up through it too, without a wait: a time step of 125 nodes, two
+// arrays up and three down, 341 -> 309 us; large ones gain nothing (5.9 ms for
+// 172 MB either way).  Copying threads beside the caller's own took the CPU from
+// it: a step of 97336 nodes 3.7 ms with one thread, 9.9 with three more for each
+// transfer, 23.7 with OpenMP's.
+struct HostArray {
+  char* dev;
+  char* host;
+  size_t bytes;
+  template <typename D, typename H>
+  HostArray(D* d, H* h, size_t count) : dev((char*)d), host((char*)h), bytes(count * sizeof(D)) {
+    static_assert(std::is_same_v<std::remove_const_t<D>, std::remove_const_t<H>>);
+  }
+};
+
+struct Cursor {  // a place in a list of arrays
+  const HostArray* a;
+  const HostArray* end;
+  size_t off;
+};
+
+// the next pieces of the list that fill one slot: f(device, host, place in the
+// slot, bytes)
+template <typename F>
+int fill_slot(phg_ctx* c, Cursor& k, F f) {
+  size_t at = 0;
+  while (k.a != k.end && at < c->stage_bytes) {
+    const size_t n = std::min(k.a->bytes - k.off, c->stage_bytes - at);
+    if (k.a->host && n > 0) {
+      PHG_TRY(f(k.a->dev + k.off, k.a->host + k.off, at, n));
+      at += (n + 63) & ~(size_t)63;
+    }
+    k.off += n;
+    if (!k.a->host || k.off == k.a->bytes) k = {k.a + 1, k.end, 0};
+  }
+  return 0;
+}
+
+size_t bytes_of(std::initializer_list<HostArray> list) {
+  size_t n = 0;
+  for (const HostArray& a : list) n += a.host ? a.bytes : 0;
+  return n;
+}
+
+// the arrays may be changed when it returns
+int upload(phg_ctx* c, std::initializer_list<HostArray> list) {
+  bool ring = bytes_of(list) <= kStageSmall;
+  for (const HostArray& a : list) ring = ring && a.host;  // a missing one is the runtime's error
+  if (!ring) {
+    for (const HostArray& a : list)
+      if (a.bytes) PHG_HIP(hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c->stream));
+    return 0;
+  }
+  for (Cursor k{list.begin(), list.end(), 0}; k.a != k.end;) {
+    const int s = c->stage_slot;
+    c->stage_slot = (s + 1) % kStageSlots;
+    char* slot = c->stage + s * c->stage_bytes;
+    PHG_HIP(hipEventSynchronize(c->stage_ev[s]));  // its last use
+    PHG_TRY(fill_slot(c, k, [&](char* dev, char* host, size_t at, size_t n) -> int {
+      std::memcpy(slot + at, host, n);
+      PHG_HIP(hipMemcpyAsync(dev, slot + at, n, hipMemcpyHostToDevice, c->stream));
+      return 0;
+    }));
+    PHG_HIP(hipEventRecord(c->stage_ev[s], c->stream));
+  }
   return 0;
 }
 
 template <typename T>
-int download(phg_ctx* c, T* dst, const T* src, size_t count) {
+int upload(phg_ctx* c, T* dst, const T* src, size_t count) {
+  return count ? upload(c, {HostArray(dst, src, count)}) : 0;
+}
+
+// complete when it returns; arrays without a host array are left out
+int download(phg_ctx* c, std::initializer_list<HostArray> list) {
+  // (a piece costs some 15 us: small slots are for small arrays only)
+  if (c->stage_bytes < kStageMin && bytes_of(list) > kStageSmall) {
+    for (const HostArray& a : list)
+      if (a.host && a.bytes)
+        PHG_HIP(hipMemcpyAsync(a.host, a.dev, a.bytes, hipMemcpyDeviceToHost, c->stream));
+    PHG_HIP(hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  Cursor out{list.begin(), list.end(), 0}, in = out;
+  for (int moved = 0, done = 0; in.a != in.end; ++done) {
+    for (; out.a != out.end && moved - done < kStageSlots; ++moved) {
+      const int s = moved % kStageSlots;
+      PHG_TRY(fill_slot(c, out, [&](char* dev, char*, size_t at, size_t n) -> int {
+        PHG_HIP(hipMemcpyAsync(c->stage + s * c->stage_bytes + at, dev, n, hipMemcpyDeviceToHost,
+                               c->stream));
+        return 0;
+      }));
+      PHG_HIP(hipEventRecord(c->stage_ev[s], c->stream));
+    }
+    const int s = done % kStageSlots;
+    PHG_HIP(hipEventSynchronize(c->stage_ev[s]));
+    PHG_TRY(fill_slot(c, in, [&](char*, char* host, size_t at, size_t n) -> int {
+      std::memcpy(host, c->stage + s * c->stage_bytes + at, n);
+      return 0;
+    }));
+  }
+  return 0;
+}
+
+// ... into pinned memory; the caller synchronises
+template <typename T>
+int download_pinned(phg_ctx* c, T* dst, const T* src, size_t count) {
   if (count == 0) return 0;
   PHG_HIP(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyDeviceToHost, c->stream));
   return 0;
+}
+
+// one array, which has to be there
+template <typename T>
+int download(phg_ctx* c, T* dst, const T* src, size_t count) {
+  if (!dst) return download_pinned(c, dst, src, count);  // the runtime's error
+  return download(c, {HostArray(const_cast<T*>(src), dst, count)});
 }
 
 int sync(phg_ctx* c) {
@@ -606,6 +720,12 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_HIP(hipHostMalloc((void**)&c->h_gm, kGmMax * sizeof(GmHost), hipHostMallocCoherent));
   std::fill(c->h_gm, c->h_gm + kGmMax, GmHost{});
   PHG_HIP(hipHostMalloc((void**)&c->h_sol, sizeof(SolveHost), hipHostMallocCoherent));
+  // slots of a fourth of a node array up to 2 MB (pinning takes 0.9 ms per MB),
+  // small ones where that is less than kStageMin
+  c->stage_bytes = std::min<size_t>((size_t)(10 * nshg) & ~(size_t)4095, 2 << 20);
+  if (c->stage_bytes < kStageMin) c->stage_bytes = 64 << 10;
+  PHG_HIP(hipHostMalloc((void**)&c->stage, kStageSlots * c->stage_bytes, hipHostMallocDefault));
+  for (auto& e : c->stage_ev) PHG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   *c->h_sol = SolveHost{};
   {
     int dev = 0, khz = 0;
@@ -776,7 +896,7 @@ int mfg_au2(phg_ctx* c, double* out) {
   const long long V = 5 * c->nshg;
   double* S = c->scal + 200;
   PHG_TRY(launch_dot(c, c->dy, c->dy, V, S));
-  PHG_TRY(download(c, c->h_scal + 200, S, 1));
+  PHG_TRY(download_pinned(c, c->h_scal + 200, S, 1));
   PHG_TRY(sync(c));
   const double eps = std::pow(c->prm.epsM, 0.6666666666666666666666666666667) /
                      std::sqrt(c->h_scal[200]);
@@ -809,7 +929,7 @@ int mfg_fdi(phg_ctx* c, const double* u, double* eg) {
   PHG_TRY(launch_i3lu(c, c->bdiag, c->mfg.t1, 1));
   PHG_TRY(launch_mfg_combine(c, c->rmes, c->mfg.t1, nullptr, epsM, c->mfg.t2, 1));
   PHG_TRY(launch_dot(c, c->mfg.t2, c->mfg.t2, V, S + 1));
-  PHG_TRY(download(c, c->h_scal + 200, S, 2));
+  PHG_TRY(download_pinned(c, c->h_scal + 200, S, 2));
   PHG_TRY(sync(c));
   const double epsA = (epsM * epsM) * std::sqrt(c->h_scal[200]);
   const double SDnrm = std::sqrt(c->h_scal[201]);
@@ -975,7 +1095,7 @@ int gmres_cycle(phg_ctx* c, double unorm, double epsnrm, double n0, phg_stats* s
     double loss = 0.0;
     for (int i = 0; i <= iKs; ++i) {
       for (int j = 0; j <= i; ++j) PHG_TRY(launch_dot(c, kvec(c, i), kvec(c, j), V, d + j));
-      PHG_TRY(download(c, c->h_scal + 128, d, i + 1));
+      PHG_TRY(download_pinned(c, c->h_scal + 128, d, i + 1));
       PHG_TRY(sync(c));
       for (int j = 0; j <= i; ++j)
         loss = std::max(loss, std::fabs(c->h_scal[128 + j] - (i == j ? 1.0 : 0.0)));
@@ -1006,7 +1126,7 @@ int mfg_core(phg_ctx* c, int fdi, phg_stats* st) {
   // ypre = U new2old(y) (solmfg.f:124-133)
   PHG_TRY(launch_yshuffle(c, c->y, c->mfg.ypre, true));
   PHG_TRY(launch_i3lu(c, c->bdiag, c->mfg.ypre, 3));
-  PHG_TRY(download(c, c->h_scal, S, 8));
+  PHG_TRY(download_pinned(c, c->h_scal, S, 8));
   PHG_TRY(sync(c));
   const double sumsq = c->h_scal[0], sumsq_m = c->h_scal[4];
   double unorm = c->h_scal[3];
@@ -1036,7 +1156,7 @@ int mfg_core(phg_ctx* c, int fdi, phg_stats* st) {
         rc = mfg_au2(c, kvec(c, 1));
         if (!rc) rc = launch_dot(c, kvec(c, 1), kvec(c, 1), V, S + 5);
         if (!rc) rc = launch_scale(c, kvec(c, 0), kvec(c, 1), V, S + 5, S + 6);
-        if (!rc) rc = download(c, c->h_scal + 6, S + 6, 1);
+        if (!rc) rc = download_pinned(c, c->h_scal + 6, S + 6, 1);
         if (!rc) rc = sync(c);
         if (rc) break;
         unorm = c->h_scal[6];
@@ -1171,7 +1291,7 @@ int sol_core(phg_ctx* c, phg_stats* st, bool correct = false) {
       }
       PHG_TRY(launch_dot(c, kvec(c, 2), kvec(c, 2), V, S + 5));
       PHG_TRY(launch_scale(c, kvec(c, 0), kvec(c, 2), V, S + 5, S + 6));
-      PHG_TRY(download(c, c->h_scal + 5, S + 5, 2));
+      PHG_TRY(download_pinned(c, c->h_scal + 5, S + 5, 2));
       PHG_TRY(sync(c));
       *norm = c->h_scal[6];
       n0 = 1.0;
@@ -1355,6 +1475,9 @@ extern "C" int phg_finalize(phg_ctx* c) {
   if (c->h_scal) (void)hipHostFree(c->h_scal);
   if (c->h_gm) (void)hipHostFree(c->h_gm);
   if (c->h_sol) (void)hipHostFree(c->h_sol);
+  if (c->stage) (void)hipHostFree(c->stage);
+  for (auto ev : c->stage_ev)
+    if (ev) (void)hipEventDestroy(ev);
   for (auto ev : c->ev)
     if (ev) (void)hipEventDestroy(ev);
   for (auto ev : c->kev)
@@ -1407,8 +1530,7 @@ extern "C" int phg_elmgmrs(phg_ctx* c, const double* y, const double* ac, double
                            double* BDiag, double* lhsK) {
   PHG_TRY(check_ctx(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   PHG_TRY(elm_core(c));
   PHG_TRY(download(c, res, c->res, 5 * n));
   if (rmes) std::memset(rmes, 0, sizeof(double) * 5 * n);  // elmgmr.f:400
@@ -1428,13 +1550,10 @@ extern "C" int phg_solgmrs(phg_ctx* c, const double* y, const double* ac, double
   phg_stats local{};
   if (!st) st = &local;
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   PHG_TRY(sol_core(c, st));
-  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
-  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
-  if (BDiag) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
-  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * n));
+  PHG_TRY(download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
+                       HostArray(c->bdiag, BDiag, 25 * n), HostArray(c->dy, Dy, 5 * n)}));
   if (lhsK) {
     PHG_TRY(ensure_tmp(c, sizeof(double) * 25 * c->nnz));
     if (c->precision == PHG_MIXED)
@@ -1448,31 +1567,28 @@ extern "C" int phg_solgmrs(phg_ctx* c, const double* y, const double* ac, double
 
 extern "C" int phg_state_upload(phg_ctx* c, const double* yold, const double* acold) {
   PHG_TRY(check_ctx(c));
-  PHG_TRY(upload(c, c->yold, yold, 5 * c->nshg));
-  PHG_TRY(upload(c, c->acold, acold, 5 * c->nshg));
+  const long long n = c->nshg;
+  PHG_TRY(upload(c, {HostArray(c->yold, yold, 5 * n), HostArray(c->acold, acold, 5 * n)}));
   return sync(c);
 }
 
 extern "C" int phg_state_download(phg_ctx* c, double* y, double* ac, double* Dy) {
   PHG_TRY(check_ctx(c));
-  if (y) PHG_TRY(download(c, y, c->y, 5 * c->nshg));
-  if (ac) PHG_TRY(download(c, ac, c->ac, 5 * c->nshg));
-  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * c->nshg));
-  return sync(c);
+  const long long n = c->nshg;
+  return download(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n),
+                      HostArray(c->dy, Dy, 5 * n)});
 }
 
 extern "C" int phg_state_upload_cur(phg_ctx* c, const double* y, const double* ac) {
   PHG_TRY(check_ctx(c));
-  PHG_TRY(upload(c, c->y, y, 5 * c->nshg));
-  PHG_TRY(upload(c, c->ac, ac, 5 * c->nshg));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * c->nshg), HostArray(c->ac, ac, 5 * c->nshg)}));
   return sync(c);
 }
 
 extern "C" int phg_state_download_old(phg_ctx* c, double* yold, double* acold) {
   PHG_TRY(check_ctx(c));
-  if (yold) PHG_TRY(download(c, yold, c->yold, 5 * c->nshg));
-  if (acold) PHG_TRY(download(c, acold, c->acold, 5 * c->nshg));
-  return sync(c);
+  const long long n = c->nshg;
+  return download(c, {HostArray(c->yold, yold, 5 * n), HostArray(c->acold, acold, 5 * n)});
 }
 
 extern "C" int phg_predict(phg_ctx* c) {
@@ -1506,13 +1622,10 @@ extern "C" int phg_elmmfg(phg_ctx* c, const double* y, const double* ac, double*
                           double* BDiag) {
   PHG_TRY(check_ctx(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   PHG_TRY(elm_mfg(c));
-  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
-  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
-  if (BDiag && c->prm.iprec != 0) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
-  return sync(c);
+  return download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
+                      HostArray(c->bdiag, c->prm.iprec != 0 ? BDiag : nullptr, 25 * n)});
 }
 
 extern "C" int phg_itrres(phg_ctx* c, const double* yp, const double* yc, const double* ac,
@@ -1521,8 +1634,7 @@ extern "C" int phg_itrres(phg_ctx* c, const double* yp, const double* yc, const 
   PHG_TRY(mfg_check(c));
   PHG_TRY(mfg_alloc(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, yc, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, yc, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   PHG_TRY(launch_pack_nodes(c));
   // the state's point records (and W PTau with the matrix tau), which the
   // modified residual reads
@@ -1546,8 +1658,7 @@ extern "C" int phg_au1mfg(phg_ctx* c, const double* ypre, const double* y, const
     return PHG_EINVAL;
   }
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   PHG_TRY(launch_pack_nodes(c));
   PHG_TRY(launch_assembly(c, false, false));  // the state's point records
   PHG_TRY(upload(c, c->bdiag, BDiag, 25 * n));
@@ -1569,15 +1680,12 @@ extern "C" int phg_solmfg(phg_ctx* c, const double* y, const double* ac, double*
   phg_stats local{};
   if (!st) st = &local;
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
-  PHG_TRY(upload(c, c->ac, ac, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(c->ac, ac, 5 * n)}));
   if (eGMRES) c->mfg.eg = *eGMRES;
   PHG_TRY(mfg_core(c, fdi, st));
   if (eGMRES) *eGMRES = c->mfg.eg;
-  if (res) PHG_TRY(download(c, res, c->res, 5 * n));
-  if (rmes) PHG_TRY(download(c, rmes, c->rmes, 5 * n));
-  if (BDiag) PHG_TRY(download(c, BDiag, c->bdiag, 25 * n));
-  if (Dy) PHG_TRY(download(c, Dy, c->dy, 5 * n));
+  PHG_TRY(download(c, {HostArray(c->res, res, 5 * n), HostArray(c->rmes, rmes, 5 * n),
+                       HostArray(c->bdiag, BDiag, 25 * n), HostArray(c->dy, Dy, 5 * n)}));
   return sync(c);
 }
 

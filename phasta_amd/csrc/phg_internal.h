@@ -227,6 +227,9 @@ struct MpNet {
   int ds_cap = 0;
 };
 
+constexpr int kStageSlots = 4;
+constexpr size_t kStageMin = 256 << 10, kStageSmall = 128 << 10;
+
 struct phg_ctx {
   long long nshg = 0, nel = 0, nelb = 0, nnz = 0;
   int ndofBC = 0;
@@ -338,6 +341,10 @@ struct phg_ctx {
   GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
   unsigned gm_seq = 0;             // token of the last iteration enqueued
   SolveHost* h_sol = nullptr;      // pinned
+  char* stage = nullptr;           // pinned ring: host arrays on their way
+  size_t stage_bytes = 0;          // of a slot
+  hipEvent_t stage_ev[kStageSlots] = {};  // the end of a slot's last use
+  int stage_slot = 0;              // the next upload's
   unsigned sol_seq = 0;            // token of the last solve enqueued
   double clk_ms = 0.0;             // ms per tick of the device clock
   double* scal = nullptr;          // device scalars (H column etc.)

@@ -169,12 +169,17 @@ class GpuSolver:
         return dict(ncolors=nc.value, ncolors_b=nb.value, dev_bytes=by.value)
 
     # ---- reference-shaped entry points (host arrays) ----
+    # (arrays that a call fills completely are not zeroed first)
+    def _bdiag(self):
+        """For a call that leaves BDiag alone with iprec = 0."""
+        make = np.empty if self._prm.iprec != 0 else np.zeros
+        return make((self.case.nshg, 5, 5), order="F")
+
     def elmgmrs(self, y, ac, want_lhs=True):
         n, nnz = self.case.nshg, self.case.nnz_tot
         y, ac = _f64(y, (n, 5)), _f64(ac, (n, 5))
-        res = np.zeros((n, 5), order="F")
-        rmes = np.zeros((n, 5), order="F")
-        bd = np.zeros((n, 5, 5), order="F")
+        res, rmes = (np.empty((n, 5), order="F") for _ in range(2))
+        bd = self._bdiag()
         lk = np.zeros((25, nnz), order="F") if want_lhs else None
         _check(lib().phg_elmgmrs(self.h, _p(y), _p(ac), _p(res), _p(rmes), _p(bd), _p(lk)))
         return res, rmes, bd, lk
@@ -187,10 +192,8 @@ class GpuSolver:
             self.set_params(iter=int(iter))
         n, nnz = self.case.nshg, self.case.nnz_tot
         y, ac = _f64(y, (n, 5)), _f64(ac, (n, 5))
-        res = np.zeros((n, 5), order="F")
-        rmes = np.zeros((n, 5), order="F")
-        bd = np.zeros((n, 5, 5), order="F")
-        dy = np.zeros((n, 5), order="F")
+        res, rmes, dy = (np.empty((n, 5), order="F") for _ in range(3))
+        bd = np.empty((n, 5, 5), order="F")
         lk = np.zeros((25, nnz), order="F") if want_lhs else None
         st = PhgStats()
         _check(lib().phg_solgmrs(self.h, _p(y), _p(ac), _p(res), _p(rmes), _p(bd), _p(lk),
@@ -204,9 +207,8 @@ class GpuSolver:
         """ElmMFG: (res, rmes, BDiag); BDiag only with iprec != 0."""
         n = self.case.nshg
         y, ac = _f64(y, (n, 5)), _f64(ac, (n, 5))
-        res = np.zeros((n, 5), order="F")
-        rmes = np.zeros((n, 5), order="F")
-        bd = np.zeros((n, 5, 5), order="F")
+        res, rmes = (np.empty((n, 5), order="F") for _ in range(2))
+        bd = self._bdiag()
         _check(lib().phg_elmmfg(self.h, _p(y), _p(ac), _p(res), _p(rmes), _p(bd)))
         return res, rmes, bd
 
@@ -233,10 +235,8 @@ class GpuSolver:
         BDiag, Dy and the interval eGMRES."""
         n = self.case.nshg
         y, ac = _f64(y, (n, 5)), _f64(ac, (n, 5))
-        res = np.zeros((n, 5), order="F")
-        rmes = np.zeros((n, 5), order="F")
-        bd = np.zeros((n, 5, 5), order="F")
-        dy = np.zeros((n, 5), order="F")
+        res, rmes, dy = (np.empty((n, 5), order="F") for _ in range(3))
+        bd = np.empty((n, 5, 5), order="F")
         eg = ctypes.c_double(egmres)
         st = PhgStats()
         _check(lib().phg_solmfg(self.h, _p(y), _p(ac), _p(res), _p(rmes), _p(bd), _p(dy),
@@ -336,9 +336,7 @@ class GpuSolver:
 
     def download_state(self):
         n = self.case.nshg
-        y = np.zeros((n, 5), order="F")
-        ac = np.zeros((n, 5), order="F")
-        dy = np.zeros((n, 5), order="F")
+        y, ac, dy = (np.empty((n, 5), order="F") for _ in range(3))
         _check(lib().phg_state_download(self.h, _p(y), _p(ac), _p(dy)))
         return y, ac, dy
 

@@ -201,6 +201,43 @@ typedef int phg_i4 __attribute__((ext_vector_type(4)));
 // two doubles at an 8-byte boundary
 typedef double phg_d2u __attribute__((ext_vector_type(2), aligned(8)));
 
+// five values of a lane in three stores (a store's lanes that go to different
+// lines cost the addresser a cycle each)
+__device__ __forceinline__ void store5(double* o, const double v[5]) {
+  phg_d2u a, b;
+  a.x = v[0];
+  a.y = v[1];
+  b.x = v[2];
+  b.y = v[3];
+  *reinterpret_cast<phg_d2u*>(o) = a;
+  *reinterpret_cast<phg_d2u*>(o + 2) = b;
+  o[4] = v[4];
+}
+
+// The sum over a quad's lanes of r_q[a] for node a = q, without the LDS pipe
+// that a shuffle takes: each lane gives its neighbour the two nodes that are the
+// neighbour's and then, two lanes on, one.  (r_q + r_q^1) + (r_q^2 + r_q^3), the
+// association of two butterfly steps.  (The exchanges come before the
+// selections: a lane's value is sent whatever the receiver takes.)
+template <int kCtrl>
+__device__ __forceinline__ double quad_dpp(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, kCtrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E;  // quad_perm 1,0,3,2 and 2,3,0,1
+__device__ __forceinline__ double quad_sum(double v) {
+  v += quad_dpp<kXor1>(v);
+  return v + quad_dpp<kXor2>(v);
+}
+__device__ __forceinline__ double quad_sum_of(const double r[4], int q) {
+  const bool odd = q & 1, up = q & 2;
+  const double s0 = quad_dpp<kXor1>(odd ? r[0] : r[1]), s1 = quad_dpp<kXor1>(odd ? r[2] : r[3]);
+  const double k0 = (odd ? r[1] : r[0]) + s0, k1 = (odd ? r[3] : r[2]) + s1;
+  const double s2 = quad_dpp<kXor2>(up ? k0 : k1);
+  return (up ? k1 : k0) + s2;
+}
 // the next lane's value (zero in lane 63)
 template <typename T>
 __device__ __forceinline__ T next_lane(T v) {
@@ -1038,6 +1075,10 @@ __device__ __forceinline__ void wall_element(const QpArgs& A, long long p) {
 // the diffusive flux and the point's factor is kept for the tangent pass.
 // kMT: the matrix tau of e3tau_nd (itau = 10) replaces Shakib's diagonal
 // tau; W PTau is kept for the tangent pass.
+// Bound by latency at two wavefronts per SIMD (vector ALU 45 % busy, 40 % of the
+// time its bytes at the copy rate): at 128^3 2.95 -> 2.65 ms with float records,
+// 4.01 -> 2.88 with double ones (shorter, and the quad's sums without shuffles);
+// three wavefronts per SIMD, with 12 words spilled, took 3.13 and 3.21.
 template <typename S, bool kDiff, bool kDC, bool kMT>
 __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   if ((int)blockIdx.x >= A.qp_groups) {
@@ -1196,9 +1237,7 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       double dq = s0 * qq[m] + s1 * qq[4 + m] + s2 * qq[8 + m];
-      dq += __shfl_xor(dq, 1, 64);
-      dq += __shfl_xor(dq, 2, 64);
-      L[1 + m] -= dq;
+      L[1 + m] -= quad_sum(dq);
     }
   }
   double DC = 0.0, gu[6], A0g[3][5];
@@ -1281,21 +1320,16 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   // lanes (q = 0..3); lane q keeps node a = q
   double mine[5];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    double r5[5];
+  for (int f = 0; f < 5; ++f) {
+    double r[4];
 #pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      r5[f] = WdetJ * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f]) +
-              Nq[a] * WdetJ * m0[f];
-      r5[f] += __shfl_xor(r5[f], 1, 64);
-      r5[f] += __shfl_xor(r5[f], 2, 64);
-      if (a == q) mine[f] = r5[f];
-    }
+    for (int a = 0; a < 4; ++a)
+      r[a] = WdetJ * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f]) +
+             Nq[a] * WdetJ * m0[f];
+    mine[f] = quad_sum_of(r, q);
   }
   if (valid) {
-    double* ro = A.resid + ((size_t)e * 4 + q) * 5;
-#pragma unroll
-    for (int f = 0; f < 5; ++f) ro[f] = mine[f];
+    store5(A.resid + ((size_t)e * 4 + q) * 5, mine);
   }
 }
 
@@ -1311,20 +1345,24 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
 // The point states are recomputed in double from the node lines, so the
 // product is the FP64 tangent whatever precision the stored matrix has.
 // bc3LHS: v's constrained components at an element node are not seen (zero
-// columns) and constrained rows are zeroed here; k_jv_nodes puts the unit
+// columns) and constrained rows are zeroed here; k_product_nodes puts the unit
 // diagonals of the constrained rows back.  v is read at the periodic master
-// of each node (the p(iper) gather of sparseap.f:33-35).
+// of each node (the p(iper) gather of sparseap.f:33-35).  k_product_in has done
+// both per node, so that a node's direction is one 64-byte line here, like its
+// state, and not five values behind two more loads.  At 128^3 (12.6 M elements)
+// 3.61 -> 2.46 ms with that, the quad's sums without shuffles and three stores
+// for five; the vector ALU's instructions alone take 1.6.  Two wavefronts per
+// SIMD: for three the compiler spills 15 words, 2.80 ms.
 struct JvArgs {
   const int* ien;          // 4 planes of nel
   const double* node;      // 16 per node: y (local order), ac, x
-  const double* v;         // 5 planes, local order
-  const int* iper;         // 0-based master
+  const double* v;         // 8 per node: the direction as the element sees it
   const uint8_t* bcm;
   double* out;             // element e's product at its node a, 5 doubles at
                            // slot eslot[4 e + a] of the node incidence layout
   const int* eslot;
   const double* dcw;       // nel*4 DC factor per point of the last assembly (kDC)
-  long long nel, nshg;
+  long long nel;
   PhysParams ph;
   double cfac;             // almi/(gami alfi) Dtgl
   double epsM;             // /precis/ epsM (kMT)
@@ -1334,13 +1372,14 @@ struct JvArgs {
 // DC sum_j giju(i,j) A0 v_,j, with the point's factor of the last assembly.
 // kMT: the matrix tau of the point (itau = 10) in place of the diagonal one.
 template <bool kDC, bool kMT>
-__global__ void __launch_bounds__(256) k_jv(JvArgs A) {
+__global__ void __launch_bounds__(256, 2) k_jv(JvArgs A) {
   const long long e_raw = blockIdx.x * 64LL + threadIdx.x / 4;
   const int q = threadIdx.x & 3;
   const bool valid = e_raw < A.nel;
   const long long e = valid ? e_raw : A.nel - 1;
-  const long long nel = A.nel, nshg = A.nshg;
+  const long long nel = A.nel;
   const PhysParams& ph = A.ph;
+  const int to = A.eslot[e * 4 + q];  // (asked for here: its wait would come last)
   int nd[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nd[k] = A.ien[k * nel + e];
@@ -1379,15 +1418,15 @@ __global__ void __launch_bounds__(256) k_jv(JvArgs A) {
   for (int f = 0; f < 5; ++f) Y[f] = vq[f] = gv[0][f] = gv[1][f] = gv[2][f] = 0.0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const long long m = A.iper[nd[k]];
-    const uint8_t cm = A.bcm[nd[k]];
+    const double2* vp = reinterpret_cast<const double2*>(A.v + 8 * (size_t)nd[k]);
+    const double2 v01 = vp[0], v23 = vp[1], v4 = vp[2];
+    const double vv[5] = {v01.x, v01.y, v23.x, v23.y, v4.x};
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
       Y[f] += Nq[k] * yl[k][f];
-      const double vv = ((cm >> f) & 1) ? 0.0 : A.v[m + f * nshg];
-      vq[f] += Nq[k] * vv;
+      vq[f] += Nq[k] * vv[f];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) gv[i][f] += shg[k][i] * vv;
+      for (int i = 0; i < 3; ++i) gv[i][f] += shg[k][i] * vv[f];
     }
   }
   Thermo t;
@@ -1464,62 +1503,21 @@ __global__ void __launch_bounds__(256) k_jv(JvArgs A) {
   }
   double mine[5];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int f = 0; f < 5; ++f) {
+    double r[4];
 #pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      double r = W * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f]) +
-                 Nq[a] * W * L[f];
-      r += __shfl_xor(r, 1, 64);
-      r += __shfl_xor(r, 2, 64);
-      if (a == q) mine[f] = r;
-    }
+    for (int a = 0; a < 4; ++a)
+      r[a] = W * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f]) +
+             Nq[a] * W * L[f];
+    mine[f] = quad_sum_of(r, q);
   }
   if (valid) {
     const int nq = sel4i(nd[0], nd[1], nd[2], nd[3], q);
     const uint8_t rm = A.bcm[nq];
-    double* o = A.out + (size_t)A.eslot[e * 4 + q] * 5;
 #pragma unroll
-    for (int f = 0; f < 5; ++f) o[f] = ((rm >> f) & 1) ? 0.0 : mine[f];
+    for (int f = 0; f < 5; ++f) mine[f] = ((rm >> f) & 1) ? 0.0 : mine[f];
+    store5(A.out + (size_t)to * 5, mine);
   }
-}
-
-// w_n = sum of the node's element products in element order (the node's
-// incidence list, sliced by 64-node groups; k_jv writes each product to its
-// slot there, so a wavefront reads whole rows); a constrained dof f of node n
-// takes the unit diagonals of its element blocks, cnt(n) v(iper(n))_f
-// (bc3lhs.f:55-235: one per element containing the node).
-__global__ void __launch_bounds__(256) k_jv_nodes(const long long* __restrict__ goff,
-                                                  const int* __restrict__ inc,
-                                                  const double* __restrict__ out,
-                                                  const double* __restrict__ v,
-                                                  const int* __restrict__ iper,
-                                                  const uint8_t* __restrict__ bcm,
-                                                  double* __restrict__ w, long long nshg) {
-  const long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (n >= nshg) return;
-  const long long g = n >> 6;
-  const int lane = (int)(n & 63);
-  const long long o0 = goff[g];
-  const int deg = (int)((goff[g + 1] - o0) >> 6);
-  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  int cnt = 0;
-  for (int j = 0; j < deg; ++j) {
-    const long long slot = o0 + 64LL * j + lane;
-    if (inc[slot] < 0) continue;
-    ++cnt;
-    const double* r = out + slot * 5;
-#pragma unroll
-    for (int f = 0; f < 5; ++f) acc[f] += r[f];
-  }
-  const uint8_t m = bcm[n];
-  if (m) {
-    const long long mm = iper[n];
-#pragma unroll
-    for (int f = 0; f < 5; ++f)
-      if ((m >> f) & 1) acc[f] = (double)cnt * v[mm + f * nshg];
-  }
-#pragma unroll
-  for (int f = 0; f < 5; ++f) w[n + f * nshg] = acc[f];
 }
 
 // ---------------- pass 2: block owners ----------------
@@ -2638,6 +2636,7 @@ __global__ void __launch_bounds__(256) k_mres(MresArgs A) {
   const long long e = valid ? e_raw : A.nel - 1;  // idle lanes load a valid element
   const long long nel = A.nel;
   const PhysParams& ph = A.ph;
+  const int to = A.eslot[e * 4 + q];
   int nd[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nd[k] = A.ien[k * nel + e];
@@ -2748,21 +2747,18 @@ __global__ void __launch_bounds__(256) k_mres(MresArgs A) {
   }
   double mine[5];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    double r5[5];
+  for (int f = 0; f < 5; ++f) {
+    double r[4];
 #pragma unroll
-    for (int f = 0; f < 5; ++f) {
-      r5[f] = WdetJ * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f] +
-                       Nq[a] * M[f]);
-      r5[f] += __shfl_xor(r5[f], 1, 64);
-      r5[f] += __shfl_xor(r5[f], 2, 64);
-      if (a == q) mine[f] = r5[f];
-    }
+    for (int a = 0; a < 4; ++a)
+      r[a] = WdetJ * (shg[a][0] * F[0][f] + shg[a][1] * F[1][f] + shg[a][2] * F[2][f] +
+                      Nq[a] * M[f]);
+    mine[f] = quad_sum_of(r, q);
   }
   if (valid) {
-    double* ro = A.resid + (size_t)A.eslot[e * 4 + q] * 5;
 #pragma unroll
-    for (int f = 0; f < 5; ++f) ro[f] = A.iabs ? fabs(mine[f]) : mine[f];
+    for (int f = 0; f < 5; ++f) mine[f] = A.iabs ? fabs(mine[f]) : mine[f];
+    store5(A.resid + (size_t)to * 5, mine);
   }
 }
 
@@ -3106,21 +3102,19 @@ int launch_assembly(phg_ctx* c, bool lhs, bool prec) {
   return 0;
 }
 
-int launch_jv(phg_ctx* c, const double* v, double* w) {
+int launch_jv(phg_ctx* c) {
   PHG_TRY(upload_quadrature());
   const PhysParams ph = phys_of(c->prm);
   JvArgs J{};
   J.ien = c->ienc;
   J.node = c->nodepack;
-  J.v = v;
-  J.iper = c->iper;
+  J.v = c->vpack;
   J.bcm = c->bcm;
   J.out = c->resid;
   J.eslot = c->eslot;
   J.dcw = c->dcw;
   J.epsM = c->prm.epsM;
   J.nel = c->nel;
-  J.nshg = c->nshg;
   J.ph = ph;
   J.cfac = ph.almi / ph.gami / ph.alfi * ph.Dtgl;
   const int gj = (int)((c->nel + 63) / 64);
@@ -3140,11 +3134,7 @@ int launch_jv(phg_ctx* c, const double* v, double* w) {
     k_jv<false, false><<<gj, 256, 0, c->stream>>>(J);
   }
   PHG_HIP(hipGetLastError());
-  const long long n = c->nshg;
-  k_jv_nodes<<<(int)((n + 255) / 256), 256, 0, c->stream>>>(c->inc_goff, c->inc, c->resid, v,
-                                                            c->iper, c->bcm, w, n);
-  PHG_HIP(hipGetLastError());
-  return launch_bc3per(c, w, 5);
+  return 0;
 }
 
 // The modified residual of the variables yp (stride 8, packed by

@@ -1085,6 +1085,201 @@ __global__ void __launch_bounds__(kNodeThreads) k_nodes(NodeArgs A) {
   }
 }
 
+// ---------------- the FP64 tangent's product around its element kernel ----------------
+// k_product_in: per node the direction as the elements read it, v at the
+// periodic master with the constrained components zero.  kLu: v = U^-1 src of
+// the master (the refinement's U^-1 dy), also stored in planes for
+// k_product_nodes.
+template <bool kLu>
+__global__ void __launch_bounds__(256) k_product_in(const double* __restrict__ src,
+                                                    const double* __restrict__ D,
+                                                    const int* __restrict__ iper,
+                                                    const uint8_t* __restrict__ bcm,
+                                                    double* __restrict__ vp,
+                                                    double* __restrict__ v, long long n) {
+  const long long k = blockIdx.x * 256LL + threadIdx.x;
+  if (k >= n) return;
+  const long long m = iper[k];
+  const uint8_t c = bcm[k];
+  double r[5];
+#pragma unroll
+  for (int f = 0; f < 5; ++f) r[f] = src[m + f * n];
+  if constexpr (kLu) {
+    double d[5][5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j)
+#pragma unroll
+      for (int i = 0; i <= j; ++i) d[i][j] = D[(i + 5 * j) * n + m];
+#pragma unroll
+    for (int i = 4; i >= 0; --i) {
+      double s = r[i];
+#pragma unroll
+      for (int q = 4; q > i; --q) s -= r[q] * d[i][q];
+      r[i] = d[i][i] * s;
+    }
+#pragma unroll
+    for (int f = 0; f < 5; ++f) v[k + f * n] = r[f];
+  }
+  double2* o = reinterpret_cast<double2*>(vp + 8 * k);
+#pragma unroll
+  for (int f = 0; f < 5; ++f) r[f] = (c >> f) & 1 ? 0.0 : r[f];
+  o[0] = make_double2(r[0], r[1]);
+  o[1] = make_double2(r[2], r[3]);
+  o[2] = make_double2(r[4], 0.0);
+}
+
+struct ProductArgs {
+  const long long* goff;   // the node incidence layout, 64-node groups
+  const int* inc;
+  const double* out;       // element products at their slots there
+  const double* v;         // direction, 5 planes
+  const int* iper;
+  const uint8_t* bcm;
+  const int2* info;        // boundary group, family (-1 without)
+  const int* sptr;
+  const int* smem;
+  int nmem;                // members, 0: no sums apart
+  double* msum;            // 8 per member: the slaves' sums
+  double* w;               // the product (without kResid)
+  const double* rmes;
+  const double* bdiag;
+  double* start;
+  long long n;
+  double* part;            // kNodeBlocks partials
+  GmDev* gm;
+  SolveHost* host;
+  unsigned seq;
+};
+
+// values f0 .. f0 + kF - 1 of the node's sum of element products in element
+// order; a constrained value f is the unit diagonals of its element blocks,
+// cnt(k) v(iper(k))_f (bc3lhs.f:55-235: one per element containing the node)
+template <int kF>
+__device__ __forceinline__ void node_product(const ProductArgs& A, long long k, int f0,
+                                             double acc[kF]) {
+  const long long o0 = A.goff[k >> 6];
+  const int deg = (int)((A.goff[(k >> 6) + 1] - o0) >> 6);
+  const uint8_t m = A.bcm[k];
+  int cnt = 0;
+#pragma unroll
+  for (int f = 0; f < kF; ++f) acc[f] = 0.0;
+  long long slot = o0 + (k & 63);
+#pragma unroll 4
+  for (int j = 0; j < deg; ++j, slot += 64) {
+    const bool on = A.inc[slot] >= 0;
+    cnt += on;
+#pragma unroll
+    for (int f = 0; f < kF; ++f) {
+      const double r = A.out[slot * 5 + f0 + f];
+      acc[f] += on ? r : 0.0;
+    }
+  }
+  if (m) {
+    const long long mm = A.iper[k];
+#pragma unroll
+    for (int f = 0; f < kF; ++f)
+      if ((m >> (f0 + f)) & 1) acc[f] = (double)cnt * A.v[mm + (f0 + f) * A.n];
+  }
+}
+
+// the periodic slaves' sums, one lane per value (in the masters' lanes they
+// would hold up nearly every wavefront of a box, see k_boundary_nodes)
+__global__ void __launch_bounds__(256) k_product_members(ProductArgs A) {
+  const long long at = blockIdx.x * 256LL + threadIdx.x;
+  const int q = (int)(at >> 3), f = (int)(at & 7);
+  if (q >= A.nmem || f >= 5) return;
+  const long long k = A.smem[q];
+  const int2 in = A.info[k];
+  if (in.y < 0 || A.sptr[in.x] == q) return;
+  double s[1];
+  node_product<1>(A, k, f, s);
+  A.msum[8 * (size_t)q + f] = s[0];
+}
+
+// per node the product with the slaves folded into their master (bc3per:
+// ascending, slaves zero); kResid: instead r = L^-1 (rmes - product) into
+// start and the sum of its squares to the host, with seq.  Bound by the element
+// products' 40 bytes per node and element from 64^3 on (0.49 ms at 128^3, 4.5
+// TB/s), by launches below: with k_product_in, the element kernel and
+// k_product_members it replaces the refinement's twelve launches and two waits
+// (a mixed step of three iterations at 16^3: 1.41 -> 1.30 ms).
+template <bool kResid>
+__global__ void __launch_bounds__(kNodeThreads) k_product_nodes(ProductArgs A) {
+  const int t = threadIdx.x;
+  const long long n = A.n;
+  double sq = 0.0;
+  for (long long k = blockIdx.x * (long long)kNodeThreads + t; k < n;
+       k += gridDim.x * (long long)kNodeThreads) {
+    double r[5];
+    node_product<5>(A, k, 0, r);
+    const int2 in = A.info[k];
+    if (in.y >= 0) {
+      const int q0 = A.sptr[in.x], q1 = A.sptr[in.x + 1];
+      if (A.smem[q0] == k) {
+        for (int q = q0 + 1; q < q1; ++q) {
+          double s[5];
+          if (A.nmem > 0) {
+#pragma unroll
+            for (int f = 0; f < 5; ++f) s[f] = A.msum[8 * (size_t)q + f];
+          } else {
+            node_product<5>(A, A.smem[q], 0, s);
+          }
+#pragma unroll
+          for (int f = 0; f < 5; ++f) r[f] += s[f];
+        }
+      } else {
+#pragma unroll
+        for (int f = 0; f < 5; ++f) r[f] = 0.0;
+      }
+    }
+    if constexpr (kResid) {
+      double a[5][5];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = j + 1; i < 5; ++i) a[i][j] = A.bdiag[k + (i + 5 * j) * n];
+#pragma unroll
+      for (int f = 0; f < 5; ++f) r[f] = A.rmes[k + f * n] - r[f];
+      lu_solve_lower(a, r);
+#pragma unroll
+      for (int f = 0; f < 5; ++f) {
+        A.start[k + f * n] = r[f];
+        sq += r[f] * r[f];
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) A.w[k + f * n] = r[f];
+    }
+  }
+  if constexpr (kResid) {
+    __shared__ double ws[kNodeThreads / 64];
+    auto block_sum = [&](double v) {
+      v = wave_sum(v);
+      __syncthreads();
+      if ((t & 63) == 0) ws[t >> 6] = v;
+      __syncthreads();
+      return ws[0] + ws[1] + ws[2] + ws[3];
+    };
+    const double s = block_sum(sq);
+    if (t == 0) part_store(A.part + blockIdx.x, s);
+    if (!arrive_last(&A.gm->cnt)) return;
+    double v[kNodeBlocks / kNodeThreads];
+#pragma unroll
+    for (int u = 0; u < kNodeBlocks / kNodeThreads; ++u) {
+      const int b = t + kNodeThreads * u;
+      v[u] = b < (int)gridDim.x ? part_load(A.part + b) : 0.0;
+    }
+    sq = 0.0;
+#pragma unroll
+    for (int u = 0; u < kNodeBlocks / kNodeThreads; ++u) sq += v[u];
+    const double all = block_sum(sq);
+    if (t != 0) return;
+    __hip_atomic_store(&A.host->rsq, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&A.host->rseq, A.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 __global__ void k_end_mark(SolveHost* h, unsigned seq) {
   __hip_atomic_store(&h->end, wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1436,6 +1631,72 @@ int launch_nodes(phg_ctx* c, bool prec, bool solve, double* raw, double* start) 
   } else {
     k_nodes<false><<<g, kNodeThreads, 0, c->stream>>>(A);
   }
+  PHG_HIP(hipGetLastError());
+  return 0;
+}
+
+namespace {
+
+ProductArgs product_args(phg_ctx* c, const double* v) {
+  ProductArgs A{};
+  A.goff = c->inc_goff;
+  A.inc = c->inc;
+  A.out = c->resid;
+  A.v = v;
+  A.iper = c->iper;
+  A.bcm = c->bcm;
+  A.info = c->ninfo;
+  A.sptr = c->sptr;
+  A.smem = c->smem;
+  // below half a wavefront per SIMD the masters' lanes take their slaves' chains
+  // along in less time than a launch (a product at 4913 nodes 98.5 -> 92 us)
+  A.nmem = c->nfold > 0 && c->nshg > 32768 ? c->nmem : 0;
+  A.msum = c->msum;
+  A.n = c->nshg;
+  A.part = c->red_part;
+  A.gm = c->gm;
+  A.host = c->h_sol;
+  return A;
+}
+
+int launch_members(phg_ctx* c, const ProductArgs& A) {
+  if (A.nmem > 0) {
+    k_product_members<<<grid_for(8LL * A.nmem, 256), 256, 0, c->stream>>>(A);
+    PHG_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
+}  // namespace
+
+int launch_tangent_product(phg_ctx* c, const double* v, double* w) {
+  const long long n = c->nshg;
+  k_product_in<false><<<grid_for(n, 256), 256, 0, c->stream>>>(v, nullptr, c->iper, c->bcm,
+                                                              c->vpack, nullptr, n);
+  PHG_HIP(hipGetLastError());
+  PHG_TRY(launch_jv(c));
+  ProductArgs A = product_args(c, v);
+  A.w = w;
+  PHG_TRY(launch_members(c, A));
+  k_product_nodes<false><<<grid_for(n, kNodeThreads), kNodeThreads, 0, c->stream>>>(A);
+  PHG_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_tangent_residual(phg_ctx* c, const double* dy, double* v, double* start) {
+  const long long n = c->nshg;
+  k_product_in<true><<<grid_for(n, 256), 256, 0, c->stream>>>(dy, c->bdiag, c->iper, c->bcm,
+                                                             c->vpack, v, n);
+  PHG_HIP(hipGetLastError());
+  PHG_TRY(launch_jv(c));
+  ProductArgs A = product_args(c, v);
+  A.rmes = c->rmes;
+  A.bdiag = c->bdiag;
+  A.start = start;
+  A.seq = ++c->res_seq;
+  PHG_TRY(launch_members(c, A));
+  const int g = std::min(grid_for(n, kNodeThreads), kNodeBlocks);
+  k_product_nodes<true><<<g, kNodeThreads, 0, c->stream>>>(A);
   PHG_HIP(hipGetLastError());
   return 0;
 }

@@ -668,6 +668,9 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_TRY(dev_alloc(c, &c->wslot, wslot.size()));
   PHG_TRY(dev_alloc(c, &c->sptr, sptr.size()));
   PHG_TRY(dev_alloc(c, &c->smem, smem.size()));
+  c->nmem = (int)smem.size();
+  PHG_TRY(dev_alloc(c, &c->msum, 8 * smem.size()));
+  PHG_TRY(dev_alloc(c, &c->vpack, 8 * (size_t)nshg));
   PHG_TRY(dev_alloc(c, &c->wptr, wptr.size()));
   PHG_TRY(dev_alloc(c, &c->ssum, (size_t)32 * c->nspec));
   PHG_TRY(dev_alloc(c, &c->ninfo, nshg));
@@ -1207,7 +1210,7 @@ constexpr int kMaxRefine = 4;
 // Mixed precision: the tangent is assembled, scaled and stored in float;
 // the Krylov basis, Gram-Schmidt, Givens and norms stay in double.  After
 // each cycle the true residual of the scaled system, b - K z, is formed with
-// the FP64 tangent (launch_jv) and its norm is tested against the same
+// the FP64 tangent (k_jv) and its norm is tested against the same
 // epsnrm as the FP64 path; cycles restart from that residual until it
 // passes (at most kMaxRefine cycles).
 // correct: itrCorrect + itrBC on the state afterwards.
@@ -1272,23 +1275,20 @@ int sol_core(phg_ctx* c, phg_stats* st, bool correct = false) {
   st->pc_fallback = set_aside && c->mp.ready && c->mp.use_pc > 0 ? 4 : 0;
   if (!(unorm < 100. * c->prm.epsM * c->prm.epsM)) {
     double rnorm = unorm, n0 = unorm;  // residual norm, kvec(0)'s norm as stored
-    // true residual of the scaled system, r = b - K dy, normalised into
-    // kvec(0); returns its norm.  FP64 path: the stored (FP64) matrix.
+    // true residual of the scaled system, r = b - K dy, into kvec(0) (n0: its
+    // norm there); returns its norm.  FP64 path: the stored (FP64) matrix.
     // Mixed path: the FP64 tangent without the stored float matrix,
     // r = L^-1 (rmes - A U^-1 dy) with A applied element by element in
-    // double (launch_jv), so the refinement converges on the FP64 system.
+    // double (k_jv), so the refinement converges on the FP64 system.
     auto true_residual = [&](double* norm) -> int {
       if (mixed) {
-        PHG_HIP(hipMemcpyAsync(kvec(c, 1), c->dy, sizeof(double) * V, hipMemcpyDeviceToDevice,
-                               c->stream));
-        PHG_TRY(launch_i3lu(c, c->bdiag, kvec(c, 1), 2));
-        PHG_TRY(launch_jv(c, kvec(c, 1), kvec(c, 2)));
-        PHG_TRY(launch_sub(c, kvec(c, 2), c->rmes, kvec(c, 2), V));
-        PHG_TRY(launch_i3lu(c, c->bdiag, kvec(c, 2), 1));
-      } else {
-        PHG_TRY(launch_spmv(c, c->dy, kvec(c, 1), true));
-        PHG_TRY(launch_sub(c, kvec(c, 2), c->res, kvec(c, 1), V));
+        PHG_TRY(launch_tangent_residual(c, c->dy, kvec(c, 1), kvec(c, 0)));
+        PHG_TRY(wait_token(c, &c->h_sol->rseq, c->res_seq, "the refinement's residual"));
+        *norm = n0 = std::sqrt(c->h_sol->rsq);
+        return 0;
       }
+      PHG_TRY(launch_spmv(c, c->dy, kvec(c, 1), true));
+      PHG_TRY(launch_sub(c, kvec(c, 2), c->res, kvec(c, 1), V));
       PHG_TRY(launch_dot(c, kvec(c, 2), kvec(c, 2), V, S + 5));
       PHG_TRY(launch_scale(c, kvec(c, 0), kvec(c, 2), V, S + 5, S + 6));
       PHG_TRY(download_pinned(c, c->h_scal + 5, S + 5, 2));
@@ -1469,7 +1469,7 @@ extern "C" int phg_finalize(phg_ctx* c) {
                   c->tmp,      c->slot2csr, c->lhs_aos, c->lhs_aos32, c->acc_res, c->acc_bd,
                   c->nodepack, c->inc_goff, c->inc,   c->eslot,   c->qrec,    c->qnode,
                   c->dcw,      c->mtau,     c->gm,      c->rowmap,  c->fam,     c->wres,
-                  c->wptr,     c->wslot,    c->sptr,    c->smem,    c->ssum,    c->ninfo,   c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
+                  c->wptr,     c->wslot,    c->sptr,    c->smem,    c->ssum,    c->ninfo,   c->msum,    c->vpack,   c->mfg.ypre, c->mfg.t1, c->mfg.t2,  c->mfg.pack};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_scal) (void)hipHostFree(c->h_scal);
@@ -1724,7 +1724,7 @@ extern "C" int phg_tangent_ap(phg_ctx* c, const double* y, double* p) {
   PHG_TRY(upload(c, c->y, y, 5 * n));
   PHG_TRY(launch_pack_nodes(c));
   PHG_TRY(upload(c, kvec(c, 0), p, 5 * n));
-  PHG_TRY(launch_jv(c, kvec(c, 0), kvec(c, 1)));
+  PHG_TRY(launch_tangent_product(c, kvec(c, 0), kvec(c, 1)));
   PHG_TRY(download(c, p, kvec(c, 1), 5 * n));
   return sync(c);
 }

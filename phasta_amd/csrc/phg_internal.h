@@ -164,7 +164,8 @@ struct SolveHost {
   double bad;                       // NaN / large entries of res and BDiag
   long long ta[5];                  // GmDev::ta and the nodal kernel's end
   long long end;                    // the solve's end
-  unsigned seq, end_seq;
+  double rsq;                       // k_product_nodes' sum of squares
+  unsigned seq, end_seq, rseq;
 };
 
 // Learned preconditioner state (k_mpnn.hip); allocated by phg_mpnn_init.
@@ -272,6 +273,9 @@ struct phg_ctx {
   int nspec = 0;
   int* sptr = nullptr;          // members of group g: smem[sptr[g] .. sptr[g+1])
   int* smem = nullptr;
+  int nmem = 0;                 // members of all groups
+  double* msum = nullptr;       // nmem x 8: a product's values at periodic slaves
+  double* vpack = nullptr;      // nshg x 8: a product's direction as elements read it
   int* wptr = nullptr;          // contributions of member q: wres[wptr[q] .. wptr[q+1])
   double* ssum = nullptr;       // 32 per group: res (5) at 25, BDiag (25)
   int2* ninfo = nullptr;        // per node: boundary group, periodic family (in
@@ -346,6 +350,7 @@ struct phg_ctx {
   hipEvent_t stage_ev[kStageSlots] = {};  // the end of a slot's last use
   int stage_slot = 0;              // the next upload's
   unsigned sol_seq = 0;            // token of the last solve enqueued
+  unsigned res_seq = 0;            // token of the last refinement residual
   double clk_ms = 0.0;             // ms per tick of the device clock
   double* scal = nullptr;          // device scalars (H column etc.)
   double* h_scal = nullptr;        // pinned mirror
@@ -382,7 +387,11 @@ int launch_diffusive_flux(phg_ctx* c);
 // the last assembly, v read at the periodic masters and w folded (bc3per):
 // the operator of SparseAp + bc3per before the two-sided scaling.  Uses
 // c->resid as scratch, so it runs after the assembly's block pass.
-int launch_jv(phg_ctx* c, const double* v, double* w);
+int launch_jv(phg_ctx* c);  // element products of c->vpack
+int launch_tangent_product(phg_ctx* c, const double* v, double* w);
+// start <- L^-1 (rmes - A U^-1 dy), its squares' sum to h_sol->rsq with res_seq;
+// v: 5 planes of scratch
+int launch_tangent_residual(phg_ctx* c, const double* dy, double* v, double* start);
 
 // matrix-free GMRES (SolMFG): the modified residual of the packed variables
 // yp (8 per node; nullptr: y itself) at the resident state into out

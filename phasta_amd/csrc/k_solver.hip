@@ -1280,6 +1280,25 @@ __global__ void __launch_bounds__(kNodeThreads) k_product_nodes(ProductArgs A) {
   }
 }
 
+// Small host arrays, between device memory and pinned host memory.  To the host
+// one workgroup, which then stores the token; 16 otherwise.  Bound by the bus's
+// latency: all arrays of a call in one launch (4 to 8 us for 5 KB to 128 KB).
+__global__ void __launch_bounds__(1024) k_small_copy(SmallCopy S, unsigned* done, unsigned token) {
+  for (int a = 0; a < S.count; ++a) {
+    unsigned* d = static_cast<unsigned*>(S.seg[a].dst);
+    const unsigned* s = static_cast<const unsigned*>(S.seg[a].src);
+    const unsigned n = (unsigned)S.seg[a].words;
+#pragma unroll 4
+    for (unsigned i = blockIdx.x * 1024 + threadIdx.x; i < n; i += gridDim.x * 1024) d[i] = s[i];
+  }
+  if (!done) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(done, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void k_end_mark(SolveHost* h, unsigned seq) {
   __hip_atomic_store(&h->end, wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1697,6 +1716,12 @@ int launch_tangent_residual(phg_ctx* c, const double* dy, double* v, double* sta
   PHG_TRY(launch_members(c, A));
   const int g = std::min(grid_for(n, kNodeThreads), kNodeBlocks);
   k_product_nodes<true><<<g, kNodeThreads, 0, c->stream>>>(A);
+  PHG_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_small_copy(phg_ctx* c, const SmallCopy& S, unsigned* done) {
+  k_small_copy<<<done ? 1 : 16, 1024, 0, c->stream>>>(S, done, done ? ++c->copy_seq : 0);
   PHG_HIP(hipGetLastError());
   return 0;
 }

@@ -65,18 +65,25 @@ int dev_alloc(phg_ctx* c, T** p, size_t count) {
   return 0;
 }
 
+int wait_token(phg_ctx* c, const volatile unsigned* at, unsigned seq, const char* what);
+
 // ---- host arrays to the device and back ----
 // hipMemcpyAsync on ordinary host memory waits for the copy, 10 to 15 us for
 // each array however small, and moves large results piece after piece through
-// one buffer.  So results move over the bus into a ring of kStageSlots pinned
-// slots while the calling thread copies from it: three arrays of 85.9 MB into
-// new memory 25.1 -> 19.4 ms (12 of them the first touch), of 11.0 MB 2.4 -> 1.2
-// ms (with arrays that are not zeroed first), of 5.6 MB 1.2 -> 0.63.  Small
-// arrays go up through it too, without a wait: a time step of 125 nodes, two
-// arrays up and three down, 341 -> 309 us; large ones gain nothing (5.9 ms for
-// 172 MB either way).  Copying threads beside the caller's own took the CPU from
-// it: a step of 97336 nodes 3.7 ms with one thread, 9.9 with three more for each
-// transfer, 23.7 with OpenMP's.
+// one buffer.  So:
+// - arrays of kSmall bytes together go through a pinned buffer that one kernel
+//   reads or writes, up without a wait, down with one for a word behind the
+//   data (a product at 729 nodes 87 -> 60 us, a time step of 27 nodes 720 -> 240
+//   with the launches saved elsewhere; above, the runtime's copies are as fast).
+// - larger results move over the bus into a ring of kStageSlots pinned slots
+//   while the calling thread copies from it: three arrays of 85.9 MB into new
+//   memory 25.1 -> 19.4 ms (12 of them the first touch), of 11.0 MB 2.4 -> 1.2 ms
+//   (with arrays that are not zeroed first), of 5.6 MB 1.2 -> 0.63.  Below slots
+//   of kStageMin it gains nothing (a piece costs some 15 us), nor do uploads (5.9
+//   ms for 172 MB either way): those are the runtime's.
+// Copying threads beside the caller's own took the CPU from it: a step of 97336
+// nodes 3.7 ms with one thread, 9.9 with three more for each transfer, 23.7 with
+// OpenMP's.
 struct HostArray {
   char* dev;
   char* host;
@@ -116,28 +123,33 @@ size_t bytes_of(std::initializer_list<HostArray> list) {
   return n;
 }
 
+// whole words of four bytes only
+bool small_list(std::initializer_list<HostArray> list) {
+  for (const HostArray& a : list)
+    if (a.bytes % 4) return false;
+  return bytes_of(list) <= kSmall && list.size() <= (size_t)kSmallArrays;
+}
+
 // the arrays may be changed when it returns
 int upload(phg_ctx* c, std::initializer_list<HostArray> list) {
-  bool ring = bytes_of(list) <= kStageSmall;
-  for (const HostArray& a : list) ring = ring && a.host;  // a missing one is the runtime's error
-  if (!ring) {
+  bool small = small_list(list);
+  for (const HostArray& a : list) small = small && a.host;  // a missing one is the runtime's error
+  if (!small) {
     for (const HostArray& a : list)
       if (a.bytes) PHG_HIP(hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c->stream));
     return 0;
   }
-  for (Cursor k{list.begin(), list.end(), 0}; k.a != k.end;) {
-    const int s = c->stage_slot;
-    c->stage_slot = (s + 1) % kStageSlots;
-    char* slot = c->stage + s * c->stage_bytes;
-    PHG_HIP(hipEventSynchronize(c->stage_ev[s]));  // its last use
-    PHG_TRY(fill_slot(c, k, [&](char* dev, char* host, size_t at, size_t n) -> int {
-      std::memcpy(slot + at, host, n);
-      PHG_HIP(hipMemcpyAsync(dev, slot + at, n, hipMemcpyHostToDevice, c->stream));
-      return 0;
-    }));
-    PHG_HIP(hipEventRecord(c->stage_ev[s], c->stream));
+  if (c->small_fill + bytes_of(list) > kSmall) {
+    PHG_HIP(hipStreamSynchronize(c->stream));
+    c->small_fill = 0;
   }
-  return 0;
+  SmallCopy S{};
+  for (const HostArray& a : list) {
+    std::memcpy(c->small + c->small_fill, a.host, a.bytes);
+    S.seg[S.count++] = {a.dev, c->small + c->small_fill, a.bytes / 4};
+    c->small_fill += a.bytes;
+  }
+  return launch_small_copy(c, S, nullptr);
 }
 
 template <typename T>
@@ -147,8 +159,29 @@ int upload(phg_ctx* c, T* dst, const T* src, size_t count) {
 
 // complete when it returns; arrays without a host array are left out
 int download(phg_ctx* c, std::initializer_list<HostArray> list) {
-  // (a piece costs some 15 us: small slots are for small arrays only)
-  if (c->stage_bytes < kStageMin && bytes_of(list) > kStageSmall) {
+  if (small_list(list)) {
+    SmallCopy S{};
+    char* at = c->small + kSmall;
+    for (const HostArray& a : list)
+      if (a.host && a.bytes) {
+        S.seg[S.count++] = {at, a.dev, a.bytes / 4};
+        at += a.bytes;
+      }
+    PHG_TRY(launch_small_copy(c, S, &c->h_sol->copy_seq));
+    PHG_TRY(wait_token(c, &c->h_sol->copy_seq, c->copy_seq, "a copy"));
+    c->small_fill = 0;  // every earlier upload has been read
+    at = c->small + kSmall;
+    for (const HostArray& a : list)
+      if (a.host && a.bytes) {
+        std::memcpy(a.host, at, a.bytes);
+        at += a.bytes;
+      }
+    return 0;
+  }
+  if (!c->stage) {
+    // (a copy asked for behind running kernels takes longer than the wait and the
+    // copy: a product at 9261 nodes 161 us, this way 124)
+    PHG_HIP(hipStreamSynchronize(c->stream));
     for (const HostArray& a : list)
       if (a.host && a.bytes)
         PHG_HIP(hipMemcpyAsync(a.host, a.dev, a.bytes, hipMemcpyDeviceToHost, c->stream));
@@ -723,12 +756,13 @@ int setup(phg_ctx* c, const phg_mesh* m) {
   PHG_HIP(hipHostMalloc((void**)&c->h_gm, kGmMax * sizeof(GmHost), hipHostMallocCoherent));
   std::fill(c->h_gm, c->h_gm + kGmMax, GmHost{});
   PHG_HIP(hipHostMalloc((void**)&c->h_sol, sizeof(SolveHost), hipHostMallocCoherent));
-  // slots of a fourth of a node array up to 2 MB (pinning takes 0.9 ms per MB),
-  // small ones where that is less than kStageMin
+  PHG_HIP(hipHostMalloc((void**)&c->small, 2 * kSmall, hipHostMallocCoherent));
+  // slots of a fourth of a node array up to 2 MB (pinning takes 0.9 ms per MB)
   c->stage_bytes = std::min<size_t>((size_t)(10 * nshg) & ~(size_t)4095, 2 << 20);
-  if (c->stage_bytes < kStageMin) c->stage_bytes = 64 << 10;
-  PHG_HIP(hipHostMalloc((void**)&c->stage, kStageSlots * c->stage_bytes, hipHostMallocDefault));
-  for (auto& e : c->stage_ev) PHG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (c->stage_bytes >= kStageMin) {
+    PHG_HIP(hipHostMalloc((void**)&c->stage, kStageSlots * c->stage_bytes, hipHostMallocDefault));
+    for (auto& e : c->stage_ev) PHG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
   *c->h_sol = SolveHost{};
   {
     int dev = 0, khz = 0;
@@ -1475,6 +1509,7 @@ extern "C" int phg_finalize(phg_ctx* c) {
   if (c->h_scal) (void)hipHostFree(c->h_scal);
   if (c->h_gm) (void)hipHostFree(c->h_gm);
   if (c->h_sol) (void)hipHostFree(c->h_sol);
+  if (c->small) (void)hipHostFree(c->small);
   if (c->stage) (void)hipHostFree(c->stage);
   for (auto ev : c->stage_ev)
     if (ev) (void)hipEventDestroy(ev);
@@ -1721,9 +1756,8 @@ extern "C" int phg_sparse_ap(phg_ctx* c, const double* lhsK, double* p) {
 extern "C" int phg_tangent_ap(phg_ctx* c, const double* y, double* p) {
   PHG_TRY(check_ctx(c));
   const long long n = c->nshg;
-  PHG_TRY(upload(c, c->y, y, 5 * n));
+  PHG_TRY(upload(c, {HostArray(c->y, y, 5 * n), HostArray(kvec(c, 0), p, 5 * n)}));
   PHG_TRY(launch_pack_nodes(c));
-  PHG_TRY(upload(c, kvec(c, 0), p, 5 * n));
   PHG_TRY(launch_tangent_product(c, kvec(c, 0), kvec(c, 1)));
   PHG_TRY(download(c, p, kvec(c, 1), 5 * n));
   return sync(c);

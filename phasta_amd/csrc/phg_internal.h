@@ -165,7 +165,7 @@ struct SolveHost {
   long long ta[5];                  // GmDev::ta and the nodal kernel's end
   long long end;                    // the solve's end
   double rsq;                       // k_product_nodes' sum of squares
-  unsigned seq, end_seq, rseq;
+  unsigned seq, end_seq, rseq, copy_seq;
 };
 
 // Learned preconditioner state (k_mpnn.hip); allocated by phg_mpnn_init.
@@ -229,7 +229,18 @@ struct MpNet {
 };
 
 constexpr int kStageSlots = 4;
-constexpr size_t kStageMin = 256 << 10, kStageSmall = 128 << 10;
+constexpr size_t kStageMin = 768 << 10, kSmall = 128 << 10;
+
+// Small host arrays: words between device memory and pinned host memory.
+constexpr int kSmallArrays = 4;
+struct SmallCopy {
+  struct {
+    void* dst;
+    const void* src;
+    size_t words;
+  } seg[kSmallArrays];
+  int count;
+};
 
 struct phg_ctx {
   long long nshg = 0, nel = 0, nelb = 0, nnz = 0;
@@ -345,10 +356,12 @@ struct phg_ctx {
   GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
   unsigned gm_seq = 0;             // token of the last iteration enqueued
   SolveHost* h_sol = nullptr;      // pinned
-  char* stage = nullptr;           // pinned ring: host arrays on their way
+  char* small = nullptr;           // pinned, kSmall up and kSmall down
+  size_t small_fill = 0;           // bytes of uploads that may still be read
+  unsigned copy_seq = 0;           // token of the last small download
+  char* stage = nullptr;           // pinned ring: results on their way
   size_t stage_bytes = 0;          // of a slot
-  hipEvent_t stage_ev[kStageSlots] = {};  // the end of a slot's last use
-  int stage_slot = 0;              // the next upload's
+  hipEvent_t stage_ev[kStageSlots] = {};  // a slot has arrived
   unsigned sol_seq = 0;            // token of the last solve enqueued
   unsigned res_seq = 0;            // token of the last refinement residual
   double clk_ms = 0.0;             // ms per tick of the device clock
@@ -388,6 +401,8 @@ int launch_diffusive_flux(phg_ctx* c);
 // the operator of SparseAp + bc3per before the two-sided scaling.  Uses
 // c->resid as scratch, so it runs after the assembly's block pass.
 int launch_jv(phg_ctx* c);  // element products of c->vpack
+// done: where to put ++copy_seq when the words are there (nullptr: nowhere)
+int launch_small_copy(phg_ctx* c, const SmallCopy& S, unsigned* done);
 int launch_tangent_product(phg_ctx* c, const double* v, double* w);
 // start <- L^-1 (rmes - A U^-1 dy), its squares' sum to h_sol->rsq with res_seq;
 // v: 5 planes of scratch

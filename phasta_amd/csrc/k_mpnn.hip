@@ -430,19 +430,57 @@ __global__ void __launch_bounds__(256) k_mp_dA(const float* __restrict__ dU,
   }
 }
 
-// dU = dh * silu'(U) (zero on inactive rows), bias gradient partials.
-__global__ void k_mp_dact(const float* __restrict__ dh, const float* __restrict__ U,
-                          const int* __restrict__ ptr, float* __restrict__ dU, long long n) {
-  const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (t >= n * kH) return;
-  const long long row = t / kH;
-  const bool act = ptr[row + 1] > ptr[row];
-  dU[t] = act ? dh[t] * dsilu(U[t]) : 0.f;
+// dU = dh * silu'(U) (zero on inactive rows) and, per workgroup, the sums of its
+// columns (the bias gradient's partials, 64 per workgroup), four columns per
+// lane.  One pass over dh, U and dU; a kernel of its own that read dU again, one
+// workgroup per column at a stride of 256 bytes, took 50 us at 35937 nodes, this
+// one takes 7.5 with its sums, as much as without.
+__global__ void __launch_bounds__(256) k_mp_dact(const float* __restrict__ dh,
+                                                 const float* __restrict__ U,
+                                                 const int* __restrict__ ptr,
+                                                 float* __restrict__ dU, float* __restrict__ bpart,
+                                                 long long n) {
+  __shared__ float4 red[16][16];
+  const int c = threadIdx.x & 15, w = threadIdx.x >> 4;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (long long row = blockIdx.x * 16LL + w; row < n; row += gridDim.x * 16LL) {
+    const bool act = ptr[row + 1] > ptr[row];
+    const size_t at = (size_t)row * kH + 4 * c;
+    const float4 g = *reinterpret_cast<const float4*>(dh + at);
+    const float4 u = *reinterpret_cast<const float4*>(U + at);
+    float4 d;
+    d.x = act ? g.x * dsilu(u.x) : 0.f;
+    d.y = act ? g.y * dsilu(u.y) : 0.f;
+    d.z = act ? g.z * dsilu(u.z) : 0.f;
+    d.w = act ? g.w * dsilu(u.w) : 0.f;
+    *reinterpret_cast<float4*>(dU + at) = d;
+    s.x += d.x;
+    s.y += d.y;
+    s.z += d.z;
+    s.w += d.w;
+  }
+  red[w][c] = s;
+  __syncthreads();
+  if (w > 0) return;
+  for (int k = 1; k < 16; ++k) {
+    const float4 v = red[k][c];
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  *reinterpret_cast<float4*>(bpart + (size_t)blockIdx.x * kH + 4 * c) = s;
 }
 
 // Weight gradient partials: dW[k][c] = sum_rows A[row][k] dU[row][c] over a
 // block's share of rows, MFMA with the rows as the reduction dimension.
-// Tiles of 32 rows are staged in LDS (A transposed on the way in).
+// Tiles of 32 rows are staged in LDS, transposed on the way in: a lane loads 16
+// bytes of two neighbouring rows and writes words of (row, row + 1) pairs, and
+// has asked for the next tile before it works on this one.  (Two bytes at a time
+// and without the next tile in flight the loads' latency made it 79 us at 35937
+// nodes; now 23.)  Rows of 20 words, so that the sixteen lanes of an operand
+// read sixteen places apart by 5 mod 16.
 template <int K>
 __global__ void __launch_bounds__(256) k_mp_dW(const uint16_t* __restrict__ A,
                                                const float* __restrict__ dU,
@@ -450,36 +488,68 @@ __global__ void __launch_bounds__(256) k_mp_dW(const uint16_t* __restrict__ A,
   constexpr int NT = (K / 16) * 4;      // 16x16 output tiles
   constexpr int TPW = NT / 4;           // tiles per wave
   static_assert(NT % 4 == 0, "tiles must split evenly over the 4 waves");
-  __shared__ uint16_t sA[K][32 + 8];    // A^T tile: [k][row]
-  __shared__ uint16_t sU[kH][32 + 8];   // dU^T tile: [c][row]
+  constexpr int kPairs = 16 + 4;        // row pairs of a tile, padded
+  constexpr int kUnits = 16 * (K / 8);  // (row pair, 8 columns)
+  constexpr int kPer = (kUnits + 255) / 256;
+  __shared__ uint32_t sA[K][kPairs];    // A^T tile: [k][row pair]
+  __shared__ uint32_t sU[kH][kPairs];   // dU^T tile: [c][row pair]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = (lane >> 4) * 8;
+  const int rp = threadIdx.x & 15, blk = threadIdx.x >> 4;
   f32x4 acc[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long long base = blockIdx.x * 32LL; base < n; base += (long long)gridDim.x * 32) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < 32 * K; e += 256) {
-      const int r = e / K, k = e % K;
-      const long long row = base + r;
-      sA[k][r] = row < n ? A[(size_t)row * K + k] : (uint16_t)0;
+  uint4 a0[kPer], a1[kPer];
+  float4 u0, u1;
+  const uint4 z4 = make_uint4(0, 0, 0, 0);
+  const float4 zf = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load = [&](long long base) {
+    const long long row = base + 2 * rp;
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int kb = blk + 16 * p;
+      const bool on = kb < K / 8;
+      a0[p] = on && row < n ? *reinterpret_cast<const uint4*>(A + (size_t)row * K + 8 * kb) : z4;
+      a1[p] = on && row + 1 < n
+                  ? *reinterpret_cast<const uint4*>(A + (size_t)(row + 1) * K + 8 * kb)
+                  : z4;
     }
-    for (int e = threadIdx.x; e < 32 * kH; e += 256) {
-      const int r = e / kH, c = e % kH;
-      const long long row = base + r;
-      sU[c][r] = row < n ? f2bf(dU[(size_t)row * kH + c]) : (uint16_t)0;
-    }
+    u0 = row < n ? *reinterpret_cast<const float4*>(dU + (size_t)row * kH + 4 * blk) : zf;
+    u1 = row + 1 < n ? *reinterpret_cast<const float4*>(dU + (size_t)(row + 1) * kH + 4 * blk) : zf;
+  };
+  long long base = blockIdx.x * 32LL;
+  load(base);
+  for (; base < n; base += (long long)gridDim.x * 32) {
     __syncthreads();
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int kb = blk + 16 * p;
+      if (kb < K / 8) {
+        const uint32_t x[4] = {a0[p].x, a0[p].y, a0[p].z, a0[p].w};
+        const uint32_t y[4] = {a1[p].x, a1[p].y, a1[p].z, a1[p].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          sA[8 * kb + 2 * k][rp] = (x[k] & 0xffffu) | (y[k] << 16);
+          sA[8 * kb + 2 * k + 1][rp] = (x[k] >> 16) | (y[k] & 0xffff0000u);
+        }
+      }
+    }
+    sU[4 * blk][rp] = f2bf(u0.x) | ((uint32_t)f2bf(u1.x) << 16);
+    sU[4 * blk + 1][rp] = f2bf(u0.y) | ((uint32_t)f2bf(u1.y) << 16);
+    sU[4 * blk + 2][rp] = f2bf(u0.z) | ((uint32_t)f2bf(u1.z) << 16);
+    sU[4 * blk + 3][rp] = f2bf(u0.w) | ((uint32_t)f2bf(u1.w) << 16);
+    load(base + (long long)gridDim.x * 32);
+    __syncthreads();
+    bf16x8 bv[4];
+#pragma unroll
+    for (int tc = 0; tc < 4; ++tc)
+      bv[tc] = *reinterpret_cast<const bf16x8*>(&sU[16 * tc + lr][lk / 2]);
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
       const int tile = wave * TPW + t;
       const int tk = tile / 4, tc = tile % 4;  // output rows k = 16 tk.., cols c = 16 tc..
-      bf16x8 a, b;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        a[e] = u2bf(sA[16 * tk + lr][lk + e]);
-        b[e] = u2bf(sU[16 * tc + lr][lk + e]);
-      }
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sA[16 * tk + lr][lk / 2]);
+      const bf16x8 b = tc == 0 ? bv[0] : tc == 1 ? bv[1] : tc == 2 ? bv[2] : bv[3];
       acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
     }
   }
@@ -493,28 +563,32 @@ __global__ void __launch_bounds__(256) k_mp_dW(const uint16_t* __restrict__ A,
   }
 }
 
-// sum of nb partial arrays of m floats, fixed order
-__global__ void k_mp_sum_parts(const float* __restrict__ part, int nb, int m, float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += part[(size_t)b * m + i];
-  out[i] = s;
-}
-
-// column sums of dU (bias gradient), fixed order per column
-__global__ void k_mp_colsum(const float* __restrict__ dU, long long n, float* __restrict__ out) {
-  __shared__ float red[256];
-  const int c = blockIdx.x;  // column
-  float s = 0.f;
-  for (long long r = threadIdx.x; r < n; r += blockDim.x) s += dU[(size_t)r * kH + c];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+// sums of partial arrays in a fixed order: nb of m floats into out and, in the
+// last workgroup, nb2 of 64 floats into out2 (without out2 none).  Four
+// wavefronts share a column's partials, eight loads each in flight: a lane that
+// added all of them took 60 us for 256 parts of 20480 values, this takes 9.
+__global__ void __launch_bounds__(256) k_mp_sum_parts(const float* __restrict__ part, int nb, int m,
+                                                      float* __restrict__ out,
+                                                      const float* __restrict__ part2, int nb2,
+                                                      float* __restrict__ out2) {
+  __shared__ float red[4][64];
+  const int c = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int i = blockIdx.x * 64 + c;
+  if (out2 && blockIdx.x == gridDim.x - 1) {
+    part = part2;
+    nb = nb2;
+    m = 64;
+    out = out2;
+    i = c;
   }
-  if (threadIdx.x == 0) out[c] = red[0];
+  float s = 0.f;
+  if (i < m) {
+#pragma unroll 8
+    for (int b = w; b < nb; b += 4) s += part[(size_t)b * m + i];
+  }
+  red[w][c] = s;
+  __syncthreads();
+  if (w == 0 && i < m) out[i] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
 }
 
 // ---------------- output ----------------
@@ -628,39 +702,48 @@ __global__ void k_mp_res_loss(double* sbuf) {
   sbuf[4] += l;
 }
 
-// dWout[k][f] = sum_i h[i][k] dY[i][f]; dbout[f] = sum_i dY[i][f]  (one block
-// per k, k = 64 for the bias)
-__global__ void k_mp_out_grad_w(const uint16_t* __restrict__ h, const float* __restrict__ dY,
-                                long long n, float* __restrict__ out /* 65 x 5 */) {
-  __shared__ float red[5][256];
-  const int k = blockIdx.x;
-  float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-    const float hv = k < kH ? bf2f(h[(size_t)i * kH + k]) : 1.0f;
+// dWout[k][f] = sum_i h[i][k] dY[i][f] and dbout[f] = sum_i dY[i][f]: each
+// workgroup's rows, 65 x 5 partials for k_mp_sum_parts.  A lane per column k, so
+// that h is read in rows (one workgroup per k read two bytes of each: 84 us at
+// 35937 nodes, now with the sum 14).
+__global__ void __launch_bounds__(256) k_mp_out_grad_w(const uint16_t* __restrict__ h,
+                                                       const float* __restrict__ dY, long long n,
+                                                       float* __restrict__ part) {
+  __shared__ float red[4][(kH + 1) * 5];
+  const int k = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, b[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (long long i = blockIdx.x * 4LL + w; i < n; i += gridDim.x * 4LL) {
+    const float hv = bf2f(h[(size_t)i * kH + k]);
 #pragma unroll
-    for (int f = 0; f < 5; ++f) s[f] += hv * dY[i * 5 + f];
-  }
-#pragma unroll
-  for (int f = 0; f < 5; ++f) red[f][threadIdx.x] = s[f];
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-#pragma unroll
-      for (int f = 0; f < 5; ++f) red[f][threadIdx.x] += red[f][threadIdx.x + o];
+    for (int f = 0; f < 5; ++f) {
+      const float d = dY[i * 5 + f];
+      s[f] += hv * d;
+      b[f] += d;
     }
-    __syncthreads();
   }
-  if (threadIdx.x < 5) out[k * 5 + threadIdx.x] = red[threadIdx.x][0];
+#pragma unroll
+  for (int f = 0; f < 5; ++f) {
+    red[w][5 * k + f] = s[f];
+    if (k == 0) red[w][5 * kH + f] = b[f];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < (kH + 1) * 5; e += 256)
+    part[(size_t)blockIdx.x * (kH + 1) * 5 + e] =
+        (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
 }
 
-// sum of a float array in fixed order (one block)
-__global__ void k_mp_sum(const float* __restrict__ a, long long n, float* __restrict__ out) {
-  __shared__ float red[256];
+// sum of a float array in fixed order (one workgroup, eight loads per lane in
+// flight: 35 -> 6 us at 35937 nodes)
+__global__ void __launch_bounds__(1024) k_mp_sum(const float* __restrict__ a, long long n,
+                                                 float* __restrict__ out) {
+  __shared__ float red[1024];
   float s = 0.f;
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) s += a[i];
+#pragma unroll 8
+  for (long long i = threadIdx.x; i < n; i += 1024) s += a[i];
   red[threadIdx.x] = s;
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
+  for (int o = 512; o > 0; o >>= 1) {
     if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
@@ -773,6 +856,7 @@ constexpr int kWoff[4] = {Layout::W0, Layout::W1, Layout::W2, Layout::W3};
 constexpr int kBoff[4] = {Layout::b0, Layout::b1, Layout::b2, Layout::b3};
 constexpr int kK[4] = {kNin, kNagg, kNagg, kNagg};
 constexpr int kPartBlocks = 256;
+constexpr int kActBlocks = 512;   // workgroups of k_mp_dact
 
 template <typename T>
 int mp_alloc(phg_ctx* c, T** p, size_t count) {
@@ -924,6 +1008,7 @@ int mp_alloc_train(phg_ctx* c) {
   PHG_TRY(mp_alloc(c, &M.sq, n));
   M.nparts = (int)std::min<long long>(kPartBlocks, (n + 31) / 32);
   PHG_TRY(mp_alloc(c, &M.part, (size_t)M.nparts * kNagg * kH));
+  PHG_TRY(mp_alloc(c, &M.bpart, (size_t)kActBlocks * kH));
   if (!M.param_owner) {
     PHG_TRY(mp_alloc(c, &M.g, Layout::total));
     PHG_TRY(mp_alloc(c, &M.m1, Layout::total));
@@ -941,7 +1026,7 @@ int mp_free(phg_ctx* c) {
   void* ptrs[] = {M.ptr,  M.col,  M.rev,  M.ev,   M.esum,  M.inv,   M.dscale, M.bd_raw, M.zhat,
                   M.x,    M.h[0], M.h[1], M.h[2], M.h[3],  M.A[0],  M.A[1],   M.A[2],   M.U[0],
                   M.U[1], M.U[2], M.U[3], M.Y,    M.Ystar, M.dh,    M.dU,     M.dA,     M.dY,
-                  M.sq,   M.part, M.sbuf, M.vin,  M.zout,  M.zbasis, M.wplain, M.ds,
+                  M.sq,   M.part, M.bpart, M.sbuf, M.vin,  M.zout,  M.zbasis, M.wplain, M.ds,
                   M.rbuf, M.gbuf};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -1093,17 +1178,21 @@ int mp_backward(phg_ctx* c, float lr, double* loss_out, bool given_dy) {
                                                           inv_na, M.dY, M.dh, M.sq, n);
     PHG_HIP(hipGetLastError());
     // loss: fixed-order float sum of the per-node squared errors
-    k_mp_sum<<<1, 256, 0, c->stream>>>(M.sq, n, M.part);
+    k_mp_sum<<<1, 1024, 0, c->stream>>>(M.sq, n, M.part);
     k_mp_loss<<<1, 1, 0, c->stream>>>(M.part, 1.0 / (double)std::max<long long>(1, M.n_act),
                                       M.sbuf + 2);
     PHG_HIP(hipGetLastError());
   }
-  k_mp_out_grad_w<<<kH + 1, 256, 0, c->stream>>>(M.h[3], M.dY, n, M.g + Layout::Wo);
+  const int go = (int)std::min<long long>(256, (n + 31) / 32), mo = (kH + 1) * 5;
+  k_mp_out_grad_w<<<go, 256, 0, c->stream>>>(M.h[3], M.dY, n, M.part);
+  PHG_HIP(hipGetLastError());
+  k_mp_sum_parts<<<grid_for(mo, 64), 256, 0, c->stream>>>(M.part, go, mo, M.g + Layout::Wo,
+                                                         nullptr, 0, nullptr);
   PHG_HIP(hipGetLastError());
   const int gd = grid_for(n, 64);
-  const long long nH = n * kH;
+  const int ga = (int)std::min<long long>(kActBlocks, (n + 15) / 16);
   for (int l = 3; l >= 0; --l) {
-    k_mp_dact<<<grid_for(nH, 256), 256, 0, c->stream>>>(M.dh, M.U[l], M.ptr, M.dU, n);
+    k_mp_dact<<<ga, 256, 0, c->stream>>>(M.dh, M.U[l], M.ptr, M.dU, M.bpart, n);
     PHG_HIP(hipGetLastError());
     const int K = kK[l];
     if (l > 0)
@@ -1111,9 +1200,8 @@ int mp_backward(phg_ctx* c, float lr, double* loss_out, bool given_dy) {
     else
       k_mp_dW<kNin><<<M.nparts, 256, 0, c->stream>>>(M.x, M.dU, M.part, n);
     PHG_HIP(hipGetLastError());
-    k_mp_sum_parts<<<grid_for(K * kH, 256), 256, 0, c->stream>>>(M.part, M.nparts, K * kH,
-                                                                 M.g + kWoff[l]);
-    k_mp_colsum<<<kH, 256, 0, c->stream>>>(M.dU, n, M.g + kBoff[l]);
+    k_mp_sum_parts<<<K * kH / 64 + 1, 256, 0, c->stream>>>(
+        M.part, M.nparts, K * kH, M.g + kWoff[l], M.bpart, ga, M.g + kBoff[l]);
     PHG_HIP(hipGetLastError());
     if (l == 0) break;
     k_mp_dA<<<gd, 256, 0, c->stream>>>(M.dU, M.wr[l], M.dA, n);

@@ -203,6 +203,7 @@ struct MpNet {
   float* sq = nullptr;       // n squared errors
   float* part = nullptr;     // weight-gradient partials
   int nparts = 0;
+  float* bpart = nullptr;      // bias gradient partials
   float* w = nullptr;        // master weights (float)
   float* g = nullptr;        // gradient
   float* m1 = nullptr;       // Adam moments

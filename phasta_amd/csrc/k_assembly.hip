@@ -197,7 +197,6 @@ __device__ __forceinline__ S* pt_at(S* qps, long long e, int q) {
 //
 // Every lane of the wavefront takes part, with an element that may be read; one
 // wavefront per workgroup, so a wait of its own is the only synchronisation.
-typedef int phg_i4 __attribute__((ext_vector_type(4)));
 // two doubles at an 8-byte boundary
 typedef double phg_d2u __attribute__((ext_vector_type(2), aligned(8)));
 
@@ -264,12 +263,6 @@ __device__ __forceinline__ S piece(const phg_i4 A[4], int k) {
   }
 }
 
-// one read of LDS that direct loads have written, complete when it returns
-__device__ __forceinline__ phg_i4 lds_i4(unsigned at) {
-  phg_i4 v;
-  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");
-  return v;
-}
 __device__ __forceinline__ int lds_int(unsigned at) {
   int v;
   asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");

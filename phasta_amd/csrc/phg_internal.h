@@ -101,6 +101,24 @@ __device__ inline void store_slot(double* blk, int r, const A a[25]) {
   blk[24 * kGroup + r] = (double)a[24];
 }
 
+typedef int phg_i4 __attribute__((ext_vector_type(4)));
+// one read of LDS that direct loads have written, complete when it returns
+__device__ __forceinline__ phg_i4 lds_i4(unsigned at) {
+  phg_i4 v;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");
+  return v;
+}
+
+// four at once
+__device__ __forceinline__ void lds_i4(const unsigned at[4], phg_i4 v[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+      "ds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+      : "memory");
+}
+
 // Largest number of element blocks one assembly lane sums (the blocks of
 // one CSR entry are split into chunks of at most this size).  Measured at
 // 128^3 (float / FP64 block pass): 2: 7.90 / 12.74 ms, 3: 7.81 / 12.41,

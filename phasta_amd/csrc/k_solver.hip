@@ -1,5 +1,6 @@
 // Linear-solver kernels on gfx950 for the block-diagonal-preconditioned
-// GMRES of SolGMRs (solgmr.f:368-744): 5x5 block LU of BDiag (i3lu.f),
+// GMRES of SolGMRs (solgmr.f:368-744): the nodal work between assembly and
+// Krylov loop (bc3res.f, bc3bdg.f, tnanq.f), 5x5 block LU of BDiag (i3lu.f),
 // two-sided block scaling of the matrix (spsi3pre.f), the block-CSR matvec
 // with the periodic gather (sparseap.f), the periodic fold (bc3per.f),
 // Krylov-vector kernels with deterministic wavefront/grid reductions
@@ -12,6 +13,8 @@
 // vals[(s*25 + e)*64 + r].  Each matrix load of a wavefront is therefore one
 // contiguous 512-byte (FP64) or 256-byte (FP32) segment.  Rows shorter than
 // the group's slot count are padded with zero blocks.
+#include <type_traits>
+
 #include "phg_internal.h"
 
 namespace {
@@ -284,15 +287,25 @@ __global__ void __launch_bounds__(kPreWaves * kGroup) k_spsi3pre(
 // scaled system lose digits to cancellation (on the 16^3 box the refinement
 // loop then needed 12 instead of 10 Krylov iterations), while the kernel is
 // bound by the matrix bytes, which float storage halves either way.
-// One workgroup of kSpmvWaves wavefronts per 64-row group: wavefront w takes
-// the group's slots w, w + kSpmvWaves, ..., so the wavefronts of a workgroup
-// stream adjacent slots together and each runs a short loop; the partial row
-// sums are added in wavefront order through LDS (fixed order, deterministic).
+// One workgroup of W wavefronts per 64-row group: wavefront w takes the group's
+// slots w, w + W, ..., so the wavefronts of a workgroup stream adjacent slots
+// together and each runs a short loop; the partial row sums are added in
+// wavefront order through LDS (fixed order, deterministic), a component per
+// wavefront.  With at most a group per CU the loop's latency is the product's
+// time, and W = 16 leaves one or two slots to each wavefront; above, the slots
+// of a workgroup in flight should be some 13 to 25 KB.  us per product for W = 4
+// | 8 | 16, float and double: 16^3 hexes (77 groups) 7.1 | 6.1 | 5.6 and 8.7 | 7.3 |
+// 6.9; 24^3 (245) 7.9 | 7.1 | 6.8 and 10.9 | 9.7 | 9.6; 28^3 (382) 10.3 | 9.9 | 11.6
+// and 15.5 | 15.6 | 16.4; 64^3 81.0 | 82.8 | 98.0 and 142.3 | 138.2 | 151.6; 128^3 644
+// | 655 | 768 and 1138 | 1101 | 1209.
 // The grid is a multiple of 8: consecutive workgroups go to different XCDs
 // (round robin), so workgroup b takes group (b % 8) * per + b / 8 and each
 // XCD sweeps one contiguous eighth of the rows, whose column neighbours
 // (rows +-1, +-(N+1), +-(N+1)^2 on the box) then stay in that XCD's L2.
-constexpr int kSpmvWaves = 4;
+template <typename T>
+constexpr int kSpmvWaves = sizeof(T) == 8 ? 8 : 4;
+constexpr int kSpmvWavesFew = 16;
+constexpr long long kSpmvFew = 256;  // groups: one per CU
 
 // rowmap: row of each (group, lane), -1 padding.  fam: per (group, lane) the
 // number of periodic slaves whose rows follow the lane's (a master), kFamSlave
@@ -302,25 +315,26 @@ constexpr int kSpmvWaves = 4;
 // product, as long as the whole product up to 16^3).
 // gate (nullable): the product is skipped when *gate is set (a Krylov
 // iteration enqueued before the host knew that the last one had converged).
-template <typename T, typename Acc>
-__global__ void __launch_bounds__(kSpmvWaves * kGroup) k_spmv(
+template <typename T, typename Acc, int W>
+__global__ void __launch_bounds__(W * kGroup) k_spmv(
     const T* __restrict__ vals, const int* __restrict__ scolp,
     const long long* __restrict__ grp_slot, const int* __restrict__ rowmap,
     const uint8_t* __restrict__ fam, const double* __restrict__ p, double* __restrict__ q,
     long long n, long long ngroups, int fold, const int* gate, long long* t0) {
   if (gate && *gate) return;
   if (t0 && blockIdx.x == 0 && threadIdx.x == 0) *t0 = wall_clock64();
-  __shared__ Acc part[kSpmvWaves][5][kGroup];
+  __shared__ Acc part[W][5][kGroup];
   const long long per = (gridDim.x + 7) / 8;
   const long long g = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (g >= ngroups) return;  // whole workgroup
   const int w = threadIdx.x / kGroup, r = threadIdx.x % kGroup;
   const long long s0 = grp_slot[g] + w, s1 = grp_slot[g + 1];
+  const long long row = rowmap[g * kGroup + r];
+  const int nf = fold ? fam[g * kGroup + r] : 0;
   Acc t[5] = {0, 0, 0, 0, 0};
   // software pipeline: the gathers of p for the next slot and the column
   // index of the one after are issued before the block of this slot is
   // consumed (padding lanes read column 0 and zero blocks)
-  constexpr int W = kSpmvWaves;
   Acc pc[5] = {0, 0, 0, 0, 0};
   if (s0 < s1) {
     const long long j0 = scolp[s0 * kGroup + r];
@@ -347,8 +361,6 @@ __global__ void __launch_bounds__(kSpmvWaves * kGroup) k_spmv(
 #pragma unroll
   for (int f = 0; f < 5; ++f) part[w][f][r] = t[f];
   __syncthreads();
-  if (w != 0) return;
-  const long long row = rowmap[g * kGroup + r];
   if (row < 0) return;
   auto rowsum = [&](int f, int rr) {
     Acc v = part[0][f][rr];
@@ -356,9 +368,7 @@ __global__ void __launch_bounds__(kSpmvWaves * kGroup) k_spmv(
     for (int k = 1; k < W; ++k) v += part[k][f][rr];
     return (double)v;
   };
-  const int nf = fold ? fam[g * kGroup + r] : 0;
-#pragma unroll
-  for (int f = 0; f < 5; ++f) {
+  for (int f = w; f < 5; f += W) {
     double v = nf == kFamSlave ? 0.0 : rowsum(f, r);
     if (nf > 0 && nf < kFamSlave)
       for (int k = 1; k <= nf; ++k) v += rowsum(f, r + k);
@@ -1489,16 +1499,24 @@ int launch_spmv(phg_ctx* c, const double* p, double* q, bool fold, const int* ga
                 long long* t0) {
   PHG_TRY(require_matrix(c, "SparseAp"));
   const int g = (int)((c->ngroups + 7) / 8 * 8);  // one workgroup per group, XCD-strided
-  const int nt = kSpmvWaves * kGroup;
   const int in_group = fold && c->fam_in_group ? 1 : 0;
+  auto run = [&](auto vals, auto waves) {
+    constexpr int W = decltype(waves)::value;
+    k_spmv<std::remove_pointer_t<decltype(vals)>, double, W><<<g, W * kGroup, 0, c->stream>>>(
+        vals, c->scolp, c->grp_slot, c->rowmap, c->fam, p, q, c->nshg, c->ngroups, in_group, gate,
+        t0);
+  };
+  auto pick = [&](auto vals) {
+    using T = std::remove_pointer_t<decltype(vals)>;
+    if (c->ngroups <= kSpmvFew)
+      run(vals, std::integral_constant<int, kSpmvWavesFew>{});
+    else
+      run(vals, std::integral_constant<int, kSpmvWaves<T>>{});
+  };
   if (c->precision == PHG_MIXED)
-    k_spmv<float, double><<<g, nt, 0, c->stream>>>(c->lhs32, c->scolp, c->grp_slot, c->rowmap,
-                                                   c->fam, p, q, c->nshg, c->ngroups, in_group,
-                                                   gate, t0);
+    pick(c->lhs32);
   else
-    k_spmv<double, double><<<g, nt, 0, c->stream>>>(c->lhs64, c->scolp, c->grp_slot, c->rowmap,
-                                                    c->fam, p, q, c->nshg, c->ngroups, in_group,
-                                                    gate, t0);
+    pick(c->lhs64);
   PHG_HIP(hipGetLastError());
   // a family of more than kGroup rows: the rows lie in several groups.  The
   // fold runs whatever the gate says: on a skipped product's old output it

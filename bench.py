@@ -134,8 +134,7 @@ def run_arm(case, precision, newton, steps, warmup, weights=None, idiff=0, mfg=F
     ms_copy, by_copy = gpu.bench_copy(5)
     # the matvec on the arm's resident matrix, 20 launches back to back
     # between two HIP events on the library stream: the kernel's own time,
-    # without the launch gaps that the per-launch events inside GMRES see
-    # (the host waits for each Hessenberg column before the next launch)
+    # without the launch gaps that the device-clock stamps inside GMRES see
     ms_mv, by_mv = gpu.bench_spmv(20) if not mfg else (float("nan"), float("nan"))
     info = gpu.info()
     gpu.close()
@@ -208,8 +207,8 @@ def main():
     head = res[head_name]
     value = nel / (head["ms"] / 1e3)
 
-    # live assembly timing of the headline arm (HIP events on the library
-    # stream around the point pass and the block pass): FLOP rate of the
+    # live assembly timing of the headline arm (device-clock stamps around
+    # the point pass and the block pass): FLOP rate of the
     # frozen e3 count against the chip's peak in the arm's tangent type
     st = head["stats"]
     ms_pt = sum(s["ms_point"] for s in st) / len(st)
@@ -229,7 +228,7 @@ def main():
                 "ms_point_pass": round(ms_pt, 4), "ms_block_pass": round(ms_bl, 4)}
     # matvec of the headline arm: HIP events on the library stream, 20
     # back-to-back launches on the arm's resident matrix after the timed
-    # steps (the kernel's time); the average of the per-launch events inside
+    # steps (the kernel's time); the average of the device-clock times inside
     # the timed GMRES solves (which include each launch's gap) beside it
     ms_spmv = sum(s["ms_spmv"] for s in st)
     n_spmv = sum(s["n_spmv"] for s in st)

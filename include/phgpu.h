@@ -99,7 +99,7 @@ typedef struct phg_stats {
   double reslast;        /* rstatCheck memory across calls                 */
   long long nnan, nlarge;
   double ms_assembly, ms_solve, ms_total;
-  double ms_spmv, ms_mgs; /* summed HIP-event times of the matvec and MGS  */
+  double ms_spmv, ms_mgs; /* summed device-clock times of matvec and MGS    */
   int n_spmv, n_mgs;      /* launches behind ms_spmv / ms_mgs              */
   int refine_cycles;      /* GMRES cycles run (1 on the plain FP64 path)   */
   int pc_fallback;        /* learned PC: 0 its cycle converged (or unused),
@@ -113,8 +113,8 @@ typedef struct phg_stats {
   double orth_loss;       /* max over the solve's cycles of
                              max_ij |u_i . u_j - delta_ij| of the Krylov basis
                              (phg_diagnostics flag PHG_DIAG_ORTH; else 0)   */
-  double ms_point;        /* HIP-event time of the assembly's point pass     */
-  double ms_blocks;       /* HIP-event time of its block (tangent) pass      */
+  double ms_point;        /* device-clock time of the assembly's point pass  */
+  double ms_blocks;       /* device-clock time of its block (tangent) pass   */
 } phg_stats;
 
 typedef struct phg_ctx phg_ctx;

@@ -1,7 +1,6 @@
 // Element assembly on gfx950: residual, 5x5 block tangent and block
 // diagonal for linear tets (the work of ElmGMRs -> AsIGMR -> e3 and
-// AsBMFG -> e3b, elmgmr.f:280-612), plus the nodal Dirichlet/periodic
-// constraints on res and BDiag (bc3res.f, bc3bdg.f).
+// AsBMFG -> e3b, elmgmr.f:280-612).
 //
 // Two passes, every output written exactly once:
 //
@@ -21,7 +20,7 @@
 //                also sums the node's residual and its BDiag.
 //  k_asm_pairs   the same with one lane forming both blocks (A,B) and (B,A)
 //                of an off-diagonal pair from one read of the element
-//                records (Shakib's or Franca's tau without DC).
+//                records (in double for Shakib's or Franca's tau without DC).
 //
 // No read-modify-write of the matrix, no atomics, no element colouring, and
 // the summation order is fixed, so the result is deterministic.

@@ -212,6 +212,40 @@ __device__ __forceinline__ void store5(double* o, const double v[5]) {
   o[4] = v[4];
 }
 
+// The node lines of a wavefront's sixteen elements through LDS: an octet of
+// lanes asks for a line of 128 bytes once (seven loads of 16 bytes to one line,
+// the first of them still on its way, held up the L1: stalls on pending lines in
+// 61 % of k_asm_qp's cycles).  Load i takes node i / 2 of elements 8 (i % 2) to
+// 8 (i % 2) + 7, an octet each; piece p of element el lies at place p ^ (el / 2 %
+// 8) of its line, so that the four elements that one LDS cycle serves are apart.
+struct NodeLines {
+  const phg_i4* at[4];  // this lane's element's lines
+  int sw;
+  __device__ __forceinline__ NodeLines(phg_i4* lds_all, const int* ien, const double* node,
+                                       long long e0, long long nel) {
+    typedef const __attribute__((address_space(1))) void* gp;
+    typedef __attribute__((address_space(3))) phg_i4* lp;
+    const int lane = threadIdx.x & 63, o = lane >> 3, el = lane >> 2;
+    phg_i4* lds = lds_all + 512 * (threadIdx.x >> 6);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int ee = 8 * (i & 1) + o;
+      const long long nd = ien[(i >> 1) * nel + min(e0 + ee, nel - 1)];
+      const phg_i4* line = reinterpret_cast<const phg_i4*>(node + 16 * nd);
+      __builtin_amdgcn_global_load_lds((gp)(line + ((lane & 7) ^ ((ee >> 1) & 7))),
+                                       (lp)(lds + 64 * i), 16, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) at[k] = lds + 128 * k + 64 * (el >> 3) + 8 * (el & 7);
+    sw = (el >> 1) & 7;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  // values 2 p and 2 p + 1 of node k's line
+  __device__ __forceinline__ double2 pair(int k, int p) const {
+    return *reinterpret_cast<const double2*>(at[k] + (p ^ sw));
+  }
+};
+
 // The sum over a quad's lanes of r_q[a] for node a = q, without the LDS pipe
 // that a shuffle takes: each lane gives its neighbour the two nodes that are the
 // neighbour's and then, two lanes on, one.  (r_q + r_q^1) + (r_q^2 + r_q^3), the
@@ -1067,12 +1101,15 @@ __device__ __forceinline__ void wall_element(const QpArgs& A, long long p) {
 // the diffusive flux and the point's factor is kept for the tangent pass.
 // kMT: the matrix tau of e3tau_nd (itau = 10) replaces Shakib's diagonal
 // tau; W PTau is kept for the tangent pass.
-// Bound by latency at two wavefronts per SIMD (vector ALU 45 % busy, 40 % of the
-// time its bytes at the copy rate): at 128^3 2.95 -> 2.65 ms with float records,
-// 4.01 -> 2.88 with double ones (shorter, and the quad's sums without shuffles);
-// three wavefronts per SIMD, with 12 words spilled, took 3.13 and 3.21.
+// Bound by latency at two wavefronts per SIMD (vector ALU 45 to 48 % busy, 40 % of
+// the time its bytes at the copy rate): at 128^3 2.95 -> 2.58 ms with float records
+// and 4.01 -> 2.75 with double ones, of that 5 and 8 % by NodeLines, the rest by shorter
+// records and the quad's sums without shuffles.  Three wavefronts per SIMD, with
+// 12 words spilled, took 3.13 and 3.21.  The variants with DC or the matrix tau
+// are held to 256 registers, two wavefronts per SIMD (float, both, 45^3 hexes: 379
+// -> 340 us with 27 words spilled, 335 with NodeLines).
 template <typename S, bool kDiff, bool kDC, bool kMT>
-__global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
+__global__ void __launch_bounds__(256, 2) k_asm_qp(QpArgs A) {
   if ((int)blockIdx.x >= A.qp_groups) {
     wall_element(A, (long long)(blockIdx.x - A.qp_groups) * 256 + threadIdx.x);
     return;
@@ -1086,12 +1123,12 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   int nd[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nd[k] = A.ien[k * nel + e];
+  __shared__ phg_i4 lines_lds[4 * 512];
+  const NodeLines lines(lines_lds, A.ien, A.node, blockIdx.x * 64LL + 16 * (threadIdx.x >> 6), nel);
   double xl[4][3];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    // node lines are 128-byte records: 16-byte loads
-    const double2* v = reinterpret_cast<const double2*>(A.node + 16 * (size_t)nd[k]);
-    const double2 x01 = v[5], x2 = v[6];
+    const double2 x01 = lines.pair(k, 5), x2 = lines.pair(k, 6);
     xl[k][0] = x01.x;
     xl[k][1] = x01.y;
     xl[k][2] = x2.x;
@@ -1130,11 +1167,10 @@ __global__ void __launch_bounds__(256) k_asm_qp(QpArgs A) {
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const double2* vp = reinterpret_cast<const double2*>(A.node + 16 * (size_t)nd[k]);
     double v[10];
 #pragma unroll
     for (int t = 0; t < 5; ++t) {
-      const double2 u = vp[t];
+      const double2 u = lines.pair(k, t);
       v[2 * t] = u.x;
       v[2 * t + 1] = u.y;
     }

@@ -1888,6 +1888,25 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
       S v[pt_vals<S>()];
       R Nqa, Nqb;
       pipe.point(q, k, more, code, next, v, Nqa, Nqb);
+      // the point's W PTau and DC weights, asked for together and before any of
+      // them is used: beside Pipe's loads into LDS, whose number depends on the
+      // lane's blocks, the compiler waits for all loads at each use, and with
+      // each load at its own use (DC and the matrix tau, double) a point took
+      // thirteen such waits: the pass 6.02 ms at 64^3 hexes, so 3.80 (4.39 with
+      // every record loaded by its lane)
+      R WPT[25];
+      double dw[6];
+      if constexpr (kMT) {
+        const S* mp = reinterpret_cast<const S*>(A.mtau) + ((size_t)e * 4 + q) * mt_stride<S>();
+#pragma unroll
+        for (int i = 0; i < 25; ++i) WPT[i] = (R)mp[i];
+        if constexpr (kDC) {
+          const double* d = A.dcw + ((size_t)e * 4 + q) * 8;
+#pragma unroll
+          for (int i = 0; i < 6; ++i) dw[i] = d[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
       const Pt<R> pt = decode_pt<R, S>(v, pc);
       const R uq[3] = {pt.u[0], pt.u[1], pt.u[2]};
       ub[0] += uq[0];
@@ -1901,12 +1920,11 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
         // point's rotated giju
         R dq;
         if constexpr (kMT) {
-          const double* d = A.dcw + ((size_t)e * 4 + q) * 8;
           dq = (R)0;
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) dq += sR[i] * (R)d[gu_idx(i, j)] * rR[j];
+            for (int j = 0; j < 3; ++j) dq += sR[i] * (R)dw[gu_idx(i, j)] * rR[j];
         } else {
           dq = (R)A.dcw[(size_t)e * 4 + q];
         }
@@ -1914,10 +1932,6 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
       }
       if constexpr (kMT) {
         // rows of P = A(s_a) W PTau + N_a I from the point's W PTau
-        R WPT[25];
-        const S* mp = reinterpret_cast<const S*>(A.mtau) + ((size_t)e * 4 + q) * mt_stride<S>();
-#pragma unroll
-        for (int k = 0; k < 25; ++k) WPT[k] = (R)mp[k];
         mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, sR, rR, W * Nqa, Nqb, acc);
         if constexpr (kNd) {
           // row m of A_k (the flux Jacobian along x_k, pressure-primitive)

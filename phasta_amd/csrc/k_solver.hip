@@ -658,6 +658,7 @@ struct GsArgs {
   long long n, kstr;     // length, stride between basis vectors (even)
   int nv, K, minIters;   // nv: the iteration number, 1..K
   int unit;              // w is the product of u_i, not of w_i
+  int clocked;           // the product's time is GmDev::t0 to the dots' start; else 0
   double unorm, epsnrm;  // of the cycle
   double n0;             // norm of the start vector as stored
   double* part;          // 2 nv channels of `chan` partials
@@ -679,7 +680,10 @@ template <int kT>
 __global__ void __launch_bounds__(kGsThreads) k_gs_dots(GsArgs A) {
   GmDev& gm = *A.gm;
   if (A.nv > 1 && gm.done) return;
-  if (blockIdx.x == 0 && threadIdx.x == 0) gm.t1 = wall_clock64();
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    gm.t1 = wall_clock64();
+    if (!A.clocked) gm.t0 = gm.t1;
+  }
   __shared__ double red[4][2 * kGmMax], D[2 * kGmMax], nr[kGmMax];
   __shared__ double G[kGmMax * (kGmMax - 1) / 2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1623,8 +1627,8 @@ int launch_dot(phg_ctx* c, const double* a, const double* b, long long n, double
   return launch_finish(c, 0, np, np, 1, out);
 }
 
-int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm, double n0,
-              unsigned seq) {
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, bool clocked, double unorm, double epsnrm,
+              double n0, unsigned seq) {
   if (iK < 1 || iK >= kGmMax) {
     phg_set_error("Gram-Schmidt: iteration %d outside 1..%d", iK, kGmMax - 1);
     return PHG_EINVAL;
@@ -1638,6 +1642,7 @@ int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double eps
   A.K = c->prm.Kspace;
   A.minIters = c->prm.minIters;
   A.unit = unit ? 1 : 0;
+  A.clocked = clocked ? 1 : 0;
   A.unorm = unorm;
   A.epsnrm = epsnrm;
   A.n0 = n0;

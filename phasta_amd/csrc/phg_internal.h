@@ -493,8 +493,9 @@ int launch_finish(phg_ctx* c, int chan0, int np0, int np, int nsums, double* out
 // vectors, the Hessenberg column, its rotations and the convergence test; the
 // result goes to h_gm with the token seq.  Skipped on the device when an
 // earlier iteration ended the cycle.
-int launch_gs(phg_ctx* c, double* w, int iK, bool unit, double unorm, double epsnrm, double n0,
-              unsigned seq);
+// clocked: the product noted its start in gm->t0
+int launch_gs(phg_ctx* c, double* w, int iK, bool unit, bool clocked, double unorm, double epsnrm,
+              double n0, unsigned seq);
 int launch_scale(phg_ctx* c, double* u, const double* src, long long n,
                  const double* sq_ptr, double* norm_out);
 // dy (+)= the cycle's combination: its first nz directions from zb (stride

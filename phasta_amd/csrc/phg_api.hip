@@ -1289,13 +1289,16 @@ int sol_core(phg_ctx* c, phg_stats* st, bool correct = false) {
   const double sumsq = c->h_sol->sumsq, sumsq_m = c->h_sol->sumsq_m;
   st->nnan = 0;
   st->nlarge = (long long)c->h_sol->bad;
+  // (an abort leaves a zero Dy behind, not an earlier call's)
   if (st->nlarge > 0) {
+    PHG_TRY(launch_fill(c, c->dy, sizeof(double) * V));
     phg_set_error("tnanq: %lld NaN/large entries in res/BDiag", st->nlarge);
     return PHG_ENAN;
   }
   // rstatCheck.f:36-79: from the second Newton iteration of a time step on
   const double totres_chk = std::sqrt(sumsq / (double)(float)n);
   if (c->prm.iter > 1 && totres_chk > 10000.0 * c->reslast) {
+    PHG_TRY(launch_fill(c, c->dy, sizeof(double) * V));
     phg_set_error("rstatCheck: residual diverging (%g > 1e4 * %g)", totres_chk, c->reslast);
     return PHG_EDIVERGE;
   }

@@ -2049,10 +2049,8 @@ extern "C" int phg_mpnn_last_pair(phg_ctx* c, double* bdiag_raw, double* b, doub
     phg_set_error("phg_mpnn_last_pair: enable keep_pair before the solve");
     return PHG_EINVAL;
   }
-  if (bdiag_raw) PHG_TRY(download(c, bdiag_raw, c->mp.bd_raw, 25 * n));
-  if (b) PHG_TRY(download(c, b, c->res, 5 * n));
-  if (zhat) PHG_TRY(download(c, zhat, c->mp.zhat, 5 * n));
-  return sync(c);
+  return download(c, {HostArray(c->mp.bd_raw, bdiag_raw, 25 * n), HostArray(c->res, b, 5 * n),
+                      HostArray(c->mp.zhat, zhat, 5 * n)});
 }
 
 extern "C" int phg_diagnostics(phg_ctx* c, int flags) {

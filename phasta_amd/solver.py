@@ -329,8 +329,7 @@ class GpuSolver:
 
     def download_old(self):
         n = self.case.nshg
-        yold = np.zeros((n, 5), order="F")
-        acold = np.zeros((n, 5), order="F")
+        yold, acold = (np.empty((n, 5), order="F") for _ in range(2))
         _check(lib().phg_state_download_old(self.h, _p(yold), _p(acold)))
         return yold, acold
 
@@ -394,9 +393,8 @@ class GpuSolver:
 
     def mpnn_last_pair(self):
         n = self.case.nshg
-        bd = np.zeros((n, 5, 5), order="F")
-        b = np.zeros((n, 5), order="F")
-        z = np.zeros((n, 5), order="F")
+        bd = np.empty((n, 5, 5), order="F")
+        b, z = (np.empty((n, 5), order="F") for _ in range(2))
         _check(lib().phg_mpnn_last_pair(self.h, _p(bd), _p(b), _p(z)))
         return bd, b, z
 

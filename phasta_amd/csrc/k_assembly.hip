@@ -325,8 +325,8 @@ struct Pipe {
   unsigned at;      // LDS address of piece 0 of this lane's line
 
   __device__ __forceinline__ Pipe(const S* q, const S* g, const int* b, int f, int cnt,
-                                  phg_i4* l)
-      : qps(q), geo(g), blk(b), first(f), last(f + cnt - 1), lds((lp)l) {
+                                  LdsPieces<kPieces>& l)
+      : qps(q), geo(g), blk(b), first(f), last(f + cnt - 1), lds((lp)l.p) {
     const int i = threadIdx.x & 7;
     at = addr(0) + 16 * (64 * i + (threadIdx.x & 56) + i);
     if (threadIdx.x < 16)
@@ -1836,7 +1836,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
   const long long l = wg * 64 + threadIdx.x;
   int4 L = make_int4(0, 0, 0, 0);
   if (l < A.nlanes) L = A.lanes[l];
-  __shared__ phg_i4 lds[Pipe<T, S>::kPieces];
+  __shared__ LdsPieces<Pipe<T, S>::kPieces> lds;
   const bool diag = (L.w >> 1) & 1;
   const int cnt = (A.lhs_on || diag) ? L.z : 0;
   // block sums in the tangent's type (float accumulation on the mixed
@@ -2148,7 +2148,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
 // without DC in double (the other double variants exceed the registers).
 template <typename T, typename S, bool kDC, bool kMT, bool kPair>
 __device__ __forceinline__ void asm_pairs_wave(const BlkArgs& A, const int4 L, const int k2,
-                                               phg_i4* lds) {
+                                               LdsPieces<Pipe<T, S>::kPieces>& lds) {
   using R = T;
   const int cnt = L.z;
   R acc[25], acc2[25];
@@ -2401,7 +2401,7 @@ __device__ __forceinline__ void asm_pairs(const BlkArgs& A) {
   }
   // a wavefront holds pairs or diagonal entries, padding lanes (no blocks, no
   // leader) behind them
-  __shared__ phg_i4 lds[Pipe<T, S>::kPieces];
+  __shared__ LdsPieces<Pipe<T, S>::kPieces> lds;
   if (__builtin_amdgcn_readfirstlane(k2) >= 0)
     asm_pairs_wave<T, S, kDC, kMT, true>(A, L, k2, lds);
   else

@@ -491,8 +491,8 @@ __global__ void __launch_bounds__(256) k_mp_dW(const uint16_t* __restrict__ A,
   constexpr int kPairs = 16 + 4;        // row pairs of a tile, padded
   constexpr int kUnits = 16 * (K / 8);  // (row pair, 8 columns)
   constexpr int kPer = (kUnits + 255) / 256;
-  __shared__ uint32_t sA[K][kPairs];    // A^T tile: [k][row pair]
-  __shared__ uint32_t sU[kH][kPairs];   // dU^T tile: [c][row pair]
+  __shared__ alignas(16) uint32_t sA[K][kPairs];   // A^T tile: [k][row pair]
+  __shared__ alignas(16) uint32_t sU[kH][kPairs];  // dU^T tile: [c][row pair]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = (lane >> 4) * 8;
   const int rp = threadIdx.x & 15, blk = threadIdx.x >> 4;

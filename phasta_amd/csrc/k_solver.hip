@@ -171,12 +171,13 @@ __global__ void __launch_bounds__(kPreWaves * kGroup) k_spsi3pre(
   constexpr int kPieces = aos_stride<TI>() * (int)sizeof(TI) / 16;  // of a record: 7 or 13
   constexpr int kLines = (kPieces + 7) / 8;
   constexpr int kWave = kLines * 512 + 16;  // pieces of LDS: the lines, the lanes' records
-  __shared__ phg_i4 lds_all[kPreWaves * kWave];
+  static_assert(kWave % 8 == 0, "a wavefront's lines begin at a multiple of 128 bytes");
+  __shared__ LdsPieces<kPreWaves * kWave> lds_all;
   typedef __attribute__((address_space(3))) phg_i4* lp;
   typedef const __attribute__((address_space(1))) void* gp;
   const long long g = blockIdx.x;
   const int w = threadIdx.x / kGroup, r = threadIdx.x % kGroup;
-  const lp lds = (lp)lds_all + w * kWave;
+  const lp lds = (lp)lds_all.p + w * kWave;
   const unsigned base = (unsigned)(size_t)lds;
   const unsigned at = base + 16 * (64 * (r & 7) + (r & 56) + (r & 7));
   const int row = max(rowmap[g * kGroup + r], 0);  // (a lane without a row has only padding)

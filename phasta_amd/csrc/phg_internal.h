@@ -102,6 +102,12 @@ __device__ inline void store_slot(double* blk, int r, const A a[25]) {
 }
 
 typedef int phg_i4 __attribute__((ext_vector_type(4)));
+// Pieces of LDS that a lane finds by XOR of the bits 4 to 6 of their address:
+// lines of 128 bytes have to begin at a multiple of 128.
+template <int N>
+struct alignas(128) LdsPieces {
+  phg_i4 p[N];
+};
 // one read of LDS that direct loads have written, complete when it returns
 __device__ __forceinline__ phg_i4 lds_i4(unsigned at) {
   phg_i4 v;

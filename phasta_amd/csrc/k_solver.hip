@@ -476,11 +476,12 @@ __global__ void k_fold_vec(double* v, const int* master, const int* ptr, const i
 }
 
 // ---------------- deterministic reductions ----------------
-// A reduction kernel writes one partial per block (wavefront shuffle, then
-// the block's waves in order) and never synchronises with other blocks;
-// the partials are summed in a fixed order by k_finish or, for the MGS
-// chain, by every block of the next step (same code, same data: the same
-// value in every block).  No atomics, so results do not depend on timing.
+// A reduction writes one partial per workgroup (sums of its wavefronts, added
+// in order); the partials are added in a fixed order, by k_finish for a single
+// inner product (k_dot), or by the workgroup that arrives last for the sums
+// inside k_gs_dots, k_gs_update, k_nodes and k_product_nodes.  The only atomic
+// is the arrival count (arrive_last): results do not depend on timing.
+//
 // Wavefront sum on the vector ALU (row shifts, then the two row broadcasts:
 // no LDS traffic), the same in every lane.
 template <int kCtrl, int kRows>
@@ -520,39 +521,15 @@ __device__ inline void block_partial(double v, double* part) {
   }
 }
 
-// sum of np partials in a fixed order, by a whole block; every thread
-// returns the total
-__device__ inline double block_sum_partials(const double* part, int np) {
-  __shared__ double ws2[kRedThreads / 64];
-  __shared__ double total;
+// *out = the sum of np partials, in a fixed order by one workgroup
+__global__ void __launch_bounds__(kRedThreads) k_finish(const double* part, int np, double* out) {
   double s = 0.0;
   for (int b = threadIdx.x; b < np; b += blockDim.x) s += part[b];
-  s = wave_sum(s);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) ws2[wid] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < kRedThreads / 64; ++w) t += ws2[w];
-    total = t;
-  }
-  __syncthreads();
-  return total;
-}
-
-// out[s] = sum of the partials of channel s (stride between channels):
-// np0 partials in channel 0, np partials in the others
-__global__ void __launch_bounds__(kRedThreads) k_finish(const double* part, int np0, int np,
-                                                        long long stride, int nsums, double* out) {
-  for (int s0 = 0; s0 < nsums; ++s0) {
-    const double t = block_sum_partials(part + (size_t)s0 * stride, s0 == 0 ? np0 : np);
-    if (threadIdx.x == 0) out[s0] = t;
-    __syncthreads();
-  }
+  block_partial(s, out);
 }
 
 // Reductions take one pass of kUnroll independent, coalesced loads per
-// thread (grid sized by red_grid), so every load of a thread is in flight
+// thread (launch_dot's grid), so every load of a thread is in flight
 // at once; a grid-stride tail covers vectors larger than the grid.
 constexpr int kUnroll = 8;
 
@@ -1598,34 +1575,14 @@ int launch_bc3per(phg_ctx* c, double* v, int nq) {
   return 0;
 }
 
-// blocks so that one unrolled pass covers n (at most red_blocks)
-inline int red_grid(const phg_ctx* c, long long n, int per_thread) {
-  const long long b = (n + (long long)kRedThreads * per_thread - 1) / ((long long)kRedThreads * per_thread);
-  return (int)std::max<long long>(1, std::min<long long>(b, c->red_blocks));
-}
-
-// partial channel k of the reduction scratch (red_blocks doubles each)
-inline double* red_chan(phg_ctx* c, int k) { return c->red_part + (size_t)k * c->red_blocks; }
-
-int launch_finish(phg_ctx* c, int chan0, int np0, int np, int nsums, double* out) {
-  k_finish<<<1, kRedThreads, 0, c->stream>>>(red_chan(c, chan0), np0, np, c->red_blocks, nsums,
-                                             out);
-  PHG_HIP(hipGetLastError());
-  return 0;
-}
-
-int launch_dot_part(phg_ctx* c, const double* a, const double* b, long long n, int chan, int* np) {
-  const int g = red_grid(c, n, kUnroll);
-  k_dot<<<g, kRedThreads, 0, c->stream>>>(a, b, n, red_chan(c, chan));
-  PHG_HIP(hipGetLastError());
-  *np = g;
-  return 0;
-}
-
 int launch_dot(phg_ctx* c, const double* a, const double* b, long long n, double* out) {
-  int np = 0;
-  PHG_TRY(launch_dot_part(c, a, b, n, 0, &np));
-  return launch_finish(c, 0, np, np, 1, out);
+  // workgroups so that one unrolled pass covers n, at most red_blocks
+  const int g = (int)std::min<long long>(grid_for(n, kRedThreads * kUnroll), c->red_blocks);
+  k_dot<<<g, kRedThreads, 0, c->stream>>>(a, b, n, c->red_part);
+  PHG_HIP(hipGetLastError());
+  k_finish<<<1, kRedThreads, 0, c->stream>>>(c->red_part, g, out);
+  PHG_HIP(hipGetLastError());
+  return 0;
 }
 
 int launch_gs(phg_ctx* c, double* w, int iK, bool unit, bool clocked, double unorm, double epsnrm,

@@ -150,8 +150,8 @@ __host__ __device__ inline uint8_t constraint_mask(int ibc) {
   return m;
 }
 
-// Longest periodic family (a master and its slaves) whose fold the matvec
-// applies itself: the family's rows have to lie in one 64-row group.
+// Mark of a periodic slave's row in phg_ctx::fam.  The matvec folds a family (a
+// master and its slaves) itself if its rows fit one group of kGroup rows.
 constexpr int kFamSlave = 255;
 
 // Scalars of one GMRES cycle, on the device (k_gs_dots, k_gs_update):
@@ -376,7 +376,7 @@ struct phg_ctx {
 
   // reductions
   int red_blocks = 0;
-  double* red_part = nullptr;      // 2 (kcap + 2) channels of red_blocks partials
+  double* red_part = nullptr;      // 2 (kcap + 3) channels of red_blocks partials
   GmDev* gm = nullptr;             // the running GMRES cycle
   GmHost* h_gm = nullptr;          // its iterations' results (pinned, kGmMax slots)
   unsigned gm_seq = 0;             // token of the last iteration enqueued
@@ -414,7 +414,7 @@ struct phg_ctx {
 
   // timing events on the library stream, created once
   hipEvent_t ev[3] = {};
-  hipEvent_t kev[4] = {};
+  hipEvent_t kev[2] = {};  // around the network's acceptance products
 };
 
 // ---- launchers (k_assembly.hip) ----
@@ -486,14 +486,8 @@ int launch_ref_to_aos(phg_ctx* c, const double* ref);
 // n doubles, n even, 16-byte aligned
 int launch_copy(phg_ctx* c, double* dst, const double* src, long long n);
 int launch_bc3per(phg_ctx* c, double* v, int nq);
-// reductions: per-block partials in channels of red_blocks doubles,
-// summed in a fixed order by launch_finish (np0 partials in the first
-// channel, np in the others)
-int launch_dot(phg_ctx* c, const double* a, const double* b, long long n,
-               double* out);
-int launch_dot_part(phg_ctx* c, const double* a, const double* b, long long n,
-                    int chan, int* np);
-int launch_finish(phg_ctx* c, int chan0, int np0, int np, int nsums, double* out);
+// *out = (a, b), in a fixed order
+int launch_dot(phg_ctx* c, const double* a, const double* b, long long n, double* out);
 // Krylov iteration iK after its product w (of the basis vector as stored, or
 // with unit of the normalised one): orthogonalised against the iK basis
 // vectors, the Hessenberg column, its rotations and the convergence test; the

@@ -1888,23 +1888,29 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
       S v[pt_vals<S>()];
       R Nqa, Nqb;
       pipe.point(q, k, more, code, next, v, Nqa, Nqb);
-      // the point's W PTau and DC weights, asked for together and before any of
-      // them is used: beside Pipe's loads into LDS, whose number depends on the
-      // lane's blocks, the compiler waits for all loads at each use, and with
-      // each load at its own use (DC and the matrix tau, double) a point took
-      // thirteen such waits: the pass 6.02 ms at 64^3 hexes, so 3.80 (4.39 with
-      // every record loaded by its lane)
+      // With DC beside the matrix tau, in double, the point's W PTau and DC weights
+      // are asked for together and before any of them is used: beside Pipe's loads
+      // into LDS, whose number depends on the lane's blocks, the compiler waits for
+      // all loads at each use, and it had put each load at its own use, thirteen
+      // waits per point: the pass 6.02 ms at 64^3 hexes, so 3.80 (4.39 with every
+      // record loaded by its lane).  In the other variants the compiler keeps the
+      // loads together at their use; asked for here they cost 1 to 3 % more.
+      constexpr bool kEarly = kMT && kDC && sizeof(S) == 8;
       R WPT[25];
       double dw[6];
-      if constexpr (kMT) {
+      auto load_dw = [&] {
+        const double* d = A.dcw + ((size_t)e * 4 + q) * 8;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) dw[i] = d[i];
+      };
+      auto load_wpt = [&] {
         const S* mp = reinterpret_cast<const S*>(A.mtau) + ((size_t)e * 4 + q) * mt_stride<S>();
 #pragma unroll
         for (int i = 0; i < 25; ++i) WPT[i] = (R)mp[i];
-        if constexpr (kDC) {
-          const double* d = A.dcw + ((size_t)e * 4 + q) * 8;
-#pragma unroll
-          for (int i = 0; i < 6; ++i) dw[i] = d[i];
-        }
+      };
+      if constexpr (kEarly) {
+        load_wpt();
+        load_dw();
         __builtin_amdgcn_sched_barrier(0);
       }
       const Pt<R> pt = decode_pt<R, S>(v, pc);
@@ -1920,6 +1926,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
         // point's rotated giju
         R dq;
         if constexpr (kMT) {
+          if constexpr (!kEarly) load_dw();
           dq = (R)0;
 #pragma unroll
           for (int i = 0; i < 3; ++i)
@@ -1932,6 +1939,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
       }
       if constexpr (kMT) {
         // rows of P = A(s_a) W PTau + N_a I from the point's W PTau
+        if constexpr (!kEarly) load_wpt();
         mtau_pq<R>(uq, rho, drdp, drdT, e1p, e3p, e4p, WPT, cfacR, sR, rR, W * Nqa, Nqb, acc);
         if constexpr (kNd) {
           // row m of A_k (the flux Jacobian along x_k, pressure-primitive)

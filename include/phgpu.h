@@ -99,7 +99,8 @@ typedef struct phg_stats {
   double reslast;        /* rstatCheck memory across calls                 */
   long long nnan, nlarge;
   double ms_assembly, ms_solve, ms_total;
-  double ms_spmv, ms_mgs; /* summed device-clock times of matvec and MGS    */
+  double ms_spmv, ms_mgs; /* summed device-clock times of matvec and MGS (the
+                             network's acceptance products: HIP events)     */
   int n_spmv, n_mgs;      /* launches behind ms_spmv / ms_mgs              */
   int refine_cycles;      /* GMRES cycles run (1 on the plain FP64 path)   */
   int pc_fallback;        /* learned PC: 0 its cycle converged (or unused),

@@ -1106,8 +1106,9 @@ __device__ __forceinline__ void wall_element(const QpArgs& A, long long p) {
 // and 4.01 -> 2.75 with double ones, of that 5 and 8 % by NodeLines, the rest by shorter
 // records and the quad's sums without shuffles.  Three wavefronts per SIMD, with
 // 12 words spilled, took 3.13 and 3.21.  The variants with DC or the matrix tau
-// are held to 256 registers, two wavefronts per SIMD (float, both, 45^3 hexes: 379
-// -> 340 us with 27 words spilled, 335 with NodeLines).
+// are held to 256 registers, two wavefronts per SIMD: float, both, 45^3 hexes 379
+// -> 340 us with 27 words spilled, 335 with NodeLines; double, both (36 words
+// spilled), 64^3 1.24 -> 1.18 ms, with the reconstructed flux (54) 1.44 -> 1.37.
 template <typename S, bool kDiff, bool kDC, bool kMT>
 __global__ void __launch_bounds__(256, 2) k_asm_qp(QpArgs A) {
   if ((int)blockIdx.x >= A.qp_groups) {
@@ -1815,7 +1816,7 @@ __device__ __forceinline__ PtConst<R> pt_const(const BlkArgs& A) {
 
 // T: stored block type and arithmetic type of the per-point tangent (float
 // on the mixed path); S: storage type of the point states.  Sums over
-// points and elements are taken in double.  kDC: discontinuity capturing
+// points and elements are taken in T, the node's residual in double.  kDC: discontinuity capturing
 // adds WdetJ DC (s_a . giju s_b) A0 per point (e3dc.f:410-446 through
 // e3wmlt), with giju recomputed from the stored shape gradients.  kMT: the
 // matrix tau (itau = 10), P = A(s_a) (W PTau) + N_a I with the stored
@@ -2073,8 +2074,9 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
   }
   // combine the chunks of one block in lane order: the leader adds the
   // partials of the next nch - 1 lanes (the entry's chunks are consecutive
-  // lanes of the wavefront) through cross-lane reads, so the pass holds no
-  // LDS and its occupancy is set by its registers
+  // lanes of the wavefront) through cross-lane reads, so that LDS holds the
+  // records only (13 KB per wavefront in double, 17 in float) and the registers
+  // (104 and more) set the occupancy
   const bool leader = (L.w & 1) && l < A.nlanes;
   const int nch = (L.w >> 8) & 0xff;
   const int total = L.w >> 16;
@@ -2082,7 +2084,7 @@ __global__ void __launch_bounds__(64) k_asm_blocks(BlkArgs A) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
   // the chunk sums stay in the tangent's type (a few float additions more
-  // on the mixed path), which keeps the pass under 64 VGPRs in float
+  // on the mixed path): half the registers in float
   R csum[25];
 #pragma unroll
   for (int i = 0; i < 25; ++i) csum[i] = acc[i];

@@ -886,8 +886,8 @@ __global__ void k_scale(double* u, const double* src, long long n, const double*
 // dy (+)= sum_k y_k u_k, k ascending (solgmr.f:690-692), over the cycle's
 // directions: the first nz from zb (network directions), the others from the
 // basis; the coefficients, each with its vector's 1/norm, as the cycle left
-// them in gm.  Two 8-byte elements per lane and four directions' loads in
-// flight.
+// them in gm.  Four directions' loads in flight per lane; bound by the bytes of
+// the directions.
 __global__ void __launch_bounds__(256) k_combine(double* __restrict__ dy,
                                                  const double* __restrict__ basis, long long kstr,
                                                  const double* __restrict__ zb, long long zstr,
@@ -1612,6 +1612,11 @@ int launch_gs(phg_ctx* c, double* w, int iK, bool unit, bool clocked, double uno
   const long long np2 = (A.n + 1) / 2;
   const int gd = (int)std::min<long long>(grid_for(np2, 256 * kGsU), kGsBlocks);
   const int gu = (int)std::min<long long>(grid_for(np2, kGsThreads), kGsBlocks);
+  // Widths up to 20 vectors, the longest cycle of the workloads, so that hardly
+  // a wavefront loads a vector twice; one width above, whose wavefronts load 15
+  // vectors whatever iK is (the last again) and spill 33 words.  Per iteration
+  // with the update, 64^3, FP64, against one launch per Gram-Schmidt step: 21 to
+  // 24 vectors 178 us (266), 25 to 32 206 (352), 41 to 60 304 (634).
   const int t = (iK + 3) / 4;
   if (t <= 1)
     k_gs_dots<1><<<gd, kGsThreads, 0, c->stream>>>(A);

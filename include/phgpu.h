@@ -311,7 +311,9 @@ int phg_mpnn_train_pair(phg_ctx* ctx, int slot, float lr, double* loss);
  * floats) are nullable.  The vectors are the context's Krylov basis as it
  * stands: host-array entry points that run in between (phg_sparse_ap,
  * phg_sparse_ap_t, phg_tangent_ap) stage their arguments in its
- * first vectors and the matrix they are given replaces K. */
+ * first vectors and the matrix they are given replaces K; and the true
+ * residual that a PHG_MIXED solve or a learned cycle ends with is formed in
+ * them, so train on plain PHG_FP64 solves. */
 int phg_mpnn_train_krylov(phg_ctx* ctx, int nvec, float lr, double* mean_loss, float* grad);
 
 /* Diagnostics (no counterpart in the reference): PHG_DIAG_ORTH measures
